@@ -20,7 +20,7 @@ namespace {
 
 // Cell numbering of the engine's own sorts: tile-major (tile t = (cx/T)*tiles_y + cy/T,
 // then cx%T, cy%T), so that every tile and every cell is one contiguous range.  The
-// operator pic_op_sort sorts whatever keys it is given (cx*ny+cy from pic_op_cell_keys).
+// operator pic_op_sort sorts whatever keys it is given (k_radix.hip).
 // Tile sizes are powers of two and cells are clamped to >= 0: shifts and masks.
 __device__ __forceinline__ int engine_cell_key(int cx, int cy, const RunDesc& rd) {
   const int sh = __builtin_ctz((unsigned)rd.tile), m = rd.tile - 1;
@@ -28,12 +28,11 @@ __device__ __forceinline__ int engine_cell_key(int cx, int cy, const RunDesc& rd
   return (((t << sh) + (cx & m)) << sh) + (cy & m);
 }
 
-template <typename R, bool FROM_POS>
+template <typename R>
 __global__ __launch_bounds__(PIC_WG) void k_sort_rank(const RunDesc* __restrict__ runs,
                                                       const RunState* __restrict__ st,
                                                       const R* __restrict__ x,
                                                       const R* __restrict__ y,
-                                                      const int* __restrict__ keys_in,
                                                       int* __restrict__ keys,
                                                       int* __restrict__ rank,
                                                       int* __restrict__ counts,
@@ -58,32 +57,23 @@ __global__ __launch_bounds__(PIC_WG) void k_sort_rank(const RunDesc* __restrict_
   int key[RANK_U];
   bool act[RANK_U];
   int kmin = INT_MAX, kmax = INT_MIN;
-  if (FROM_POS) {
-    R xv[RANK_U], yv[RANK_U];
+  R xv[RANK_U], yv[RANK_U];
 #pragma unroll
-    for (int u = 0; u < RANK_U; ++u) {
-      const int p = p0 + threadIdx.x + u * PIC_WG;
-      act[u] = p < p1;
-      const int pl = act[u] ? p : p1 - 1;
-      xv[u] = x[pb + pl];
-      yv[u] = y[pb + pl];
-    }
+  for (int u = 0; u < RANK_U; ++u) {
+    const int p = p0 + threadIdx.x + u * PIC_WG;
+    act[u] = p < p1;
+    const int pl = act[u] ? p : p1 - 1;
+    xv[u] = x[pb + pl];
+    yv[u] = y[pb + pl];
+  }
 #pragma unroll
-    for (int u = 0; u < RANK_U; ++u) {
-      int cx, cy;
-      R f;
-      locate(xv[u], dxr, nx, cx, f);
-      locate(yv[u], dyr, ny, cy, f);
-      key[u] = engine_cell_key(cx, cy, rd);
-      if (act[u]) keys[pb + p0 + threadIdx.x + u * PIC_WG] = key[u];
-    }
-  } else {
-#pragma unroll
-    for (int u = 0; u < RANK_U; ++u) {
-      const int p = p0 + threadIdx.x + u * PIC_WG;
-      act[u] = p < p1;
-      key[u] = keys_in[pb + (act[u] ? p : p1 - 1)];
-    }
+  for (int u = 0; u < RANK_U; ++u) {
+    int cx, cy;
+    R f;
+    locate(xv[u], dxr, nx, cx, f);
+    locate(yv[u], dyr, ny, cy, f);
+    key[u] = engine_cell_key(cx, cy, rd);
+    if (act[u]) keys[pb + p0 + threadIdx.x + u * PIC_WG] = key[u];
   }
 #pragma unroll
   for (int u = 0; u < RANK_U; ++u)
@@ -122,15 +112,13 @@ __global__ __launch_bounds__(PIC_WG) void k_sort_rank(const RunDesc* __restrict_
   }
 }
 
-// exclusive scan of the counts of one chunk of PIC_CELL_CHUNK cells; with `clear` the counts
-// are zeroed once read (the engine's sorts keep them zero between sorts, so no fill launch
-// precedes the rank kernel)
+// exclusive scan of the counts of one chunk of PIC_CELL_CHUNK cells; the counts are zeroed
+// once read (they are zero between sorts, so no fill launch precedes the rank kernel)
 __global__ __launch_bounds__(PIC_WG) void k_scan_local(const RunDesc* __restrict__ runs,
                                                        int* __restrict__ counts,
                                                        int* __restrict__ offsets,
                                                        int* __restrict__ chunk_sums,
-                                                       const int2* __restrict__ items,
-                                                       int clear) {
+                                                       const int2* __restrict__ items) {
   __shared__ int wsum[4];
   const int2 it = items[blockIdx.x];
   const RunDesc rd = runs[it.x];
@@ -143,11 +131,9 @@ __global__ __launch_bounds__(PIC_WG) void k_scan_local(const RunDesc* __restrict
     v[k] = (c < G) ? counts[rd.cbase + c] : 0;
     s += v[k];
   }
-  if (clear) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (c0 + k < G) counts[rd.cbase + c0 + k] = 0;
-  }
+  for (int k = 0; k < 8; ++k)
+    if (c0 + k < G) counts[rd.cbase + c0 + k] = 0;
   // inclusive wave scan of per-thread totals
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   int inc = s;
@@ -172,9 +158,8 @@ __global__ __launch_bounds__(PIC_WG) void k_scan_local(const RunDesc* __restrict
 
 // The chunk's base added to its offsets: the base is the sum of the run's chunk totals
 // before it (integer adds, so any order gives the same base), added up by the workgroup
-// itself, which saves a launch that scanned the chunk totals.  With toff (a tile-major cell
-// numbering: tile t owns cells [t T^2, (t + 1) T^2)) also the tile offsets toff[t] =
-// offsets[t T^2].  The run's last chunk writes the total: offsets[G], nsorted and the
+// itself, which saves a launch that scanned the chunk totals.  Also the tile offsets toff[t] =
+// offsets[t T^2] (the cell numbering is tile-major: tile t owns cells [t T^2, (t + 1) T^2)).  The run's last chunk writes the total: offsets[G], nsorted and the
 // closing tile offset; the first workgroup clears the count of cells too large for the
 // within-cell sort's small kernel (which appends to it next).
 __global__ __launch_bounds__(PIC_WG) void k_scan_add(const RunDesc* __restrict__ runs,
@@ -204,7 +189,7 @@ __global__ __launch_bounds__(PIC_WG) void k_scan_add(const RunDesc* __restrict__
     if (c < G) {
       const int o = offsets[rd.cbase + c] + add;
       offsets[rd.cbase + c] = o;
-      if (toff && c % TT == 0) toff[rd.toffbase + c / TT] = o;
+      if (c % TT == 0) toff[rd.toffbase + c / TT] = o;
     }
   }
   if (threadIdx.x == 0) {
@@ -212,7 +197,7 @@ __global__ __launch_bounds__(PIC_WG) void k_scan_add(const RunDesc* __restrict__
       const int total = add + chunk_sums[blockIdx.x];
       offsets[rd.cbase + G] = total;
       st[it.x].nsorted = total;
-      if (toff) toff[rd.toffbase + rd.nbuckets] = total;
+      toff[rd.toffbase + rd.nbuckets] = total;
     }
     if (blockIdx.x == 0) *big_count = 0;
   }
@@ -243,20 +228,11 @@ __device__ __forceinline__ unsigned long long shfl_xor_u64(unsigned long long v,
   return ((unsigned long long)hi << 32) | lo;
 }
 
-__device__ __forceinline__ unsigned long long shfl_u64(unsigned long long v, int src) {
-  unsigned lo = (unsigned)v, hi = (unsigned)(v >> 32);
-  lo = __shfl(lo, src, 64);
-  hi = __shfl(hi, src, 64);
-  return ((unsigned long long)hi << 32) | lo;
-}
-
 __device__ __forceinline__ unsigned long long seg_key(const int* id, long long pb, int slot) {
-  unsigned k = id ? (unsigned)id[pb + slot] : (unsigned)slot;
-  return ((unsigned long long)k << 32) | (unsigned)slot;
+  return ((unsigned long long)(unsigned)id[pb + slot] << 32) | (unsigned)slot;
 }
 
-// Canonical order inside each cell: ascending key (id, or the source index when id is
-// NULL, which makes the sort stable).  One wavefront per cell: <= 64 entries by a bitonic
+// Canonical order inside each cell: ascending id.  One wavefront per cell: <= 64 entries by a bitonic
 // network across lanes, <= 256 entries by counting ranks (4 entries per lane, keys are
 // unique); larger cells are queued for k_segsort_big.  Items cover PIC_SEG_CELLS cells
 // (one per wave).
@@ -950,15 +926,6 @@ __global__ __launch_bounds__(PIC_WG) void k_op_fixed_to_double(const unsigned lo
   }
 }
 
-__global__ __launch_bounds__(PIC_WG) void k_op_validate_keys(const int* keys, int64_t n,
-                                                             int ncells, int* flag) {
-  bool bad = false;
-  for (int64_t p = blockIdx.x * (int64_t)PIC_WG + threadIdx.x; p < n;
-       p += (int64_t)gridDim.x * PIC_WG)
-    if (keys[p] < 0 || keys[p] >= ncells) bad = true;
-  if (bad) atomicOr(flag, 1);
-}
-
 __global__ void k_reduce_sum(const double* parts, int n, double* out) {
   __shared__ double red[4];
   double v = 0.0;
@@ -996,9 +963,6 @@ void launch_op_fixed_to_double(hipStream_t s, const unsigned long long* hi,
                                double* out) {
   k_op_fixed_to_double<<<grid_for(G), PIC_WG, 0, s>>>(hi, lo, G, fp64, scale, out);
 }
-void launch_op_validate_keys(hipStream_t s, const int* keys, int64_t n, int ncells, int* flag) {
-  k_op_validate_keys<<<grid_for(n), PIC_WG, 0, s>>>(keys, n, ncells, flag);
-}
 void launch_reduce_sum(hipStream_t s, const double* parts, int n, double* out) {
   k_reduce_sum<<<1, PIC_WG, 0, s>>>(parts, n, out);
 }
@@ -1011,12 +975,10 @@ static void sort_tail(hipStream_t s, const RunDesc* runs, RunState* st, const in
                                        sb.scratch);
 }
 
-// clear: zero the counts once scanned; toff: also write the tile offsets (nullptr: not)
 static void sort_scan(hipStream_t s, const RunDesc* runs, RunState* st, int nruns, SortBufs sb,
-                      const int2* citems, int ncitems, int clear, int* toff) {
-  k_scan_local<<<ncitems, PIC_WG, 0, s>>>(runs, sb.counts, sb.offsets, sb.chunk_sums, citems,
-                                          clear);
-  k_scan_add<<<ncitems, PIC_WG, 0, s>>>(runs, st, sb.offsets, sb.chunk_sums, citems, toff,
+                      const int2* citems, int ncitems) {
+  k_scan_local<<<ncitems, PIC_WG, 0, s>>>(runs, sb.counts, sb.offsets, sb.chunk_sums, citems);
+  k_scan_add<<<ncitems, PIC_WG, 0, s>>>(runs, st, sb.offsets, sb.chunk_sums, citems, sb.toff,
                                         sb.big_count);
 }
 
@@ -1026,10 +988,9 @@ void launch_sort(hipStream_t s, const RunDesc* runs, RunState* st, int nruns, Pa
                  const int2* citems, int ncitems, long long ctotal, bool move_data) {
   // sb.counts is zero here: zeroed at allocation and by the scan of every sort since
   (void)ctotal;
-  k_sort_rank<R, true><<<npitems * PIC_SORT_SLICES, PIC_WG, 0, s>>>(runs, st, src.x, src.y,
-                                                                   nullptr, sb.keys,
-                                                 sb.rank, sb.counts, pitems);
-  sort_scan(s, runs, st, nruns, sb, citems, ncitems, 1, sb.toff);
+  k_sort_rank<R><<<npitems * PIC_SORT_SLICES, PIC_WG, 0, s>>>(runs, st, src.x, src.y, sb.keys,
+                                                             sb.rank, sb.counts, pitems);
+  sort_scan(s, runs, st, nruns, sb, citems, ncitems);
   k_sort_scatter<<<npitems * PIC_SORT_SLICES, PIC_WG, 0, s>>>(runs, st, sb.keys, sb.rank,
                                                               sb.offsets, sb.perm, pitems);
   sort_tail(s, runs, st, src.id, sb, citems, ncitems);
@@ -1060,19 +1021,6 @@ void launch_fused_scan(hipStream_t s, const RunDesc* runs, RunState* st, int nru
   k_fscan_base<<<nruns, PIC_WG, 0, s>>>(runs, st, sb.fchunk_sums, sb.max_buckets, toff_new);
   k_fscan_rows<<<sb.nfscan_items, PIC_WG, 0, s>>>(runs, sb.ftable, sb.fchunk_sums,
                                                   sb.max_buckets, sb.fscan_items);
-}
-
-void launch_sort_keys_only(hipStream_t s, const RunDesc* runs, RunState* st, const int* keys,
-                           SortBufs sb, const int2* pitems, int npitems, const int2* citems,
-                           int ncitems, long long ctotal) {
-  launch_fill_i32(s, sb.counts, ctotal, 0);
-  k_sort_rank<float, false><<<npitems * PIC_SORT_SLICES, PIC_WG, 0, s>>>(runs, st, nullptr,
-                                                                        nullptr, keys,
-                                                      sb.keys, sb.rank, sb.counts, pitems);
-  sort_scan(s, runs, st, 1, sb, citems, ncitems, 0, nullptr);
-  k_sort_scatter<<<npitems * PIC_SORT_SLICES, PIC_WG, 0, s>>>(runs, st, keys, sb.rank, sb.offsets,
-                                                              sb.perm, pitems);
-  sort_tail(s, runs, st, nullptr, sb, citems, ncitems);
 }
 
 // End of a step, one workgroup per run: the diagnostics row, then the step counter.

@@ -62,10 +62,23 @@ template <typename R>
 void launch_tile_sort(hipStream_t s, const RunDesc* runs, RunState* st, int nruns,
                       PartBufs<R> src, PartBufs<R> dst, SortBufs sb, const int2* pitems,
                       int npitems);
-// op: keys given (run 0 layout), produce perm/counts/offsets
-void launch_sort_keys_only(hipStream_t s, const RunDesc* runs, RunState* st, const int* keys,
-                           SortBufs sb, const int2* pitems, int npitems, const int2* citems,
-                           int ncitems, long long ctotal);
+
+// ---- stable sort of given keys (k_radix.hip)
+struct RadixPlan {
+  int bits, passes;    // digit width and number of digits
+  int items, tiles;    // items per thread, tiles of items * PIC_WG
+};
+struct RadixBufs {
+  int* table;          // [2^bits][tiles]
+  int* totals;         // [2^bits]
+  int* keys[2];        // [n]: pass q writes keys[q & 1]
+  int* idx[2];         // [n]: pass q writes idx[q & 1]; the last writes perm (so one pass
+                       // needs none of them, two need idx[0])
+  int* flag;           // [1], zero: set when a key lies outside [0, ncells)
+};
+RadixPlan radix_plan(long long n, int ncells);
+void launch_radix_sort(hipStream_t s, const int* keys, int n, int ncells, const RadixPlan& p,
+                       RadixBufs b, int* perm, int* counts, int* offsets);
 
 #define FSCAN_ROWS 64  // rows (push items) per fused count-table scan item
 #define PUSH_NT 512            // threads per push workgroup
@@ -127,7 +140,6 @@ void launch_op_deposit(hipStream_t s, const R* x, const R* y, int64_t n, int nx,
 void launch_op_fixed_to_double(hipStream_t s, const unsigned long long* hi,
                                const unsigned long long* lo, long long G, int fp64,
                                double scale, double* out);
-void launch_op_validate_keys(hipStream_t s, const int* keys, int64_t n, int ncells, int* flag);
 void launch_fill_i32(hipStream_t s, int* p, long long n, int v);
 void launch_fill_u64(hipStream_t s, unsigned long long* p, long long n);
 void launch_reduce_sum(hipStream_t s, const double* parts, int n, double* out);

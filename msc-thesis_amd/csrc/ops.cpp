@@ -85,56 +85,25 @@ int pic_op_sort(const int32_t* keys, int64_t n, int ncells, int32_t* perm, int32
   if (n < 0 || ncells < 1 || n > 0x7fff0000) return fail(PIC_ERR_ARG, "bad sizes");
   if (!perm || !counts || !offsets || (n > 0 && !keys)) return fail(PIC_ERR_ARG, "NULL array");
   hipStream_t s = (hipStream_t)stream;
+  const RadixPlan p = radix_plan(n, ncells);
+  const size_t nn = (size_t)std::max<int64_t>(n, 1), nd = (size_t)1 << p.bits;
   DevMem m;
-  int* flag;
-  PIC_HIP(m.get(&flag, 1));
-  PIC_HIP(hipMemsetAsync(flag, 0, sizeof(int), s));
-  if (n > 0) launch_op_validate_keys(s, keys, n, ncells, flag);
+  RadixBufs b;
+  std::memset(&b, 0, sizeof(b));
+  PIC_HIP(m.get(&b.flag, 1));
+  PIC_HIP(m.get(&b.totals, nd));
+  PIC_HIP(m.get(&b.table, nd * std::max(p.tiles, 1)));
+  for (int k = 0; k < 2; ++k) {
+    if (p.passes > k) PIC_HIP(m.get(&b.keys[k], nn));
+    if (p.passes > k + 1) PIC_HIP(m.get(&b.idx[k], nn));
+  }
+  launch_fill_i32(s, b.flag, 1, 0);
+  launch_radix_sort(s, keys, (int)n, ncells, p, b, perm, counts, offsets);
+  PIC_HIP(hipGetLastError());
   int h = 0;
-  PIC_HIP(hipMemcpyAsync(&h, flag, sizeof(int), hipMemcpyDeviceToHost, s));
+  PIC_HIP(hipMemcpyAsync(&h, b.flag, sizeof(int), hipMemcpyDeviceToHost, s));
   PIC_HIP(hipStreamSynchronize(s));
   if (h) return fail(PIC_ERR_ARG, "key outside [0, ncells)");
-  // one run with nx = ncells, ny = 1 (G = ncells); counts/offsets are the caller's arrays
-  RunDesc d = op_desc(ncells, 1, 1.0, 1.0, n);
-  RunDesc* dd;
-  RunState* st;
-  PIC_HIP(m.get(&dd, 1));
-  PIC_HIP(m.get(&st, 1));
-  RunState hs;
-  std::memset(&hs, 0, sizeof(hs));
-  hs.np = (int)n;
-  std::vector<int2> pit, cit, sit;
-  for (long long q = 0; q < std::max<long long>(n, 1); q += PIC_CHUNK) pit.push_back(make_int2(0, (int)q));
-  for (int c = 0; c < ncells; c += PIC_CELL_CHUNK) cit.push_back(make_int2(0, c));
-  for (int c = 0; c < ncells; c += PIC_SEG_CELLS) sit.push_back(make_int2(0, c));
-  d.cell_item_begin = 0;
-  d.cell_item_end = (int)cit.size();
-  int2 *dp, *dc, *ds;
-  PIC_HIP(m.get(&dp, pit.size()));
-  PIC_HIP(m.get(&dc, cit.size()));
-  PIC_HIP(m.get(&ds, sit.size()));
-  PIC_HIP(hipMemcpyAsync(ds, sit.data(), sizeof(int2) * sit.size(), hipMemcpyHostToDevice, s));
-  SortBufs sb;
-  std::memset(&sb, 0, sizeof(sb));
-  sb.segitems = ds;
-  sb.nsegitems = (int)sit.size();
-  PIC_HIP(m.get(&sb.rank, std::max<int64_t>(n, 1)));
-  PIC_HIP(m.get(&sb.chunk_sums, cit.size()));
-  PIC_HIP(m.get(&sb.big_list, 2 * (size_t)ncells));
-  PIC_HIP(m.get(&sb.big_count, 1));
-  PIC_HIP(m.get(&sb.scratch, 2 * (size_t)std::max<int64_t>(n, 1)));
-  sb.keys = nullptr;
-  sb.perm = perm;
-  sb.counts = counts;
-  // offsets need ncells + 1 entries: the caller's array
-  sb.offsets = offsets;
-  PIC_HIP(hipMemcpyAsync(dd, &d, sizeof(d), hipMemcpyHostToDevice, s));
-  PIC_HIP(hipMemcpyAsync(st, &hs, sizeof(hs), hipMemcpyHostToDevice, s));
-  PIC_HIP(hipMemcpyAsync(dp, pit.data(), sizeof(int2) * pit.size(), hipMemcpyHostToDevice, s));
-  PIC_HIP(hipMemcpyAsync(dc, cit.data(), sizeof(int2) * cit.size(), hipMemcpyHostToDevice, s));
-  launch_sort_keys_only(s, dd, st, keys, sb, dp, (int)pit.size(), dc, (int)cit.size(), ncells);
-  PIC_HIP(hipGetLastError());
-  PIC_HIP(hipStreamSynchronize(s));
   return PIC_OK;
 }
 
