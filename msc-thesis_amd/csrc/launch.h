@@ -285,7 +285,10 @@ struct DsmcArgs {
 void launch_dsmc(hipStream_t s, const DsmcArgs& a);
 
 // ---- the reference's own collide arithmetic on an injected uniform stream (k_refcollide.hip)
-#define REF_CHAIN_CHUNK 1024  // stream positions per chunk of the consumer-start resolution
+#define REF_CHAIN_CHUNK 4096  // stream positions per chunk of the consumer-start resolution
+// positions that m consumers can reach (at most 7 uniforms each): the part of a stream of nu
+// that has to be resolved
+inline long long ref_chain_stream(long long nu, long long m) { return nu / 7 < m ? nu : 7 * m; }
 struct RefChainBufs {
   int2* maps;            // [7 * nchunks] (exit offset, consumers) per chunk and entry offset
   int* entry;            // [nchunks]

@@ -34,7 +34,7 @@ struct Scratch {
 // consumer starts of m consumers on u[nu]; *used = uniforms they take
 int resolve_chain(hipStream_t s, Scratch& sc, const double* u, long long nu, double prob,
                   long long m, long long** start, long long* used) {
-  const long long nchunks = (nu + REF_CHAIN_CHUNK - 1) / REF_CHAIN_CHUNK;
+  const long long nchunks = (ref_chain_stream(nu, m) + REF_CHAIN_CHUNK - 1) / REF_CHAIN_CHUNK;
   RefChainBufs b;
   PIC_HIP(sc.get(&b.maps, 7 * std::max(nchunks, 1LL)));
   PIC_HIP(sc.get(&b.entry, std::max(nchunks, 1LL)));
