@@ -896,22 +896,6 @@ __global__ __launch_bounds__(PIC_WG) void k_op_gather_push(R* x, R* y, R* vx, R*
   if (partials && threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
-template <typename R>
-__global__ __launch_bounds__(PIC_WG) void k_op_deposit(const R* __restrict__ x,
-                                                       const R* __restrict__ y, int64_t n,
-                                                       int nx, int ny, double lx, double ly,
-                                                       unsigned long long* hi,
-                                                       unsigned long long* lo) {
-  const Geo<R> g = make_geo<R>(nx, ny, lx, ly);
-  for (int64_t p = blockIdx.x * (int64_t)PIC_WG + threadIdx.x; p < n;
-       p += (int64_t)gridDim.x * PIC_WG) {
-    int cx, cy;
-    long long w[4];
-    deposit_weights<R>(x[p], y[p], g, cx, cy, w);
-    deposit_global<R>(hi, lo, cx, cy, w, g);
-  }
-}
-
 __global__ __launch_bounds__(PIC_WG) void k_op_fixed_to_double(const unsigned long long* hi,
                                                                const unsigned long long* lo,
                                                                long long G, int fp64,
@@ -948,16 +932,6 @@ void launch_fill_i32(hipStream_t s, int* p, long long n, int v) {
 void launch_fill_u64(hipStream_t s, unsigned long long* p, long long n) {
   if (n > 0) k_fill_u64<<<grid_for(n), PIC_WG, 0, s>>>(p, n);
 }
-template <typename R>
-void launch_op_deposit(hipStream_t s, const R* x, const R* y, int64_t n, int nx, int ny,
-                       double lx, double ly, unsigned long long* hi, unsigned long long* lo) {
-  k_op_deposit<R><<<grid_for(n), PIC_WG, 0, s>>>(x, y, n, nx, ny, lx, ly, hi, lo);
-}
-template void launch_op_deposit<float>(hipStream_t, const float*, const float*, int64_t, int, int,
-                                       double, double, unsigned long long*, unsigned long long*);
-template void launch_op_deposit<double>(hipStream_t, const double*, const double*, int64_t, int,
-                                        int, double, double, unsigned long long*,
-                                        unsigned long long*);
 void launch_op_fixed_to_double(hipStream_t s, const unsigned long long* hi,
                                const unsigned long long* lo, long long G, int fp64, double scale,
                                double* out) {

@@ -78,11 +78,12 @@ __global__ __launch_bounds__(PIC_WG) void k_radix_hist(const int* __restrict__ k
 }
 
 // one workgroup per digit: its row of the table scanned in place, four tiles per thread
+// (flag may be NULL)
 __global__ __launch_bounds__(PIC_WG) void k_radix_rows(int* __restrict__ table, int ntiles,
                                                        int* __restrict__ totals,
                                                        const int* __restrict__ flag) {
   __shared__ int wsum[RADIX_NW];
-  if (*flag) return;
+  if (flag && *flag) return;
   int* row = table + (long long)blockIdx.x * ntiles;
   int carry = 0;
   for (int t0 = 0; t0 < ntiles; t0 += 4 * PIC_WG) {
@@ -239,7 +240,7 @@ void radix_passes(hipStream_t s, const int* keys, int n, int ncells, const Radix
     else
       k_radix_hist<IT, false><<<p.tiles, PIC_WG, 0, s>>>(kin, n, shift, p.bits, ncells, p.tiles,
                                                          b.table, b.flag);
-    k_radix_rows<<<1 << p.bits, PIC_WG, 0, s>>>(b.table, p.tiles, b.totals, b.flag);
+    launch_scan_rows(s, b.table, 1 << p.bits, p.tiles, b.totals, b.flag);
     if (q == 0)
       k_radix_scatter<IT, true><<<p.tiles, PIC_WG, 0, s>>>(kin, iin, n, shift, p.bits, p.tiles,
                                                            b.table, b.totals, kout, iout, b.flag);
@@ -257,6 +258,11 @@ void radix_passes(hipStream_t s, const int* keys, int n, int ncells, const Radix
 }
 
 }  // namespace
+
+void launch_scan_rows(hipStream_t s, int* table, int rows, int cols, int* totals,
+                      const int* flag) {
+  k_radix_rows<<<rows, PIC_WG, 0, s>>>(table, cols, totals, flag);
+}
 
 // Tiles of 1024 items until they fill the chip four times over, of 4096 above (a tile's
 // digit runs, and so the pieces it writes, are longer).

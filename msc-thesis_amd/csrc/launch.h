@@ -63,6 +63,28 @@ void launch_tile_sort(hipStream_t s, const RunDesc* runs, RunState* st, int nrun
                       PartBufs<R> src, PartBufs<R> dst, SortBufs sb, const int2* pitems,
                       int npitems);
 
+// ---- deposit of particles in any order (k_deposit.hip)
+enum { DEPOSIT_DIRECT, DEPOSIT_GRID, DEPOSIT_BINNED };
+struct DepositPlan {
+  int form;            // DEPOSIT_*
+  int ltx, lty;        // binned: log2 of the tile sides
+  int tiles, tiles_y;
+  int items, groups;   // positions per thread and workgroups of the moving pass
+  int slice;           // positions per workgroup of the summing pass
+};
+struct DepositBufs {   // binned form only
+  int* table;          // [tiles][groups]
+  int* totals;         // [tiles]
+  int* offs;           // [tiles + 1]
+  void* pos;           // [n] (x, y) pairs
+};
+// scratch: DepositBufs can be had (the binned form may be chosen)
+DepositPlan deposit_plan(int64_t n, int nx, int ny, int fp64, bool scratch);
+template <typename R>
+void launch_op_deposit(hipStream_t s, const DepositPlan& p, const R* x, const R* y, int64_t n,
+                       int nx, int ny, double lx, double ly, unsigned long long* hi,
+                       unsigned long long* lo, DepositBufs b);
+
 // ---- stable sort of given keys (k_radix.hip)
 struct RadixPlan {
   int bits, passes;    // digit width and number of digits
@@ -77,6 +99,10 @@ struct RadixBufs {
   int* flag;           // [1], zero: set when a key lies outside [0, ncells)
 };
 RadixPlan radix_plan(long long n, int ncells);
+// exclusive scan of every row of table[rows][cols] in place, and the rows' sums; does nothing
+// when flag is given and set
+void launch_scan_rows(hipStream_t s, int* table, int rows, int cols, int* totals,
+                      const int* flag);
 void launch_radix_sort(hipStream_t s, const int* keys, int n, int ncells, const RadixPlan& p,
                        RadixBufs b, int* perm, int* counts, int* offsets);
 
@@ -134,9 +160,6 @@ template <typename R>
 void launch_op_gather_push(hipStream_t s, R* x, R* y, R* vx, R* vy, int64_t n, const double* ex,
                            const double* ey, int nx, int ny, double lx, double ly, double dt,
                            double qm, double c, double* ke_partials, int nblocks);
-template <typename R>
-void launch_op_deposit(hipStream_t s, const R* x, const R* y, int64_t n, int nx, int ny,
-                       double lx, double ly, unsigned long long* hi, unsigned long long* lo);
 void launch_op_fixed_to_double(hipStream_t s, const unsigned long long* hi,
                                const unsigned long long* lo, long long G, int fp64,
                                double scale, double* out);

@@ -115,21 +115,36 @@ int pic_op_deposit(const void* x, const void* y, int64_t n, int precision, const
   if (precision != PIC_FP32 && precision != PIC_FP64) return fail(PIC_ERR_ARG, "bad precision");
   hipStream_t s = (hipStream_t)stream;
   const long long G = (long long)g->nx * g->ny;
+  const bool fp64 = precision == PIC_FP64;
+  DepositPlan p = deposit_plan(n, g->nx, g->ny, fp64, true);
   DevMem m;
   unsigned long long *hi, *lo = nullptr;
   PIC_HIP(m.get(&hi, G));
-  PIC_HIP(hipMemsetAsync(hi, 0, sizeof(unsigned long long) * G, s));
-  if (precision == PIC_FP64) {
-    PIC_HIP(m.get(&lo, G));
-    PIC_HIP(hipMemsetAsync(lo, 0, sizeof(unsigned long long) * G, s));
+  if (fp64) PIC_HIP(m.get(&lo, G));
+  DepositBufs b;
+  std::memset(&b, 0, sizeof(b));
+  if (p.form == DEPOSIT_BINNED) {
+    char* pos = nullptr;
+    const size_t table = (size_t)p.tiles * p.groups;
+    if (m.get(&b.table, table + 2 * (size_t)p.tiles + 1) == hipSuccess &&
+        m.get(&pos, (fp64 ? 16 : 8) * (size_t)n) == hipSuccess) {
+      b.totals = b.table + table;
+      b.offs = b.totals + p.tiles;
+      b.pos = pos;
+    } else {  // no memory for the moved positions: a form that needs none
+      (void)hipGetLastError();
+      p = deposit_plan(n, g->nx, g->ny, fp64, false);
+    }
   }
+  launch_fill_u64(s, hi, G);
+  if (fp64) launch_fill_u64(s, lo, G);
   if (n > 0) {
-    if (precision == PIC_FP64)
-      launch_op_deposit<double>(s, (const double*)x, (const double*)y, n, g->nx, g->ny, g->lx,
-                                g->ly, hi, lo);
+    if (fp64)
+      launch_op_deposit<double>(s, p, (const double*)x, (const double*)y, n, g->nx, g->ny, g->lx,
+                                g->ly, hi, lo, b);
     else
-      launch_op_deposit<float>(s, (const float*)x, (const float*)y, n, g->nx, g->ny, g->lx, g->ly,
-                               hi, lo);
+      launch_op_deposit<float>(s, p, (const float*)x, (const float*)y, n, g->nx, g->ny, g->lx,
+                               g->ly, hi, lo, b);
   }
   const double dx = g->lx / g->nx, dy = g->ly / g->ny;
   const double scale = qp / (dx * dy) * (precision == PIC_FP64 ? 1.0 : std::ldexp(1.0, -36));
@@ -190,12 +205,15 @@ int pic_op_deposit_noalloc(const void* x, const void* y, int64_t n, int precisio
   launch_fill_u64(s, hi, G);
   if (precision == PIC_FP64) launch_fill_u64(s, lo, G);
   if (n > 0) {
+    // the forms that need no memory of their own
+    const DepositPlan p = deposit_plan(n, g->nx, g->ny, precision == PIC_FP64, false);
+    const DepositBufs none = {nullptr, nullptr, nullptr, nullptr};
     if (precision == PIC_FP64)
-      launch_op_deposit<double>(s, (const double*)x, (const double*)y, n, g->nx, g->ny, g->lx,
-                                g->ly, hi, lo);
+      launch_op_deposit<double>(s, p, (const double*)x, (const double*)y, n, g->nx, g->ny, g->lx,
+                                g->ly, hi, lo, none);
     else
-      launch_op_deposit<float>(s, (const float*)x, (const float*)y, n, g->nx, g->ny, g->lx, g->ly,
-                               hi, nullptr);
+      launch_op_deposit<float>(s, p, (const float*)x, (const float*)y, n, g->nx, g->ny, g->lx,
+                               g->ly, hi, nullptr, none);
   }
   const double dx = g->lx / g->nx, dy = g->ly / g->ny;
   const double scale = qp / (dx * dy) * (precision == PIC_FP64 ? 1.0 : std::ldexp(1.0, -36));
