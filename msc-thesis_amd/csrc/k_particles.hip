@@ -7,6 +7,7 @@
 //   positionUpdate     :372-420  -> leapfrog push, periodic wrap into [0, L)
 //   cellTrackerSetup   thesisCode/dsmcCollisions/cellTrackerAdvanced/src/pic.cu:419-445
 //                                -> stable counting sort by key cx*ny+cy (ties by id)
+#include <algorithm>
 #include <climits>
 #include <type_traits>
 #include "launch.h"
@@ -849,51 +850,141 @@ __global__ __launch_bounds__(PIC_WG) void k_op_cell_keys(const R* __restrict__ x
   }
 }
 
+// ---- gather + push of a caller's particles, in place and in any order.  Three sources of the
+// field give the same values (each is the node's FP64 field rounded to R):
+//   GP_NODES   the caller's two node arrays: eight 8-byte loads per particle
+//   GP_PACKED  (Ex, Ey) pairs on the padded (nx + 1) x (ny + 1) nodes, made by k_op_pack_E:
+//              a cell's two node rows are two contiguous pieces of two pairs
+//   GP_LDS     the same padded pairs of a small grid, in every workgroup's LDS
+// Random positions are bound by the vector L1: 64 lanes of a load meet up to 64 lines, so the
+// number of load instructions sets the time (launch_op_gather_push has the measurements).
+enum { GP_NODES, GP_PACKED, GP_LDS };
+
 template <typename R>
-__global__ __launch_bounds__(PIC_WG) void k_op_gather_push(R* x, R* y, R* vx, R* vy, int64_t n,
-                                                           const double* __restrict__ ex,
-                                                           const double* __restrict__ ey,
-                                                           int nx, int ny, double lx, double ly,
-                                                           double dt, double qm, double c,
-                                                           double* partials) {
-  __shared__ double red[4];
+__global__ __launch_bounds__(PIC_WG) void k_op_pack_E(const double* __restrict__ ex,
+                                                      const double* __restrict__ ey, int nx,
+                                                      int ny,
+                                                      typename EWin<R>::R2* __restrict__ E) {
+  const int lny = __builtin_ctz((unsigned)ny);
+  const int G = nx * ny;
+  for (int q = blockIdx.x * PIC_WG + threadIdx.x; q < G; q += gridDim.x * PIC_WG) {
+    const int i = q >> lny, j = q & (ny - 1);
+    typename EWin<R>::R2 v;
+    v.x = (R)ex[q];
+    v.y = (R)ey[q];
+    typename EWin<R>::R2* row = E + (long long)i * (ny + 1);
+    row[j] = v;
+    if (j == 0) row[ny] = v;
+    if (i == 0) {
+      typename EWin<R>::R2* last = E + (long long)nx * (ny + 1);
+      last[j] = v;
+      if (j == 0) last[ny] = v;
+    }
+  }
+}
+
+template <typename R, int SRC>
+__global__ __launch_bounds__(SRC == GP_LDS ? GP_LDS_NT : PIC_WG) void k_op_gather_push(
+    R* x, R* y, R* vx, R* vy, int64_t n, const double* __restrict__ ex,
+    const double* __restrict__ ey, const typename EWin<R>::R2* __restrict__ E, int nx, int ny,
+    double lx, double ly, double dt, double qm, double c, double* partials) {
+  typedef typename EWin<R>::R2 R2;
+  constexpr int NT = SRC == GP_LDS ? GP_LDS_NT : PIC_WG, U = SRC == GP_NODES ? 1 : 4;
+  extern __shared__ double2 gp_lds[];
+  __shared__ double red[NT / 64];
   const Geo<R> g = make_geo<R>(nx, ny, lx, ly);
   const R hk = (R)(c * dt * qm), dtr = (R)dt;
   const double skc = (c - 0.5) * dt * qm;
-  double ke = 0, px = 0, py = 0;
-  for (int64_t p = blockIdx.x * (int64_t)PIC_WG + threadIdx.x; p < n;
-       p += (int64_t)gridDim.x * PIC_WG) {
-    R xr = x[p], yr = y[p], vxr = vx[p], vyr = vy[p];
-    int cx, cy;
-    R fx, fy;
-    locate_w(xr, g.idx, nx, cx, fx);
-    locate_w(yr, g.idy, ny, cy, fy);
-    const R qs = (R)(1.0 / (double)(1 << Fix<R>::QB));
-    const R gx1 = (R)qweight(fx) * qs, gy1 = (R)qweight(fy) * qs;
-    const R gx0 = (R)1 - gx1, gy0 = (R)1 - gy1;
-    const R g00 = gx0 * gy0, g10 = gx1 * gy0, g01 = gx0 * gy1, g11 = gx1 * gy1;
-    const int cxp = (cx + 1 == nx) ? 0 : cx + 1, cyp = (cy + 1 == ny) ? 0 : cy + 1;
-    const long long n00 = (long long)cx * ny + cy, n10 = (long long)cxp * ny + cy,
-                    n01 = (long long)cx * ny + cyp, n11 = (long long)cxp * ny + cyp;
-    R epx = g00 * (R)ex[n00];
-    epx = fmar(g10, (R)ex[n10], epx);
-    epx = fmar(g01, (R)ex[n01], epx);
-    epx = fmar(g11, (R)ex[n11], epx);
-    R epy = g00 * (R)ey[n00];
-    epy = fmar(g10, (R)ey[n10], epy);
-    epy = fmar(g01, (R)ey[n01], epy);
-    epy = fmar(g11, (R)ey[n11], epy);
-    const double vsx = (double)vxr + skc * (double)epx, vsy = (double)vyr + skc * (double)epy;
-    ke += vsx * vsx + vsy * vsy;
-    vxr = fmar(hk, epx, vxr);
-    vyr = fmar(hk, epy, vyr);
-    x[p] = wrap_pos(fmar(dtr, vxr, xr), g.Lx);
-    y[p] = wrap_pos(fmar(dtr, vyr, yr), g.Ly);
-    vx[p] = vxr;
-    vy[p] = vyr;
+  const int ny1 = ny + 1;
+  R2* el = reinterpret_cast<R2*>(gp_lds);
+  if (SRC == GP_LDS) {
+    const int lny = __builtin_ctz((unsigned)ny);
+#pragma unroll 4
+    for (int q = threadIdx.x; q < nx * ny; q += NT) {
+      const int i = q >> lny, j = q & (ny - 1);
+      R2 v;
+      v.x = (R)ex[q];
+      v.y = (R)ey[q];
+      el[i * ny1 + j] = v;
+      if (j == 0) el[i * ny1 + ny] = v;
+      if (i == 0) {
+        el[nx * ny1 + j] = v;
+        if (j == 0) el[nx * ny1 + ny] = v;
+      }
+    }
+    __syncthreads();
   }
-  const double s = block_sum(ke, red);
-  if (partials && threadIdx.x == 0) partials[blockIdx.x] = s;
+  double ke = 0;
+  const int64_t stride = (int64_t)gridDim.x * NT;
+  for (int64_t p0 = blockIdx.x * (int64_t)NT + threadIdx.x; p0 < n; p0 += U * stride) {
+    // the state of U particles, then their fields, then their pushes (past the end: the last)
+    R xr[U], yr[U], vxr[U], vyr[U], g00[U], g10[U], g01[U], g11[U];
+    R2 e00[U], e10[U], e01[U], e11[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t p = p0 + u * stride;
+      const int64_t pl = p < n ? p : n - 1;
+      xr[u] = x[pl]; yr[u] = y[pl]; vxr[u] = vx[pl]; vyr[u] = vy[pl];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int cx, cy;
+      R fx, fy;
+      locate_w(xr[u], g.idx, nx, cx, fx);
+      locate_w(yr[u], g.idy, ny, cy, fy);
+      const R qs = (R)(1.0 / (double)(1 << Fix<R>::QB));
+      const R gx1 = (R)qweight(fx) * qs, gy1 = (R)qweight(fy) * qs;
+      const R gx0 = (R)1 - gx1, gy0 = (R)1 - gy1;
+      g00[u] = gx0 * gy0; g10[u] = gx1 * gy0; g01[u] = gx0 * gy1; g11[u] = gx1 * gy1;
+      if (SRC == GP_NODES) {
+        const int cxp = (cx + 1 == nx) ? 0 : cx + 1, cyp = (cy + 1 == ny) ? 0 : cy + 1;
+        const long long n00 = (long long)cx * ny + cy, n10 = (long long)cxp * ny + cy,
+                        n01 = (long long)cx * ny + cyp, n11 = (long long)cxp * ny + cyp;
+        e00[u].x = (R)ex[n00]; e10[u].x = (R)ex[n10]; e01[u].x = (R)ex[n01]; e11[u].x = (R)ex[n11];
+        e00[u].y = (R)ey[n00]; e10[u].y = (R)ey[n10]; e01[u].y = (R)ey[n01]; e11[u].y = (R)ey[n11];
+      } else if (SRC == GP_LDS) {
+        const int i0 = cx * ny1 + cy;
+        e00[u] = el[i0]; e01[u] = el[i0 + 1]; e10[u] = el[i0 + ny1]; e11[u] = el[i0 + ny1 + 1];
+      } else {
+        // two neighbouring pairs as one piece (16 B in FP32, aligned to 8)
+        R2 r0[2], r1[2];
+        const R2* e = E + (long long)cx * ny1 + cy;
+        __builtin_memcpy(r0, e, sizeof(r0));
+        __builtin_memcpy(r1, e + ny1, sizeof(r1));
+        e00[u] = r0[0]; e01[u] = r0[1]; e10[u] = r1[0]; e11[u] = r1[1];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t p = p0 + u * stride;
+      if (p >= n) continue;
+      R epx = g00[u] * e00[u].x;
+      epx = fmar(g10[u], e10[u].x, epx);
+      epx = fmar(g01[u], e01[u].x, epx);
+      epx = fmar(g11[u], e11[u].x, epx);
+      R epy = g00[u] * e00[u].y;
+      epy = fmar(g10[u], e10[u].y, epy);
+      epy = fmar(g01[u], e01[u].y, epy);
+      epy = fmar(g11[u], e11[u].y, epy);
+      const double vsx = (double)vxr[u] + skc * (double)epx;
+      const double vsy = (double)vyr[u] + skc * (double)epy;
+      ke += vsx * vsx + vsy * vsy;
+      const R wx = fmar(hk, epx, vxr[u]), wy = fmar(hk, epy, vyr[u]);
+      x[p] = wrap_pos(fmar(dtr, wx, xr[u]), g.Lx);
+      y[p] = wrap_pos(fmar(dtr, wy, yr[u]), g.Ly);
+      vx[p] = wx;
+      vy[p] = wy;
+    }
+  }
+  if (!partials) return;  // uniform
+  ke = wave_sum(ke);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ke;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+    for (int w = 0; w < NT / 64; ++w) s += red[w];
+    partials[blockIdx.x] = s;
+  }
 }
 
 __global__ __launch_bounds__(PIC_WG) void k_op_fixed_to_double(const unsigned long long* hi,
@@ -1051,12 +1142,50 @@ void launch_op_cell_keys(hipStream_t s, const R* x, const R* y, int64_t n, int n
   k_op_cell_keys<R><<<grid_for(n), PIC_WG, 0, s>>>(x, y, n, nx, ny, lx / nx, ly / ny, keys);
 }
 
+// LDS: grids whose padded pairs leave two workgroups per CU.  Packed: enough particles to pay
+// for packing (an allocation, a launch, and 24 or 32 bytes per node).  Whole calls, random
+// order, node arrays -> new form, FP32 / FP64 (us):
+//   LDS, 64^2: 8,000,009 particles 145 / 155 -> 59 / 100, 1,048,576: 36 / 39 -> 29 / 33,
+//   524,288: 27 / 28 -> 27 / 31
+//   packed, 512^2: 8,000,009 particles 316 / 319 -> 171 / 238 (the kernel 269 -> 97 + 5 to
+//   pack, FP32), 4,194,304: 157 / 166 -> 92 / 145, 1,048,576: 56 / 60 -> 61 / 78
+GatherPushPlan gather_push_plan(int64_t n, int nx, int ny, int fp64) {
+  GatherPushPlan p;
+  const long long G = (long long)nx * ny, pad = (long long)(nx + 1) * (ny + 1);
+  const long long bytes = pad * (fp64 ? 16 : 8);
+  p.pairs = 0;
+  p.lds = 0;
+  if (bytes <= 72 * 1024 && n >= (1 << 20)) {
+    p.lds = (int)bytes;
+    const long long per = std::max<long long>(2 * GP_LDS_NT, 2 * G);
+    const long long b = (n + per - 1) / per;
+    p.blocks = (int)(b > 512 ? 512 : b);
+    return p;
+  }
+  const long long b = (n + PIC_WG - 1) / PIC_WG;
+  p.blocks = (int)(b < 1 ? 1 : (b > 4096 ? 4096 : b));
+  if (n >= (3 << 19) && n >= G && bytes < (64 << 20)) p.pairs = pad;
+  return p;
+}
+
 template <typename R>
-void launch_op_gather_push(hipStream_t s, R* x, R* y, R* vx, R* vy, int64_t n, const double* ex,
-                           const double* ey, int nx, int ny, double lx, double ly, double dt,
-                           double qm, double c, double* ke_partials, int nblocks) {
-  k_op_gather_push<R><<<nblocks, PIC_WG, 0, s>>>(x, y, vx, vy, n, ex, ey, nx, ny, lx, ly, dt, qm,
-                                                 c, ke_partials);
+void launch_op_gather_push(hipStream_t s, const GatherPushPlan& p, R* x, R* y, R* vx, R* vy,
+                           int64_t n, const double* ex, const double* ey, int nx, int ny,
+                           double lx, double ly, double dt, double qm, double c,
+                           double* ke_partials, void* pairs) {
+  typedef typename EWin<R>::R2 R2;
+  R2* E = (R2*)pairs;
+  if (p.lds) {
+    k_op_gather_push<R, GP_LDS><<<p.blocks, GP_LDS_NT, p.lds, s>>>(
+        x, y, vx, vy, n, ex, ey, nullptr, nx, ny, lx, ly, dt, qm, c, ke_partials);
+  } else if (E) {
+    k_op_pack_E<R><<<grid_for((long long)nx * ny), PIC_WG, 0, s>>>(ex, ey, nx, ny, E);
+    k_op_gather_push<R, GP_PACKED><<<p.blocks, PIC_WG, 0, s>>>(
+        x, y, vx, vy, n, nullptr, nullptr, E, nx, ny, lx, ly, dt, qm, c, ke_partials);
+  } else {
+    k_op_gather_push<R, GP_NODES><<<p.blocks, PIC_WG, 0, s>>>(
+        x, y, vx, vy, n, ex, ey, nullptr, nx, ny, lx, ly, dt, qm, c, ke_partials);
+  }
 }
 
 #define PIC_INST(R)                                                                          \
@@ -1075,8 +1204,9 @@ void launch_op_gather_push(hipStream_t s, R* x, R* y, R* vx, R* vy, int64_t n, c
                                        const int2*, int, int*);                             \
   template void launch_op_cell_keys<R>(hipStream_t, const R*, const R*, int64_t, int, int,  \
                                        double, double, int*);                               \
-  template void launch_op_gather_push<R>(hipStream_t, R*, R*, R*, R*, int64_t,              \
-                                         const double*, const double*, int, int, double,    \
-                                         double, double, double, double, double*, int);
+  template void launch_op_gather_push<R>(hipStream_t, const GatherPushPlan&, R*, R*, R*, R*, \
+                                         int64_t, const double*, const double*, int, int,   \
+                                         double, double, double, double, double, double*,   \
+                                         void*);
 PIC_INST(float)
 PIC_INST(double)

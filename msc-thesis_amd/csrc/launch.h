@@ -156,10 +156,19 @@ void launch_check_finite(hipStream_t s, const RunDesc* runs, RunState* st, PartB
 template <typename R>
 void launch_op_cell_keys(hipStream_t s, const R* x, const R* y, int64_t n, int nx, int ny,
                          double lx, double ly, int* keys);
+#define GP_LDS_NT 512   // threads per workgroup of the gather + push with the field in LDS
+struct GatherPushPlan {
+  int blocks;           // workgroups (and kinetic-energy partials)
+  int lds;              // bytes of the padded field in LDS, 0: not there
+  long long pairs;      // (Ex, Ey) pairs of the packed field, 0: not used
+};
+GatherPushPlan gather_push_plan(int64_t n, int nx, int ny, int fp64);
+// pairs: memory for the plan's packed field, or NULL (then the node arrays are read)
 template <typename R>
-void launch_op_gather_push(hipStream_t s, R* x, R* y, R* vx, R* vy, int64_t n, const double* ex,
-                           const double* ey, int nx, int ny, double lx, double ly, double dt,
-                           double qm, double c, double* ke_partials, int nblocks);
+void launch_op_gather_push(hipStream_t s, const GatherPushPlan& p, R* x, R* y, R* vx, R* vy,
+                           int64_t n, const double* ex, const double* ey, int nx, int ny,
+                           double lx, double ly, double dt, double qm, double c,
+                           double* ke_partials, void* pairs);
 void launch_op_fixed_to_double(hipStream_t s, const unsigned long long* hi,
                                const unsigned long long* lo, long long G, int fp64,
                                double scale, double* out);

@@ -298,18 +298,23 @@ int pic_op_gather_push(void* x, void* y, void* vx, void* vy, int64_t n, int prec
   if (n < 0 || !ex || !ey || (n > 0 && (!x || !y || !vx || !vy))) return fail(PIC_ERR_ARG, "bad arrays");
   if (precision != PIC_FP32 && precision != PIC_FP64) return fail(PIC_ERR_ARG, "bad precision");
   hipStream_t s = (hipStream_t)stream;
-  long long b = (n + PIC_WG - 1) / PIC_WG;
-  const int nb = (int)std::max(1LL, std::min(b, 4096LL));
+  const bool fp64 = precision == PIC_FP64;
+  const GatherPushPlan p = gather_push_plan(n, g->nx, g->ny, fp64);
   DevMem m;
   double* parts = nullptr;
-  if (ke) PIC_HIP(m.get(&parts, nb));
-  if (precision == PIC_FP64)
-    launch_op_gather_push<double>(s, (double*)x, (double*)y, (double*)vx, (double*)vy, n, ex, ey,
-                                  g->nx, g->ny, g->lx, g->ly, dt, qm, c, parts, nb);
+  if (ke) PIC_HIP(m.get(&parts, p.blocks));
+  char* pairs = nullptr;
+  if (p.pairs && m.get(&pairs, (fp64 ? 16 : 8) * (size_t)p.pairs) != hipSuccess) {
+    (void)hipGetLastError();  // no memory for the packed field: the node arrays are read
+    pairs = nullptr;
+  }
+  if (fp64)
+    launch_op_gather_push<double>(s, p, (double*)x, (double*)y, (double*)vx, (double*)vy, n, ex,
+                                  ey, g->nx, g->ny, g->lx, g->ly, dt, qm, c, parts, pairs);
   else
-    launch_op_gather_push<float>(s, (float*)x, (float*)y, (float*)vx, (float*)vy, n, ex, ey, g->nx,
-                                 g->ny, g->lx, g->ly, dt, qm, c, parts, nb);
-  if (ke) launch_reduce_sum(s, parts, nb, ke);
+    launch_op_gather_push<float>(s, p, (float*)x, (float*)y, (float*)vx, (float*)vy, n, ex, ey,
+                                 g->nx, g->ny, g->lx, g->ly, dt, qm, c, parts, pairs);
+  if (ke) launch_reduce_sum(s, parts, p.blocks, ke);
   PIC_HIP(hipGetLastError());
   PIC_HIP(hipStreamSynchronize(s));
   return PIC_OK;
