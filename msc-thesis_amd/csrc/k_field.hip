@@ -13,10 +13,14 @@
 //   field   : Ex + i Ey from one inverse complex row FFT per row (groups of rows per
 //             workgroup); writes the padded (Ex, Ey) node array and the field energy
 //             (fixed-order reduction)
+// A solve that wants phi alone (pic_op_poisson) transforms one output per column instead of
+// three and skips the field pass: at 1024^2 the column pass took 42 us (four rows of a column
+// left room for one workgroup per CU) and takes 16.5, the field pass took 20.
 // Inside a captured sequence of steps the three kernels also run the previous step's
 // end-of-step work in extra workgroups after their own items (step_tail.h): its
 // diagnostics row (rows) and step counter (columns), and on the step after a count step
 // the fused sort's count-table scan (rows, columns, field).
+#include <algorithm>
 #include <type_traits>
 #include "fft_lds.h"
 #include "launch.h"
@@ -107,13 +111,16 @@ __device__ __forceinline__ void fft_col_item(const FieldArgs& a, double2* lds) {
   const RunDesc rd = a.runs[it.x];
   const int nx = rd.nx, ny = rd.ny, lognx = rd.lognx;
   const int k = it.y;
-  // nxp slots per row; A, B, C back to back (row r of a buffer starts at slot r nxp)
+  // nxp slots per row; the outputs back to back (row r of a buffer starts at slot r nxp): Ex,
+  // Ey and, when wanted, phi, or phi alone
   const int nxp = fft_slot<PAD>(nx), mxp = a.max_nx + (a.max_nx >> 3);
+  const bool want_E = !a.phi_only;
+  const int nout = want_E ? (a.want_phi ? 3 : 2) : 1;
   double2* col = lds;
   double2* A = lds + nxp;
   double2* B = lds + 2 * nxp;
-  double2* C = lds + 3 * nxp;
-  double2* twl = lds + (a.want_phi ? 4 : 3) * mxp;
+  double2* C = lds + nout * nxp;
+  double2* twl = lds + (1 + nout) * mxp;
   double2* S = a.S + rd.sbase + (long long)k * nx;
   fft_stage_twiddles(twl, nx, a.tw);
   for (int i = threadIdx.x; i < nx; i += PIC_WG) col[fft_slot<PAD>(bitrev(i, lognx))] = S[i];
@@ -143,20 +150,24 @@ __device__ __forceinline__ void fft_col_item(const FieldArgs& a, double2* lds) {
     const double2 r = col[fft_slot<PAD>(m)];
     double2 ph = make_double2(0.0, 0.0);
     if (m != 0 || k != 0) ph = make_double2(r.x / k2, r.y / k2);
-    const double sx = sin2pi_frac(m, nx, twl, lognx) / rd.dx;
     const int br = fft_slot<PAD>(bitrev(m, lognx));
-    A[br] = make_double2(sx * ph.y, -sx * ph.x);
-    B[br] = make_double2(sy * ph.y, -sy * ph.x);
+    if (want_E) {
+      const double sx = sin2pi_frac(m, nx, twl, lognx) / rd.dx;
+      A[br] = make_double2(sx * ph.y, -sx * ph.x);
+      B[br] = make_double2(sy * ph.y, -sy * ph.x);
+    }
     if (a.want_phi) C[br] = ph;
   }
   __syncthreads();
-  fft_lds_rows<PAD>(A, a.want_phi ? 3 : 2, nx, lognx, +1, twl, lognx);  // A, B, C consecutive
+  fft_lds_rows<PAD>(A, nout, nx, lognx, +1, twl, lognx);  // the outputs, consecutive rows
   double2* Sx = a.Sx + rd.sbase + (long long)k * nx;
   double2* Sy = a.Sy + rd.sbase + (long long)k * nx;
   for (int i = threadIdx.x; i < nx; i += PIC_WG) {
     const int q = fft_slot<PAD>(i);
-    Sx[i] = A[q];
-    Sy[i] = B[q];
+    if (want_E) {
+      Sx[i] = A[q];
+      Sy[i] = B[q];
+    }
     if (a.want_phi) S[i] = C[q];
   }
 }
@@ -253,10 +264,10 @@ __global__ __launch_bounds__(PIC_WG) void k_op_efield(const double* __restrict__
                                                       double* __restrict__ ex,
                                                       double* __restrict__ ey, int nx, int ny,
                                                       double dx, double dy) {
-  const long long G = (long long)nx * ny;
-  for (long long q = blockIdx.x * (long long)PIC_WG + threadIdx.x; q < G;
-       q += (long long)gridDim.x * PIC_WG) {
-    const int i = (int)(q / ny), j = (int)(q % ny);
+  const int lny = 31 - __clz(ny);
+  const int G = nx * ny;
+  for (int q = blockIdx.x * PIC_WG + threadIdx.x; q < G; q += gridDim.x * PIC_WG) {
+    const int i = q >> lny, j = q & (ny - 1);
     const int im = i == 0 ? nx - 1 : i - 1, ip = i == nx - 1 ? 0 : i + 1;
     const int jm = j == 0 ? ny - 1 : j - 1, jp = j == ny - 1 ? 0 : j + 1;
     ex[q] = (phi[(long long)im * ny + j] - phi[(long long)ip * ny + j]) / (2.0 * dx);
@@ -296,6 +307,22 @@ __global__ __launch_bounds__(PIC_WG) void k_rho_to_double(const RunDesc* __restr
     out[q] = fixed_to_density(h[q], fp64 ? l[q] : 0ull, fp64, rd.rho_scale) + background;
 }
 
+// Descriptor, state and work items of a one-grid solve, written on the device: the row pairs
+// (0, i * 2 fft_pp) and the columns (0, k).  (Copies of them from the host cost 15-20 us each.)
+__global__ __launch_bounds__(PIC_WG) void k_op_setup(RunDesc d, RunDesc* dd, RunState* st,
+                                                     int2* rp, int nrp, int2* cl, int ncl) {
+  const int t = blockIdx.x * PIC_WG + threadIdx.x;
+  if (t == 0) {
+    *dd = d;
+    RunState z;
+    z.np = z.nsorted = z.vsync = z.err = 0;
+    z.step = z.next_id = 0;
+    *st = z;
+  }
+  if (t < nrp) rp[t] = make_int2(0, t * 2 * d.fft_pp);
+  if (t < ncl) cl[t] = make_int2(0, t);
+}
+
 inline int grid_for(long long n) {
   long long b = (n + PIC_WG - 1) / PIC_WG;
   return (int)(b < 1 ? 1 : (b > 8192 ? 8192 : b));
@@ -307,7 +334,7 @@ void launch_field(hipStream_t s, const FieldArgs& a, hipEvent_t* ev) {
   // data, then the n/2 twiddles of the transform length
   const size_t lrow = ((size_t)a.row_lds + a.max_ny / 2) * sizeof(double2);
   const size_t lcol = (size_t)(a.max_nx + a.max_nx / 8) * sizeof(double2) *
-                          (a.want_phi ? 4 : 3) +
+                          (a.phi_only ? 2 : (a.want_phi ? 4 : 3)) +
                       (size_t)(a.max_nx / 2) * sizeof(double2);
   // extra workgroups of the folded end-of-step work
   const int xrows = (a.fold_finish ? a.nruns : 0) + (a.fold_scan ? a.nfscan_items : 0);
@@ -317,12 +344,20 @@ void launch_field(hipStream_t s, const FieldArgs& a, hipEvent_t* ev) {
   if (ev) (void)hipEventRecord(ev[1], s);
   k_fft_cols<<<a.n_col_items + xcols, PIC_WG, lcol, s>>>(a);
   if (ev) (void)hipEventRecord(ev[2], s);
-  if (a.fp64)
+  if (a.phi_only)
+    ;  // the caller wants no E
+  else if (a.fp64)
     k_fft_field<double, 0><<<a.n_row_items + xfield, PIC_WG, lrow, s>>>(a);
   else
     k_fft_field<float, 0><<<a.n_row_items + xfield, PIC_WG, lrow, s>>>(a);
   if (a.want_phi && a.phi) k_fft_field<float, 1><<<a.n_row_pair_items, PIC_WG, lrow, s>>>(a);
   if (ev) (void)hipEventRecord(ev[3], s);
+}
+
+void launch_op_setup(hipStream_t s, const RunDesc& d, RunDesc* dd, RunState* st, int2* rp,
+                     int nrp, int2* cl, int ncl) {
+  k_op_setup<<<(std::max(nrp, ncl) + PIC_WG - 1) / PIC_WG, PIC_WG, 0, s>>>(d, dd, st, rp, nrp, cl,
+                                                                          ncl);
 }
 
 void launch_op_efield(hipStream_t s, const double* phi, double* ex, double* ey, int nx, int ny,

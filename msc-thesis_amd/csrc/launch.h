@@ -227,6 +227,7 @@ struct FieldArgs {
   int nruns;
   int fp64;                          // particle precision (E type, rho words)
   int want_phi;
+  int phi_only;                      // 1 (with want_phi): no Ex, Ey transforms, E untouched
   int max_nx, max_ny;                // largest grid of the context (LDS sizing)
   int row_lds;                       // complex values per row-pass workgroup: the largest
                                      // max(fft_pp, fft_rf) * ny over the runs
@@ -249,6 +250,9 @@ struct FieldArgs {
   int* ftoff;                        // tile offsets of the order the next push writes
 };
 void launch_field(hipStream_t s, const FieldArgs& a, hipEvent_t* ev /* 4 events or NULL */);
+// one-grid descriptor, state and items into device memory (all of them read by launch_field)
+void launch_op_setup(hipStream_t s, const RunDesc& d, RunDesc* dd, RunState* st, int2* rp,
+                     int nrp, int2* cl, int ncl);
 void launch_op_efield(hipStream_t s, const double* phi, double* ex, double* ey, int nx, int ny,
                       double lx, double ly);
 // copy padded E (float/double pairs) of one run out to two FP64 node arrays

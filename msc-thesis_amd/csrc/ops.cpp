@@ -161,10 +161,35 @@ int pic_op_deposit(const void* x, const void* y, int64_t n, int precision, const
 // copy (16 MiB) until the process ends.  In host code the array's name is only a
 // stand-in symbol: its device address comes from hipGetSymbolAddress, once per device.
 static __device__ __align__(256) unsigned long long scratch[2 * PIC_DEPOSIT_NOALLOC_MAX_NODES];
+// Twiddles of the field solve, exp(-2 pi i j / PIC_FFT_MAX): 16 KiB per device, filled on the
+// first call there.
+static __device__ double2 op_tw[PIC_FFT_MAX / 2];
 
 namespace {
 std::mutex g_scratch_mu;
 unsigned long long* g_scratch_ptr[64];  // device address of `scratch` per device ordinal
+double2* g_tw_ptr[64];                  // device address of `op_tw`, once filled
+
+int op_twiddles(double2** out) {
+  int dev = 0;
+  PIC_HIP(hipGetDevice(&dev));
+  if (dev < 0 || dev >= 64) return fail(PIC_ERR_UNSUPPORTED, "device ordinal above 63");
+  std::lock_guard<std::mutex> lk(g_scratch_mu);
+  if (!g_tw_ptr[dev]) {
+    std::vector<double2> h(PIC_FFT_MAX / 2);
+    for (int j = 0; j < PIC_FFT_MAX / 2; ++j) {
+      const long double a = 2.0L * 3.141592653589793238462643383279L * j / PIC_FFT_MAX;
+      h[j] = make_double2((double)cosl(a), (double)-sinl(a));
+    }
+    void* p = nullptr;
+    PIC_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(op_tw)));
+    // synchronous: in place before any stream's kernel reads it
+    PIC_HIP(hipMemcpy(p, h.data(), sizeof(double2) * h.size(), hipMemcpyHostToDevice));
+    g_tw_ptr[dev] = (double2*)p;
+  }
+  *out = g_tw_ptr[dev];
+  return PIC_OK;
+}
 
 // Device address of `scratch` on the current device, looked up on the first call there.
 int noalloc_scratch(unsigned long long** out) {
@@ -230,50 +255,29 @@ int pic_op_poisson(const double* rho, double* phi, const pic_grid* g, void* stre
   if (!rho || !phi) return fail(PIC_ERR_ARG, "NULL array");
   hipStream_t s = (hipStream_t)stream;
   const int nx = g->nx, ny = g->ny;
-  DevMem m;
+  double2* tw = nullptr;
+  if ((rc = op_twiddles(&tw))) return rc;
   RunDesc d = op_desc(nx, ny, g->lx, g->ly, 0);
-  d.row_item_begin = 0;
-  d.row_item_end = nx / d.fft_rf;
+  const int nrp = nx / (2 * d.fft_pp), ncl = ny / 2 + 1;
+  const size_t ss = (size_t)ncl * nx;
+  DevMem m;
+  double2* S;
   RunDesc* dd;
   RunState* st;
+  int2* items;
+  PIC_HIP(m.get(&S, ss));
   PIC_HIP(m.get(&dd, 1));
   PIC_HIP(m.get(&st, 1));
-  PIC_HIP(hipMemsetAsync(st, 0, sizeof(RunState), s));
-  PIC_HIP(hipMemcpyAsync(dd, &d, sizeof(d), hipMemcpyHostToDevice, s));
-  const long long ss = (long long)(ny / 2 + 1) * nx;
-  double2 *S, *Sx, *Sy, *tw;
-  float* E;
-  PIC_HIP(m.get(&S, ss));
-  PIC_HIP(m.get(&Sx, ss));
-  PIC_HIP(m.get(&Sy, ss));
-  PIC_HIP(m.get(&E, 2 * (size_t)(nx + 1) * (ny + 1)));
-  PIC_HIP(m.get(&tw, PIC_FFT_MAX / 2));
-  std::vector<double2> h(PIC_FFT_MAX / 2);
-  for (int j = 0; j < PIC_FFT_MAX / 2; ++j) {
-    const long double a = 2.0L * 3.141592653589793238462643383279L * j / PIC_FFT_MAX;
-    h[j] = make_double2((double)cosl(a), (double)-sinl(a));
-  }
-  PIC_HIP(hipMemcpyAsync(tw, h.data(), sizeof(double2) * h.size(), hipMemcpyHostToDevice, s));
-  std::vector<int2> rp, cl, rw;
-  for (int i = 0; i < nx; i += 2 * d.fft_pp) rp.push_back(make_int2(0, i));
-  for (int k = 0; k <= ny / 2; ++k) cl.push_back(make_int2(0, k));
-  for (int i = 0; i < nx; i += d.fft_rf) rw.push_back(make_int2(0, i));
-  int2 *drp, *dcl, *drw;
-  PIC_HIP(m.get(&drp, rp.size()));
-  PIC_HIP(m.get(&dcl, cl.size()));
-  PIC_HIP(m.get(&drw, rw.size()));
-  PIC_HIP(hipMemcpyAsync(drp, rp.data(), sizeof(int2) * rp.size(), hipMemcpyHostToDevice, s));
-  PIC_HIP(hipMemcpyAsync(dcl, cl.data(), sizeof(int2) * cl.size(), hipMemcpyHostToDevice, s));
-  PIC_HIP(hipMemcpyAsync(drw, rw.data(), sizeof(int2) * rw.size(), hipMemcpyHostToDevice, s));
+  PIC_HIP(m.get(&items, (size_t)nrp + ncl));
+  launch_op_setup(s, d, dd, st, items, nrp, items + nrp, ncl);
   FieldArgs a;
   std::memset(&a, 0, sizeof(a));
   a.runs = dd; a.st = st;
-  a.S = S; a.Sx = Sx; a.Sy = Sy; a.E = E; a.phi = phi; a.tw = tw;
-  a.row_pair_items = drp; a.n_row_pair_items = (int)rp.size();
-  a.col_items = dcl; a.n_col_items = (int)cl.size();
-  a.row_items = drw; a.n_row_items = (int)rw.size();
-  a.nruns = 1; a.fp64 = 0; a.want_phi = 1; a.max_nx = nx; a.max_ny = ny;
-  a.row_lds = std::max(d.fft_pp, d.fft_rf) * ny;
+  a.S = S; a.phi = phi; a.tw = tw;
+  a.row_pair_items = items; a.n_row_pair_items = nrp;
+  a.col_items = items + nrp; a.n_col_items = ncl;
+  a.nruns = 1; a.fp64 = 0; a.want_phi = 1; a.phi_only = 1; a.max_nx = nx; a.max_ny = ny;
+  a.row_lds = d.fft_pp * ny;
   a.rho_in = rho;
   launch_field(s, a, nullptr);
   PIC_HIP(hipGetLastError());
