@@ -32,7 +32,7 @@ struct pic_adjoint {
   double *xl = nullptr, *yl = nullptr, *mkx = nullptr, *mky = nullptr;
   void *x = nullptr, *y = nullptr, *vx = nullptr, *vy = nullptr;
   void* ckpt = nullptr;                       // nseg x 4 x n
-  void *trx = nullptr, *try_ = nullptr;       // (K+1) x n
+  void *trx = nullptr, *try_ = nullptr;       // K x n: positions after a segment's steps
   void* trE = nullptr;                        // nsteps x padded field (E_0 .. E_{N-1})
   double *lE = nullptr, *lrho = nullptr;
   unsigned long long *hi = nullptr, *lo = nullptr;
@@ -112,38 +112,38 @@ inline double kick(int k) { return k == 0 ? 0.5 : 1.0; }
 // saving (x, y, vx, vy) every K steps; then E_N and its energy partials.
 template <typename R>
 void record_forward(pic_adjoint& a) {
-  R *x = (R*)a.x, *y = (R*)a.y, *vx = (R*)a.vx, *vy = (R*)a.vy;
+  R* const cur[4] = {(R*)a.x, (R*)a.y, (R*)a.vx, (R*)a.vy};
   const size_t n = (size_t)a.n;
   for (int k = 0; k < a.nsteps; ++k) {
     R* Ek = (R*)a.at(a.trE, (size_t)k * a.epad());
     const int seg = k / a.K;
     const int* toff = a.toffs + (size_t)seg * (a.nb + 1);
+    const R* in[4] = {cur[0], cur[1], cur[2], cur[3]};
     if (k > 0) field(a, Ek);  // the charge of x_k (deposited by the previous push)
     if (k % a.K == 0) {
-      // checkpoint = the state sorted by tile; ids = each slot's slot before the sort
+      // checkpoint = the state sorted by tile; ids = each slot's slot before the sort.  The
+      // step's push reads the checkpoint itself.
       R* ck = (R*)a.at(a.ckpt, (size_t)seg * 4 * n);
-      PartBufs<R> src{x, y, vx, vy, a.iota};
+      PartBufs<R> src{cur[0], cur[1], cur[2], cur[3], a.iota};
       PartBufs<R> dst{ck, ck + n, ck + 2 * n, ck + 3 * n, a.ids + (size_t)seg * n};
       SortBufs sb = a.sb;
       sb.toff = a.toffs + (size_t)seg * (a.nb + 1);
       launch_tile_sort<R>(a.s, a.dd, a.st, 1, src, dst, sb, a.pitems, a.npitems);
-      R* cur[4] = {x, y, vx, vy};
-      for (int q = 0; q < 4; ++q)
-        (void)hipMemcpyAsync(cur[q], ck + q * n, a.rs * n, hipMemcpyDeviceToDevice, a.s);
+      for (int q = 0; q < 4; ++q) in[q] = ck + q * n;
     }
     if (k == 0) {  // the initial charge, deposited once the particles are sorted
-      adj_push_win<R>(a.s, a.g, a.items, toff, x, y, vx, vy, nullptr, 0.0, a.hi, a.lo);
+      adj_push_win<R>(a.s, a.g, a.items, toff, in, cur, nullptr, 0.0, a.hi, a.lo);
       field(a, Ek);
     }
-    adj_push_win<R>(a.s, a.g, a.items, toff, x, y, vx, vy, Ek, kick(k), a.hi, a.lo);
+    adj_push_win<R>(a.s, a.g, a.items, toff, in, cur, Ek, kick(k), a.hi, a.lo);
   }
   field(a, a.E);
   adj_energy<R>(a.s, a.g, (const R*)a.E, a.part, kEnergyBlocks);
 }
 
 // Reverse sweep for dL = 1 (the caller scales the outputs): seed from E_N, then for each
-// segment restore its checkpoint, recompute its steps into the trajectory buffers (pushes
-// in the stored fields of the forward) and run the reverse steps over them.
+// segment recompute the positions of its steps from its checkpoint (pushes in the stored
+// fields of the forward) and run the reverse steps over them.
 template <typename R>
 void record_backward(pic_adjoint& a) {
   const size_t n = (size_t)a.n;
@@ -153,8 +153,7 @@ void record_backward(pic_adjoint& a) {
   adj_zero(a.s, a.lam[cur], 4 * a.n);
   auto L = [&](int k) { return a.lam[cur] + (size_t)k * n; };
   const double cq = a.qp / (a.g.dx * a.g.dy);
-  auto X = [&](int slot) { return (R*)a.at(a.trx, (size_t)slot * n); };
-  auto Y = [&](int slot) { return (R*)a.at(a.try_, (size_t)slot * n); };
+  R *xs = (R*)a.trx, *ys = (R*)a.try_;
   auto Ek = [&](int k) { return (R*)a.at(a.trE, (size_t)k * a.epad()); };
   for (int seg = a.nseg - 1; seg >= 0; --seg) {
     const int k0 = seg * a.K, k1 = std::min(k0 + a.K, a.nsteps);
@@ -165,13 +164,11 @@ void record_backward(pic_adjoint& a) {
       adj_reorder(a.s, a.ids + (size_t)(seg + 1) * n, a.lam[cur], a.lam[1 - cur], a.n);
       cur = 1 - cur;
     }
-    adj_restore<R>(a.s, a.g, (const R*)a.at(a.ckpt, (size_t)seg * 4 * n), a.n, X(0), Y(0),
-                   (R*)a.vx, (R*)a.vy, nullptr, nullptr);
-    for (int k = k0; k < k1; ++k) {
-      const int sl = k - k0;
-      adj_push<R>(a.s, a.g, X(sl), Y(sl), X(sl + 1), Y(sl + 1), (R*)a.vx, (R*)a.vy, Ek(k), a.n,
-                  kick(k), nullptr, nullptr, nullptr);
-    }
+    const R* ck = (const R*)a.at(a.ckpt, (size_t)seg * 4 * n);
+    // positions at step k0 + sl: the checkpoint's, then the recomputed ones
+    auto X = [&](int sl) { return sl ? xs + (size_t)(sl - 1) * n : ck; };
+    auto Y = [&](int sl) { return sl ? ys + (size_t)(sl - 1) * n : ck + n; };
+    adj_segment<R>(a.s, a.g, ck, Ek(k0), (long long)a.epad(), k0, k1 - k0, xs, ys, a.n);
     for (int k = k1; k > k0; --k) {
       const int sl = k - k0;
       adj_pass_win<R>(a.s, a.g, a.items, toff, X(sl), Y(sl), a.lrho, cq, X(sl - 1), Y(sl - 1),
@@ -179,9 +176,9 @@ void record_backward(pic_adjoint& a) {
       adj_mt(a.s, a.g, a.lE, a.A, a.lrho, a.tw);
     }
   }
-  // deposit Jacobian of step 0 at x_0 (slot 0 of segment 0)
-  adj_pass<R>(a.s, a.g, X(0), Y(0), a.lrho, cq, nullptr, nullptr, nullptr, 0.0, L(0), L(1),
-              L(2), L(3), a.lE, a.n);
+  // deposit Jacobian of step 0 at x_0 (the checkpoint of segment 0)
+  const R* c0 = (const R*)a.ckpt;
+  adj_pass_end<R>(a.s, a.g, c0, c0 + n, a.lrho, cq, L(0), L(1), a.n);
   // results in the original particle order (segment 0 was sorted from it)
   adj_reorder(a.s, a.ids, a.lam[cur], a.lam[1 - cur], a.n);
   a.res = a.lam[1 - cur];
@@ -295,13 +292,13 @@ int pic_adjoint_create(const pic_config* cfg, const double* xl, const double* yl
   PIC_HIP(A.getb(&A.vx, A.rs * n));
   PIC_HIP(A.getb(&A.vy, A.rs * n));
   PIC_HIP(A.getb(&A.ckpt, A.rs * 4 * n * A.nseg));
-  PIC_HIP(A.getb(&A.trx, A.rs * n * (A.K + 1)));
-  PIC_HIP(A.getb(&A.try_, A.rs * n * (A.K + 1)));
+  PIC_HIP(A.getb(&A.trx, A.rs * n * A.K));
+  PIC_HIP(A.getb(&A.try_, A.rs * n * A.K));
   PIC_HIP(A.getb(&A.trE, A.rs * A.epad() * (size_t)nsteps));
   PIC_HIP(A.get(&A.lam[0], 4 * (size_t)n));
   PIC_HIP(A.get(&A.lam[1], 4 * (size_t)n));
   PIC_HIP(A.get(&A.lE, 2 * G));
-  PIC_HIP(A.get(&A.lrho, G));
+  PIC_HIP(A.get(&A.lrho, A.epad() / 2));
   PIC_HIP(A.get(&A.hi, G));
   PIC_HIP(A.get(&A.lo, G));
   PIC_HIP(A.getb(&A.E, A.rs * A.epad()));
@@ -358,6 +355,9 @@ int pic_adjoint_create(const pic_config* cfg, const double* xl, const double* yl
     d.win = g.win; d.splits = g.splits; d.nbuckets = A.nb;
     // sort chunks of 1024 particles: the adjoint's runs are small (config 5: 512 chunks)
     d.schunk = 1024;
+    // tiles of the positions half a segment on: the drift of a segment is half of it either
+    // way, so fewer nodes of the windows are touched (each costs an item's flush an atomic)
+    d.sort_lead = 0.5 * std::min(A.K, nsteps) * cfg->dt;
     d.nchunks = (int)((n + d.schunk - 1) / d.schunk);
     d.pcap = (int)n; d.tbase = 0; d.toffbase = 0; d.pbase = 0;
     std::vector<int2> ts, pi;

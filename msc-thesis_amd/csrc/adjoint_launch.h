@@ -14,25 +14,24 @@ template <typename R>
 void adj_init(hipStream_t s, const AdjGrid& g, const double* xl, const double* yl, int64_t n,
               const double* amps, const double* mkx, const double* mky, int nm, R* x, R* y,
               unsigned long long* hi, unsigned long long* lo);
+// positions after each of the nst steps that follow a checkpoint ck (taken before step k0), in
+// the stored fields Eseg, Eseg + estride, ...: xs, ys hold n entries per step
 template <typename R>
-void adj_push(hipStream_t s, const AdjGrid& g, const R* xi, const R* yi, R* xo, R* yo, R* vx,
-              R* vy, const R* E, int64_t n, double c, R* ck, unsigned long long* hi,
-              unsigned long long* lo);
-template <typename R>
-void adj_restore(hipStream_t s, const AdjGrid& g, const R* ck, int64_t n, R* x, R* y, R* vx,
-                 R* vy, unsigned long long* hi, unsigned long long* lo);
+void adj_segment(hipStream_t s, const AdjGrid& g, const R* ck, const R* Eseg, long long estride,
+                 int k0, int nst, R* xs, R* ys, int64_t n);
 void adj_zero(hipStream_t s, double* a, long long n);
+// deposit Jacobian of step 0; lrho here and below: (nx + 1) x (ny + 1) padded nodes
 template <typename R>
-void adj_pass(hipStream_t s, const AdjGrid& g, const R* xk, const R* yk, const double* lrho,
-              double cq, const R* xp, const R* yp, const R* Eprev, double ck1, double* lx,
-              double* ly, double* lvx, double* lvy, double* lE, int64_t n);
-// forward step of tile-sorted particles (in place) with LDS windows for the field and
-// the new charge; items {tile x, tile y, split} over the tile offsets `toff`.  E == NULL:
-// deposit the charge of the positions as they are, no push
+void adj_pass_end(hipStream_t s, const AdjGrid& g, const R* xk, const R* yk, const double* lrho,
+                  double cq, double* lx, double* ly, int64_t n);
+// forward step of tile-sorted particles with LDS windows for the field and the new charge,
+// from the arrays in (x, y, vx, vy) to out (may be the same); items {tile x, tile y, split}
+// over the tile offsets `toff`.  E == NULL: deposit the charge of the positions as they are,
+// no push
 template <typename R>
-void adj_push_win(hipStream_t s, const AdjGrid& g, const int4* items, const int* toff, R* x,
-                  R* y, R* vx, R* vy, const R* E, double c, unsigned long long* hi,
-                  unsigned long long* lo);
+void adj_push_win(hipStream_t s, const AdjGrid& g, const int4* items, const int* toff,
+                  const R* const in[4], R* const out[4], const R* E, double c,
+                  unsigned long long* hi, unsigned long long* lo);
 // reverse step of tile-sorted particles; the E sensitivity is summed in an LDS window
 template <typename R>
 void adj_pass_win(hipStream_t s, const AdjGrid& g, const int4* items, const int* toff,
