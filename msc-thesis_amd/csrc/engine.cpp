@@ -148,7 +148,7 @@ Ctx::~Ctx() {
   free_graphs();
   auto F = [](void* p) { if (p) (void)hipFree(p); };
   F(d_runs); F(d_st);
-  for (int i = 0; i < 2; ++i) { F(px[i]); F(py[i]); F(pvx[i]); F(pvy[i]); F(pid[i]); }
+  for (int i = 0; i < 2; ++i) { F(px[i]); F(pid[i]); }
   F(rho); F(rho_lo); F(E); F(S); F(Sx); F(Sy); F(phi); F(tw);
   F(sb.keys); F(sb.rank); F(sb.perm); F(sb.counts); F(sb.offsets); F(sb.chunk_sums);
   F(sb.big_list); F(sb.big_count); F(sb.scratch); F(sb.table); F(sb.tchunk_sums);
@@ -177,7 +177,7 @@ int Ctx::upload_runs() {
 
 int Ctx::build_items() {
   pitems.clear(); citems.clear(); rowpair.clear(); cols.clear(); rows.clear(); push_items.clear();
-  segitems.clear(); tscan_items.clear();
+  segitems.clear(); tscan_items.clear(); rp_begin.clear(); col_begin.clear();
   lds_push = 0;
   long long tsum = 0;
   toffsum = 0;
@@ -216,12 +216,16 @@ int Ctx::build_items() {
     push_items_for(r, nullptr);
     d.fchunks = 0;
     fft_groups(rows_total, d.nx, d.ny, &d.fft_pp, &d.fft_rf);
+    rp_begin.push_back((int)rowpair.size());
+    col_begin.push_back((int)cols.size());
     for (int i = 0; i < d.nx; i += 2 * d.fft_pp) rowpair.push_back(make_int2(r, i));
     for (int k = 0; k <= d.ny / 2; ++k) cols.push_back(make_int2(r, k));
     d.row_item_begin = (int)rows.size();
     for (int i = 0; i < d.nx; i += d.fft_rf) rows.push_back(make_int2(r, i));
     d.row_item_end = (int)rows.size();
   }
+  rp_begin.push_back((int)rowpair.size());
+  col_begin.push_back((int)cols.size());
   if (lds_push > 160 * 1024) return fail(PIC_ERR_INVALID_CONFIG, "deposit window exceeds LDS");
   // Sort fused into the push: needs no cell lists (no DSMC), a cadence of at least two
   // steps (the count is taken one step ahead), and room in LDS for one counter per tile
@@ -349,10 +353,10 @@ int Ctx::alloc() {
   PIC_HIP(dalloc(&d_st, nruns));
   const size_t rs = rsize;
   for (int i = 0; i < 2; ++i) {
-    PIC_HIP(hipMalloc(&px[i], rs * ptotal));
-    PIC_HIP(hipMalloc(&py[i], rs * ptotal));
-    PIC_HIP(hipMalloc(&pvx[i], rs * ptotal));
-    PIC_HIP(hipMalloc(&pvy[i], rs * ptotal));
+    PIC_HIP(hipMalloc(&px[i], 4 * rs * ptotal));
+    py[i] = (char*)px[i] + rs * ptotal;
+    pvx[i] = (char*)py[i] + rs * ptotal;
+    pvy[i] = (char*)pvx[i] + rs * ptotal;
     PIC_HIP(dalloc(&pid[i], ptotal));
   }
   PIC_HIP(dalloc(&rho, 2 * gsum));
@@ -451,9 +455,16 @@ PushArgs<R> Ctx::push_args(int mode, int sort_mode) const {
   return a;
 }
 
-int Ctx::launch_field_stage(int want_phi, hipEvent_t* ev4) {
+int Ctx::launch_field_run(int run, int want_phi) {
   FieldArgs a = field_args(want_phi);
-  launch_field(stream, a, ev4);
+  a.row_pair_items += rp_begin[run];
+  a.n_row_pair_items = rp_begin[run + 1] - rp_begin[run];
+  a.col_items += col_begin[run];
+  a.n_col_items = col_begin[run + 1] - col_begin[run];
+  a.row_items += rd[run].row_item_begin;
+  a.n_row_items = rd[run].row_item_end - rd[run].row_item_begin;
+  a.partials += rd[run].row_item_begin;  // the field-energy partials go by row item
+  launch_field(stream, a, nullptr);
   return PIC_OK;
 }
 
@@ -881,6 +892,13 @@ static int read_state(Ctx& x, int run, RunState* s) {
   return PIC_OK;
 }
 
+// Particles up to which the output arrays are written directly: a launch less.  Whole calls
+// (state read, field, output), direct against records, FP32 (us): 59 / 65 at 10,000 particles,
+// 66 / 63 at 100,000, 104 / 76 at 1,000,001, 247 / 128 at 4,000,001, 1094 / 555 at 16,777,216.
+static const int OUT_DIRECT_MAX = 1 << 16;
+
+// Records of an output live in the run's slice of the particle buffer that is not in use (the
+// next sort overwrites it).
 template <typename R>
 static int get_particles_t(Ctx& x, int run, void* ox, void* oy, void* ovx, void* ovy, int64_t n,
                            int sync, bool device_dst) {
@@ -889,40 +907,46 @@ static int get_particles_t(Ctx& x, int run, void* ox, void* oy, void* ovx, void*
   if (rc) return rc;
   if (n < s.np) return fail(PIC_ERR_ARG, "output arrays smaller than the particle count");
   const int np = s.np;
-  R *t = nullptr;
-  PIC_HIP(dalloc(&t, 6 * (size_t)std::max(np, 1)));
-  R *tx = t, *ty = t + np, *tvx = t + 2 * (size_t)np, *tvy = t + 3 * (size_t)np;
-  R *svx = nullptr, *svy = nullptr;
+  const R* E = nullptr;
   if (sync && !s.vsync) {
-    svx = t + 4 * (size_t)np;
-    svy = t + 5 * (size_t)np;
-    x.launch_field_stage(0);
-    launch_half_kick_out<R>(x.stream, x.d_runs, x.d_st, run, x.bufs<R>(x.cur), (const R*)x.E, svx,
-                            svy, x.d_pitems, (int)x.pitems.size());
+    x.launch_field_run(run, 0);
+    E = (const R*)x.E;
   }
-  launch_unpermute<R>(x.stream, x.d_runs, x.d_st, run, x.bufs<R>(x.cur), svx, svy, tx, ty, tvx, tvy,
-                      x.d_pitems, (int)x.pitems.size());
+  R* rec = (R*)x.px[1 - x.cur] + 4 * x.rd[run].pbase;
+  const PartBufs<R> p = x.bufs<R>(x.cur);
+  if (device_dst) {
+    // on the null stream, so that the writes are ordered with the caller's work on it
+    PIC_HIP(hipEventRecord(x.ev[0], x.stream));
+    PIC_HIP(hipStreamWaitEvent(nullptr, x.ev[0], 0));
+    if (np <= OUT_DIRECT_MAX) {
+      launch_out_particles<R>(nullptr, x.d_runs, x.d_st, run, np, p, E, nullptr, (R*)ox, (R*)oy,
+                              (R*)ovx, (R*)ovy);
+    } else {
+      launch_out_particles<R>(nullptr, x.d_runs, x.d_st, run, np, p, E, rec, nullptr, nullptr,
+                              nullptr, nullptr);
+      launch_out_split<R>(nullptr, rec, np, (R*)ox, (R*)oy, (R*)ovx, (R*)ovy);
+    }
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess)
+      return fail(PIC_ERR_HIP, std::string("get_particles: ") + hipGetErrorString(e));
+    return PIC_OK;
+  }
+  launch_out_particles<R>(x.stream, x.d_runs, x.d_st, run, np, p, E, rec, nullptr, nullptr,
+                          nullptr, nullptr);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(x.stream);
-  if (e != hipSuccess) {
-    (void)hipFree(t);
-    return fail(PIC_ERR_HIP, std::string("get_particles: ") + hipGetErrorString(e));
+  double* outs[4] = {(double*)ox, (double*)oy, (double*)ovx, (double*)ovy};
+  const int chunk = std::min(np, 1 << 20);
+  std::vector<R> h(4 * (size_t)chunk);
+  for (int b = 0; b < np && e == hipSuccess; b += chunk) {
+    const int m = std::min(chunk, np - b);
+    e = hipMemcpy(h.data(), rec + 4 * (size_t)b, 4 * sizeof(R) * m, hipMemcpyDeviceToHost);
+    for (int k = 0; k < 4; ++k)
+      if (outs[k])
+        for (int i = 0; i < m; ++i) outs[k][b + i] = (double)h[4 * (size_t)i + k];
   }
-  void* outs[4] = {ox, oy, ovx, ovy};
-  R* srcs[4] = {tx, ty, tvx, tvy};
-  for (int k = 0; k < 4; ++k) {
-    if (!outs[k]) continue;
-    if (device_dst) {
-      e = hipMemcpy(outs[k], srcs[k], sizeof(R) * np, hipMemcpyDeviceToDevice);
-    } else {
-      std::vector<R> h(np);
-      e = hipMemcpy(h.data(), srcs[k], sizeof(R) * np, hipMemcpyDeviceToHost);
-      for (int i = 0; i < np; ++i) ((double*)outs[k])[i] = (double)h[i];
-    }
-    if (e != hipSuccess) break;
-  }
-  (void)hipFree(t);
-  if (e != hipSuccess) return fail(PIC_ERR_HIP, std::string("get_particles copy: ") + hipGetErrorString(e));
+  if (e != hipSuccess) return fail(PIC_ERR_HIP, std::string("get_particles: ") + hipGetErrorString(e));
   return PIC_OK;
 }
 
@@ -1010,7 +1034,7 @@ int pic_get_grid(pic_ctx* ctx, int run, int which, double* out) {
   RunState s;
   int rc = read_state(x, run, &s);
   if (rc) { (void)hipFree(t); return rc; }
-  x.launch_field_stage(which == PIC_GRID_PHI);
+  x.launch_field_run(run, which == PIC_GRID_PHI);
   const double* src = t;
   if (which == PIC_GRID_RHO) {
     const double bg = -d.qp * s.np / (d.lx * d.ly);

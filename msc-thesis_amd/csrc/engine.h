@@ -56,6 +56,8 @@ struct Ctx {
 
   RunDesc* d_runs = nullptr;
   RunState* d_st = nullptr;
+  // x, y, vx, vy of a buffer are one allocation (at px), one after the other, so that the
+  // buffer not in use (a sort's target) can hold the 4-value records of an output
   void* px[2] = {nullptr, nullptr};
   void* py[2] = {nullptr, nullptr};
   void* pvx[2] = {nullptr, nullptr};
@@ -75,6 +77,7 @@ struct Ctx {
                                        // stage runs (its births are counted; else NULL)
   bool fused = false;                  // sort fused into the push (see build_items)
   std::vector<int2> pitems, citems, rowpair, cols, rows, segitems, tscan_items, fscan_items;
+  std::vector<int> rp_begin, col_begin;  // first row-pair and column item of each run
   std::vector<int4> push_items;
   int2 *d_pitems = nullptr, *d_citems = nullptr, *d_rowpair = nullptr, *d_cols = nullptr,
        *d_rows = nullptr, *d_segitems = nullptr, *d_tscan_items = nullptr,
@@ -119,7 +122,7 @@ struct Ctx {
   template <typename R> PushArgs<R> push_args(int mode, int sort_mode = 0) const;
 
   // launches (no synchronisation)
-  int launch_field_stage(int want_phi, hipEvent_t* ev4 = nullptr);
+  int launch_field_run(int run, int want_phi);  // the field of one run's current positions
   int launch_push_stage(int mode, int sort_mode = 0);
   int launch_sort_stage();
   int launch_collide_stage();

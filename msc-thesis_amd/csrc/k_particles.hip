@@ -707,113 +707,80 @@ __global__ void k_fill_u64(unsigned long long* p, long long n) {
 // is accumulated in an LDS window of (T+2H+1)^2 nodes around the tile with int64 atomics
 // and flushed once per workgroup; particles that drifted outside the window since the
 // last sort deposit straight to HBM.  Gather reads the padded E array (L2-resident).
-// gather + kick + drift of one particle; returns synchronous-velocity sums
-// E window in LDS: ew[r*W + c] = E at node (x0 + r, y0 + c) (periodic), or NULL
 template <typename R>
 struct EWin {
   typedef typename std::conditional<sizeof(R) == 4, float2, double2>::type R2;
-  const R2* ew;
-  int W, x0, y0;
 };
-
-template <typename R>
-__device__ __forceinline__ void push_one(R& xr, R& yr, R& vxr, R& vyr, const R* __restrict__ E,
-                                         const Geo<R>& g, R hk, R dtr, double skc, double& ke,
-                                         double& px, double& py, const EWin<R>& w) {
-  int cx, cy;
-  R fx, fy;
-  locate_w(xr, g.idx, g.nx, cx, fx);
-  locate_w(yr, g.idy, g.ny, cy, fy);
-  const R qs = (R)(1.0 / (double)(1 << Fix<R>::QB));
-  const R gx1 = (R)qweight(fx) * qs, gy1 = (R)qweight(fy) * qs;
-  const R gx0 = (R)1 - gx1, gy0 = (R)1 - gy1;
-  const R g00 = gx0 * gy0, g10 = gx1 * gy0, g01 = gx0 * gy1, g11 = gx1 * gy1;
-  typedef typename EWin<R>::R2 R2;
-  R2 e00, e01, e10, e11;
-  int rx = cx - w.x0, ry = cy - w.y0;
-  rx = pwrap(rx, g.nx);
-  ry = pwrap(ry, g.ny);
-  if (w.ew && rx < w.W - 1 && ry < w.W - 1) {
-    const int i0 = rx * w.W + ry;
-    e00 = w.ew[i0]; e01 = w.ew[i0 + 1]; e10 = w.ew[i0 + w.W]; e11 = w.ew[i0 + w.W + 1];
-  } else {
-    const R2* e = reinterpret_cast<const R2*>(E);
-    const long long i00 = (long long)cx * (g.ny + 1) + cy;
-    e00 = e[i00]; e01 = e[i00 + 1]; e10 = e[i00 + g.ny + 1]; e11 = e[i00 + g.ny + 2];
-  }
-  R epx = g00 * e00.x;
-  epx = fmar(g10, e10.x, epx);
-  epx = fmar(g01, e01.x, epx);
-  epx = fmar(g11, e11.x, epx);
-  R epy = g00 * e00.y;
-  epy = fmar(g10, e10.y, epy);
-  epy = fmar(g01, e01.y, epy);
-  epy = fmar(g11, e11.y, epy);
-  const double vsx = (double)vxr + skc * (double)epx, vsy = (double)vyr + skc * (double)epy;
-  ke += vsx * vsx + vsy * vsy;
-  px += vsx;
-  py += vsy;
-  vxr = fmar(hk, epx, vxr);
-  vyr = fmar(hk, epy, vyr);
-  xr = wrap_pos(fmar(dtr, vxr, xr), g.Lx);
-  yr = wrap_pos(fmar(dtr, vyr, yr), g.Ly);
-}
 
 #include "push_kernel.inc"
 
-// synchronous velocities for output: v + 1/2 dt qm E(x) when a half kick is pending
+// One particle's state as it leaves: (x, y, vx, vy) together.
 template <typename R>
-__global__ __launch_bounds__(PIC_WG) void k_half_kick_out(const RunDesc* __restrict__ runs,
+struct alignas(4 * sizeof(R)) OutRec {
+  R x, y, vx, vy;
+};
+
+// Particles of run `run` in id order.  KICK: synchronous velocities, v + 1/2 dt qm E(x) (the
+// pending half kick on the copy).  REC: one record per particle to rec[id], for
+// k_out_split; else straight to the output arrays (those that are not NULL).
+// The particles lie in tile order, so after some steps consecutive ones have unrelated ids and
+// every store is a line of its own: bound by those lines.  A record is one line where four
+// arrays are four (16,777,216 FP32 particles, the whole output call: 1697 us with the kick in a
+// launch of its own, four scattered stores and four copies, 555 with records).
+template <typename R, bool KICK, bool REC>
+__global__ __launch_bounds__(PIC_WG) void k_out_particles(const RunDesc* __restrict__ runs,
                                                           const RunState* __restrict__ st,
                                                           int run, PartBufs<R> p,
                                                           const R* __restrict__ Eall,
+                                                          OutRec<R>* __restrict__ rec,
+                                                          R* __restrict__ ox, R* __restrict__ oy,
                                                           R* __restrict__ ovx,
-                                                          R* __restrict__ ovy,
-                                                          const int2* __restrict__ items) {
-  const int2 it = items[blockIdx.x];
-  if (it.x != run) return;
+                                                          R* __restrict__ ovy) {
   const RunDesc rd = runs[run];
-  const RunState rs = st[run];
-  const Geo<R> g = make_geo<R>(rd.nx, rd.ny, rd.lx, rd.ly);
-  const R* E = Eall + 2 * rd.ebase;
-  const R hk = rs.vsync ? (R)0 : (R)(0.5 * rd.dt * rd.qm);
-  const int p1 = min(it.y + PIC_CHUNK, rs.np);
-  for (int q = it.y + threadIdx.x; q < p1; q += PIC_WG) {
-    const long long i = rd.pbase + q;
-    R xr = p.x[i], yr = p.y[i], vxr = p.vx[i], vyr = p.vy[i];
-    double ke = 0, px = 0, py = 0;
-    R x2 = xr, y2 = yr;
-    EWin<R> none;
-    none.ew = nullptr; none.W = 0; none.x0 = 0; none.y0 = 0;
-    push_one<R>(x2, y2, vxr, vyr, E, g, hk, (R)0, 0.0, ke, px, py, none);
-    ovx[q] = vxr;
-    ovy[q] = vyr;
+  const int np = st[run].np;
+  const long long q = blockIdx.x * (long long)PIC_WG + threadIdx.x;
+  if (q >= np) return;
+  const long long i = rd.pbase + q;
+  OutRec<R> o;
+  o.x = p.x[i]; o.y = p.y[i]; o.vx = p.vx[i]; o.vy = p.vy[i];
+  const int k = p.id[i];
+  if (KICK) {
+    typedef typename EWin<R>::R2 R2;
+    const Geo<R> g = make_geo<R>(rd.nx, rd.ny, rd.lx, rd.ly);
+    const R hk = (R)(0.5 * rd.dt * rd.qm);
+    const R2* E = reinterpret_cast<const R2*>(Eall) + rd.ebase;
+    const int ny1 = g.ny + 1;
+    int cx, cy;
+    R g00, g10, g01, g11, epx, epy;
+    gather_weights<R>(o.x, o.y, g, cx, cy, g00, g10, g01, g11);
+    const int i00 = cx * ny1 + cy;
+    interp<R>(g00, g10, g01, g11, E[i00], E[i00 + ny1], E[i00 + 1], E[i00 + ny1 + 1], epx, epy);
+    o.vx = fmar(hk, epx, o.vx);
+    o.vy = fmar(hk, epy, o.vy);
+  }
+  if (k < 0 || k >= np) return;
+  if (REC) {
+    rec[k] = o;
+  } else {
+    if (ox) ox[k] = o.x;
+    if (oy) oy[k] = o.y;
+    if (ovx) ovx[k] = o.vx;
+    if (ovy) ovy[k] = o.vy;
   }
 }
 
-// scatter slot q of run `run` to output index id[q] (id order)
 template <typename R>
-__global__ __launch_bounds__(PIC_WG) void k_unpermute(const RunDesc* __restrict__ runs,
-                                                      const RunState* __restrict__ st, int run,
-                                                      PartBufs<R> p, const R* __restrict__ vxs,
-                                                      const R* __restrict__ vys,
+__global__ __launch_bounds__(PIC_WG) void k_out_split(const OutRec<R>* __restrict__ rec, int n,
                                                       R* __restrict__ ox, R* __restrict__ oy,
-                                                      R* __restrict__ ovx, R* __restrict__ ovy,
-                                                      const int2* __restrict__ items) {
-  const int2 it = items[blockIdx.x];
-  if (it.x != run) return;
-  const RunDesc rd = runs[run];
-  const int np = st[run].np;
-  const int p1 = min(it.y + PIC_CHUNK, np);
-  for (int q = it.y + threadIdx.x; q < p1; q += PIC_WG) {
-    const long long i = rd.pbase + q;
-    const int k = p.id[i];
-    if (k < 0 || k >= np) continue;
-    ox[k] = p.x[i];
-    oy[k] = p.y[i];
-    ovx[k] = vxs ? vxs[q] : p.vx[i];
-    ovy[k] = vys ? vys[q] : p.vy[i];
-  }
+                                                      R* __restrict__ ovx,
+                                                      R* __restrict__ ovy) {
+  const long long k = blockIdx.x * (long long)PIC_WG + threadIdx.x;
+  if (k >= n) return;
+  const OutRec<R> o = rec[k];
+  if (ox) ox[k] = o.x;
+  if (oy) oy[k] = o.y;
+  if (ovx) ovx[k] = o.vx;
+  if (ovy) ovy[k] = o.vy;
 }
 
 template <typename R>
@@ -1116,18 +1083,33 @@ void launch_push(hipStream_t s, const PushArgs<R>& a) {
     k_push<R, 0, 0><<<a.nitems, PUSH_NT, a.lds_bytes, s>>>(a);
 }
 
+// n: the run's particle count (st[run].np).  rec given: records (and nothing else); else the
+// output arrays.
 template <typename R>
-void launch_half_kick_out(hipStream_t s, const RunDesc* runs, RunState* st, int run,
-                          PartBufs<R> p, const R* E, R* out_vx, R* out_vy, const int2* pitems,
-                          int npitems) {
-  k_half_kick_out<R><<<npitems, PIC_WG, 0, s>>>(runs, st, run, p, E, out_vx, out_vy, pitems);
+void launch_out_particles(hipStream_t s, const RunDesc* runs, RunState* st, int run, int n,
+                          PartBufs<R> p, const R* E, void* rec, R* ox, R* oy, R* ovx, R* ovy) {
+  if (n <= 0) return;
+  const int blocks = (int)(((long long)n + PIC_WG - 1) / PIC_WG);
+  OutRec<R>* r = (OutRec<R>*)rec;
+  if (r && E)
+    k_out_particles<R, true, true><<<blocks, PIC_WG, 0, s>>>(runs, st, run, p, E, r, ox, oy, ovx,
+                                                             ovy);
+  else if (r)
+    k_out_particles<R, false, true><<<blocks, PIC_WG, 0, s>>>(runs, st, run, p, E, r, ox, oy, ovx,
+                                                              ovy);
+  else if (E)
+    k_out_particles<R, true, false><<<blocks, PIC_WG, 0, s>>>(runs, st, run, p, E, r, ox, oy, ovx,
+                                                              ovy);
+  else
+    k_out_particles<R, false, false><<<blocks, PIC_WG, 0, s>>>(runs, st, run, p, E, r, ox, oy,
+                                                               ovx, ovy);
 }
 
 template <typename R>
-void launch_unpermute(hipStream_t s, const RunDesc* runs, RunState* st, int run, PartBufs<R> p,
-                      const R* vxs, const R* vys, R* ox, R* oy, R* ovx, R* ovy,
-                      const int2* pitems, int npitems) {
-  k_unpermute<R><<<npitems, PIC_WG, 0, s>>>(runs, st, run, p, vxs, vys, ox, oy, ovx, ovy, pitems);
+void launch_out_split(hipStream_t s, const void* rec, int n, R* ox, R* oy, R* ovx, R* ovy) {
+  if (n > 0)
+    k_out_split<R><<<(int)(((long long)n + PIC_WG - 1) / PIC_WG), PIC_WG, 0, s>>>(
+        (const OutRec<R>*)rec, n, ox, oy, ovx, ovy);
 }
 
 template <typename R>
@@ -1195,11 +1177,9 @@ void launch_op_gather_push(hipStream_t s, const GatherPushPlan& p, R* x, R* y, R
   template void launch_tile_sort<R>(hipStream_t, const RunDesc*, RunState*, int, PartBufs<R>,\
                                     PartBufs<R>, SortBufs, const int2*, int);                 \
   template void launch_push<R>(hipStream_t, const PushArgs<R>&);                            \
-  template void launch_half_kick_out<R>(hipStream_t, const RunDesc*, RunState*, int,        \
-                                        PartBufs<R>, const R*, R*, R*, const int2*, int);   \
-  template void launch_unpermute<R>(hipStream_t, const RunDesc*, RunState*, int,            \
-                                    PartBufs<R>, const R*, const R*, R*, R*, R*, R*,        \
-                                    const int2*, int);                                      \
+  template void launch_out_particles<R>(hipStream_t, const RunDesc*, RunState*, int, int,   \
+                                        PartBufs<R>, const R*, void*, R*, R*, R*, R*);      \
+  template void launch_out_split<R>(hipStream_t, const void*, int, R*, R*, R*, R*);         \
   template void launch_check_finite<R>(hipStream_t, const RunDesc*, RunState*, PartBufs<R>, \
                                        const int2*, int, int*);                             \
   template void launch_op_cell_keys<R>(hipStream_t, const R*, const R*, int64_t, int, int,  \

@@ -140,14 +140,14 @@ void launch_push(hipStream_t s, const PushArgs<R>& a);
 void launch_step_finish(hipStream_t s, const RunDesc* runs, RunState* st, int nruns,
                         const double* ppush, const double* prows, double* diag);
 
+// The n particles of a run in id order.  E: the run context's padded field, to add the pending
+// half kick, or NULL.  rec: n records {x, y, vx, vy} by id are written there, for
+// launch_out_split; NULL: the output arrays (those not NULL) are written.
 template <typename R>
-void launch_half_kick_out(hipStream_t s, const RunDesc* runs, RunState* st, int run,
-                          PartBufs<R> p, const R* E, R* out_vx, R* out_vy,
-                          const int2* pitems, int npitems);
+void launch_out_particles(hipStream_t s, const RunDesc* runs, RunState* st, int run, int n,
+                          PartBufs<R> p, const R* E, void* rec, R* ox, R* oy, R* ovx, R* ovy);
 template <typename R>
-void launch_unpermute(hipStream_t s, const RunDesc* runs, RunState* st, int run,
-                      PartBufs<R> p, const R* vxs, const R* vys, R* ox, R* oy, R* ovx, R* ovy,
-                      const int2* pitems, int npitems);
+void launch_out_split(hipStream_t s, const void* rec, int n, R* ox, R* oy, R* ovx, R* ovy);
 template <typename R>
 void launch_check_finite(hipStream_t s, const RunDesc* runs, RunState* st, PartBufs<R> p,
                          const int2* pitems, int npitems, int* flag);
