@@ -386,7 +386,7 @@ int pic_adjoint_create(const pic_config* cfg, const double* xl, const double* yl
     PIC_HIP(A.get(&A.ids, (size_t)A.nseg * n));
     PIC_HIP(A.get(&A.iota, n));
     PIC_HIP(A.get(&A.toffs, (size_t)A.nseg * (A.nb + 1)));
-    adj_iota(A.s, A.iota, n);
+    launch_iota(A.s, A.iota, n);
     PIC_HIP(hipStreamSynchronize(A.s));
   }
   PIC_HIP(hipMemcpy(A.dd, &d, sizeof(d), hipMemcpyHostToDevice));

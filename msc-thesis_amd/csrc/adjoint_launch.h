@@ -40,7 +40,6 @@ void adj_pass_win(hipStream_t s, const AdjGrid& g, const int4* items, const int*
                   double* lvx, double* lvy, double* lE);
 // four particle arrays (a: 4 x n) into the order before a sort: b[k][from[d]] = a[k][d]
 void adj_reorder(hipStream_t s, const int* from, const double* a, double* b, int64_t n);
-void adj_iota(hipStream_t s, int* id, int64_t n);
 template <typename R>
 void adj_seed(hipStream_t s, const AdjGrid& g, const R* E, double sc, double* lE);
 template <typename R>

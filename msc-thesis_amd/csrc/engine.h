@@ -25,6 +25,38 @@ hipError_t dalloc(T** p, size_t count) {
   return hipMalloc((void**)p, count * sizeof(T));
 }
 
+// Temporaries of one operator call (workspace.cpp): blocks kept from earlier calls or newly
+// allocated, returned when the object ends.  done(): the call's stream has been waited for.
+class Workspace {
+ public:
+  struct Block {
+    void* p;
+    size_t bytes;
+    int device;
+    bool host;
+  };
+  Workspace() = default;
+  Workspace(const Workspace&) = delete;
+  Workspace& operator=(const Workspace&) = delete;
+  ~Workspace();
+  template <typename T>
+  hipError_t get(T** p, size_t count) {
+    return raw((void**)p, count * sizeof(T), false);
+  }
+  template <typename T>
+  hipError_t pinned(T** p, size_t count) {  // pinned host memory
+    return raw((void**)p, count * sizeof(T), true);
+  }
+  void done() { finished = true; }
+
+ private:
+  hipError_t raw(void** p, size_t bytes, bool host);
+  std::vector<Block> blocks;
+  bool finished = false;
+};
+// frees the blocks kept for later calls on a device
+void workspace_trim(int device);
+
 int validate_config(const pic_config& c);
 double mcc_nu_max(const pic_config& c);
 

@@ -437,12 +437,6 @@ __global__ __launch_bounds__(PIC_WG) void k_adj_reorder(const int* __restrict__ 
   }
 }
 
-__global__ __launch_bounds__(PIC_WG) void k_adj_iota(int* __restrict__ id, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)PIC_WG + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * PIC_WG)
-    id[i] = (int)i;
-}
-
 // lE = s * E (unpadded FP64 two-component array from the padded field)
 template <typename R>
 __global__ __launch_bounds__(PIC_WG) void k_adj_seed(AdjGrid g, const R* __restrict__ Epad,
@@ -660,7 +654,6 @@ void adj_pass_win(hipStream_t s, const AdjGrid& g, const int4* items, const int*
 void adj_reorder(hipStream_t s, const int* from, const double* a, double* b, int64_t n) {
   k_adj_reorder<<<gridn(n), PIC_WG, 0, s>>>(from, a, b, n);
 }
-void adj_iota(hipStream_t s, int* id, int64_t n) { k_adj_iota<<<gridn(n), PIC_WG, 0, s>>>(id, n); }
 template <typename R>
 void adj_seed(hipStream_t s, const AdjGrid& g, const R* E, double sc, double* lE) {
   k_adj_seed<R><<<gridn((long long)g.nx * g.ny), PIC_WG, 0, s>>>(g, E, sc, lE);

@@ -695,6 +695,11 @@ __global__ void k_fill_i32(int* p, long long n, int v) {
        i += (long long)gridDim.x * PIC_WG)
     p[i] = v;
 }
+__global__ void k_iota(int* p, long long n) {
+  for (long long i = blockIdx.x * (long long)PIC_WG + threadIdx.x; i < n;
+       i += (long long)gridDim.x * PIC_WG)
+    p[i] = (int)i;
+}
 __global__ void k_fill_u64(unsigned long long* p, long long n) {
   for (long long i = blockIdx.x * (long long)PIC_WG + threadIdx.x; i < n;
        i += (long long)gridDim.x * PIC_WG)
@@ -986,6 +991,9 @@ inline int grid_for(long long n) {
 // ====================================================================== launchers
 void launch_fill_i32(hipStream_t s, int* p, long long n, int v) {
   if (n > 0) k_fill_i32<<<grid_for(n), PIC_WG, 0, s>>>(p, n, v);
+}
+void launch_iota(hipStream_t s, int* p, long long n) {
+  if (n > 0) k_iota<<<grid_for(n), PIC_WG, 0, s>>>(p, n);
 }
 void launch_fill_u64(hipStream_t s, unsigned long long* p, long long n) {
   if (n > 0) k_fill_u64<<<grid_for(n), PIC_WG, 0, s>>>(p, n);

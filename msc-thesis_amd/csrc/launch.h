@@ -173,6 +173,7 @@ void launch_op_fixed_to_double(hipStream_t s, const unsigned long long* hi,
                                const unsigned long long* lo, long long G, int fp64,
                                double scale, double* out);
 void launch_fill_i32(hipStream_t s, int* p, long long n, int v);
+void launch_iota(hipStream_t s, int* p, long long n);  // p[i] = i
 void launch_fill_u64(hipStream_t s, unsigned long long* p, long long n);
 void launch_reduce_sum(hipStream_t s, const double* parts, int n, double* out);
 

@@ -3,8 +3,8 @@
 // The reference keeps each stage as a file-static kernel configured through
 // __constant__ symbols (thesisCode/collisionless/double/src/pic.cu:13-26, 69-420); these
 // entry points expose the same stages with explicit arguments so each can be dropped into
-// another driver or tested alone.  Temporaries are allocated per call, except in
-// pic_op_deposit_noalloc (a static device array).
+// another driver or tested alone.  Temporaries come from blocks kept between calls
+// (workspace.cpp), except in pic_op_deposit_noalloc (a static device array).
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -17,19 +17,6 @@
 using namespace pic;
 
 namespace {
-
-struct DevMem {
-  std::vector<void*> ptrs;
-  ~DevMem() {
-    for (void* p : ptrs) (void)hipFree(p);
-  }
-  template <typename T>
-  hipError_t get(T** p, size_t count) {
-    hipError_t e = dalloc(p, count);
-    if (e == hipSuccess) ptrs.push_back((void*)*p);
-    return e;
-  }
-};
 
 int check_grid(const pic_grid* g) {
   if (!g) return fail(PIC_ERR_ARG, "NULL grid");
@@ -87,7 +74,7 @@ int pic_op_sort(const int32_t* keys, int64_t n, int ncells, int32_t* perm, int32
   hipStream_t s = (hipStream_t)stream;
   const RadixPlan p = radix_plan(n, ncells);
   const size_t nn = (size_t)std::max<int64_t>(n, 1), nd = (size_t)1 << p.bits;
-  DevMem m;
+  Workspace m;
   RadixBufs b;
   std::memset(&b, 0, sizeof(b));
   PIC_HIP(m.get(&b.flag, 1));
@@ -100,10 +87,12 @@ int pic_op_sort(const int32_t* keys, int64_t n, int ncells, int32_t* perm, int32
   launch_fill_i32(s, b.flag, 1, 0);
   launch_radix_sort(s, keys, (int)n, ncells, p, b, perm, counts, offsets);
   PIC_HIP(hipGetLastError());
-  int h = 0;
-  PIC_HIP(hipMemcpyAsync(&h, b.flag, sizeof(int), hipMemcpyDeviceToHost, s));
+  int* h;
+  PIC_HIP(m.pinned(&h, 1));
+  PIC_HIP(hipMemcpyAsync(h, b.flag, sizeof(int), hipMemcpyDeviceToHost, s));
   PIC_HIP(hipStreamSynchronize(s));
-  if (h) return fail(PIC_ERR_ARG, "key outside [0, ncells)");
+  m.done();
+  if (*h) return fail(PIC_ERR_ARG, "key outside [0, ncells)");
   return PIC_OK;
 }
 
@@ -117,7 +106,7 @@ int pic_op_deposit(const void* x, const void* y, int64_t n, int precision, const
   const long long G = (long long)g->nx * g->ny;
   const bool fp64 = precision == PIC_FP64;
   DepositPlan p = deposit_plan(n, g->nx, g->ny, fp64, true);
-  DevMem m;
+  Workspace m;
   unsigned long long *hi, *lo = nullptr;
   PIC_HIP(m.get(&hi, G));
   if (fp64) PIC_HIP(m.get(&lo, G));
@@ -151,6 +140,7 @@ int pic_op_deposit(const void* x, const void* y, int64_t n, int precision, const
   launch_op_fixed_to_double(s, hi, lo, G, precision == PIC_FP64, scale, rho);
   PIC_HIP(hipGetLastError());
   PIC_HIP(hipStreamSynchronize(s));
+  m.done();
   return PIC_OK;
 }
 
@@ -260,7 +250,7 @@ int pic_op_poisson(const double* rho, double* phi, const pic_grid* g, void* stre
   RunDesc d = op_desc(nx, ny, g->lx, g->ly, 0);
   const int nrp = nx / (2 * d.fft_pp), ncl = ny / 2 + 1;
   const size_t ss = (size_t)ncl * nx;
-  DevMem m;
+  Workspace m;
   double2* S;
   RunDesc* dd;
   RunState* st;
@@ -282,6 +272,7 @@ int pic_op_poisson(const double* rho, double* phi, const pic_grid* g, void* stre
   launch_field(s, a, nullptr);
   PIC_HIP(hipGetLastError());
   PIC_HIP(hipStreamSynchronize(s));
+  m.done();
   return PIC_OK;
 }
 
@@ -304,7 +295,7 @@ int pic_op_gather_push(void* x, void* y, void* vx, void* vy, int64_t n, int prec
   hipStream_t s = (hipStream_t)stream;
   const bool fp64 = precision == PIC_FP64;
   const GatherPushPlan p = gather_push_plan(n, g->nx, g->ny, fp64);
-  DevMem m;
+  Workspace m;
   double* parts = nullptr;
   if (ke) PIC_HIP(m.get(&parts, p.blocks));
   char* pairs = nullptr;
@@ -321,6 +312,7 @@ int pic_op_gather_push(void* x, void* y, void* vx, void* vy, int64_t n, int prec
   if (ke) launch_reduce_sum(s, parts, p.blocks, ke);
   PIC_HIP(hipGetLastError());
   PIC_HIP(hipStreamSynchronize(s));
+  m.done();
   return PIC_OK;
 }
 
@@ -334,7 +326,7 @@ int pic_op_mcc(float* x, float* y, float* vx, float* vy, int32_t* id, int64_t* n
   int rc = validate_config(c);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  DevMem m;
+  Workspace m;
   RunState* st;
   RunDesc* dd;
   int *bc, *bp, *cl, *cc, *cp;
@@ -385,6 +377,7 @@ int pic_op_mcc(float* x, float* y, float* vx, float* vy, int32_t* id, int64_t* n
   PIC_HIP(hipGetLastError());
   PIC_HIP(hipMemcpyAsync(&hs, st, sizeof(hs), hipMemcpyDeviceToHost, s));
   PIC_HIP(hipStreamSynchronize(s));
+  m.done();
   *n_io = hs.np;
   if (hs.err & 1) return fail(PIC_ERR_OVERFLOW, "births exceeded capacity");
   return PIC_OK;

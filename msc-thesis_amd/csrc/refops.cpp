@@ -18,21 +18,8 @@ using namespace pic;
 
 namespace {
 
-struct Scratch {
-  std::vector<void*> ptrs;
-  ~Scratch() {
-    for (void* p : ptrs) (void)hipFree(p);
-  }
-  template <typename T>
-  hipError_t get(T** p, size_t count) {
-    hipError_t e = dalloc(p, count);
-    if (e == hipSuccess) ptrs.push_back((void*)*p);
-    return e;
-  }
-};
-
 // consumer starts of m consumers on u[nu]; *used = uniforms they take
-int resolve_chain(hipStream_t s, Scratch& sc, const double* u, long long nu, double prob,
+int resolve_chain(hipStream_t s, Workspace& sc, const double* u, long long nu, double prob,
                   long long m, long long** start, long long* used) {
   const long long nchunks = (ref_chain_stream(nu, m) + REF_CHAIN_CHUNK - 1) / REF_CHAIN_CHUNK;
   RefChainBufs b;
@@ -44,12 +31,13 @@ int resolve_chain(hipStream_t s, Scratch& sc, const double* u, long long nu, dou
   PIC_HIP(sc.get(&b.consumed, 1));
   launch_ref_chain(s, u, nu, prob, m, b);
   PIC_HIP(hipGetLastError());
-  long long c = -1;
-  PIC_HIP(hipMemcpyAsync(&c, b.consumed, sizeof(c), hipMemcpyDeviceToHost, s));
+  long long* c;
+  PIC_HIP(sc.pinned(&c, 1));
+  PIC_HIP(hipMemcpyAsync(c, b.consumed, sizeof(*c), hipMemcpyDeviceToHost, s));
   PIC_HIP(hipStreamSynchronize(s));
-  if (c < 0) return fail(PIC_ERR_ARG, "uniform stream too short for the particles that draw");
+  if (*c < 0) return fail(PIC_ERR_ARG, "uniform stream too short for the particles that draw");
   *start = b.start;
-  *used = c;
+  *used = *c;
   return PIC_OK;
 }
 
@@ -64,7 +52,7 @@ int pic_op_mcc_reference(double* vx, double* vy, int64_t n, double prob, const d
   if (n < 0 || nu < 0 || !consumed || !finite_prob(prob)) return fail(PIC_ERR_ARG, "bad argument");
   if (n > 0 && (!vx || !vy || !u)) return fail(PIC_ERR_ARG, "NULL array");
   hipStream_t s = (hipStream_t)stream;
-  Scratch sc;
+  Workspace sc;
   long long* start = nullptr;
   long long used = 0;
   int rc = resolve_chain(s, sc, u, nu, prob, n, &start, &used);
@@ -72,6 +60,7 @@ int pic_op_mcc_reference(double* vx, double* vy, int64_t n, double prob, const d
   launch_mcc_reference(s, vx, vy, n, prob, u, start);
   PIC_HIP(hipGetLastError());
   PIC_HIP(hipStreamSynchronize(s));
+  sc.done();
   *consumed = used;
   return PIC_OK;
 }
@@ -89,7 +78,7 @@ int pic_op_dsmc_reference(const double* x, const double* y, double* vx, double* 
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   const int G = g->nx * g->ny;
-  Scratch sc;
+  Workspace sc;
   int *keys, *bad, *perm, *counts, *offsets, *target, *drawkey, *cons, *ccount, *coff;
   PIC_HIP(sc.get(&keys, std::max<int64_t>(n, 1)));
   PIC_HIP(sc.get(&bad, 1));
@@ -102,21 +91,23 @@ int pic_op_dsmc_reference(const double* x, const double* y, double* vx, double* 
   PIC_HIP(sc.get(&ccount, 2));
   PIC_HIP(sc.get(&coff, 3));
   // the reference's cells, (int)(x/dx) and (int)(y/dy), keyed cx*ny + cy
-  PIC_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
+  int* host;  // what the host reads back: bad; offsets of the drawing particles
+  unsigned long long* hn;
+  PIC_HIP(sc.pinned(&host, 2));
+  PIC_HIP(sc.pinned(&hn, 1));
+  launch_fill_i32(s, bad, 1, 0);
   launch_ref_cell_keys(s, x, y, n, g->nx, g->ny, g->lx / g->nx, g->ly / g->ny, keys, bad);
-  int hbad = 0;
-  PIC_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+  PIC_HIP(hipMemcpyAsync(host, bad, sizeof(int), hipMemcpyDeviceToHost, s));
   PIC_HIP(hipStreamSynchronize(s));
-  if (hbad) return fail(PIC_ERR_ARG, "particle outside [0, lx) x [0, ly)");
+  if (host[0]) return fail(PIC_ERR_ARG, "particle outside [0, lx) x [0, ly)");
   // cell lists in ascending particle index: the stable counting sort by cell
   if ((rc = pic_op_sort(keys, n, G, perm, counts, offsets, stream))) return rc;
   launch_ref_nearest(s, x, y, n, keys, perm, offsets, target, drawkey);
   // the particles that draw, in ascending index: stable sort by (draws ? 0 : 1)
   if ((rc = pic_op_sort(drawkey, n, 2, cons, ccount, coff, stream))) return rc;
-  int hoff[2] = {0, 0};
-  PIC_HIP(hipMemcpyAsync(hoff, coff, sizeof(hoff), hipMemcpyDeviceToHost, s));
+  PIC_HIP(hipMemcpyAsync(host, coff, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
   PIC_HIP(hipStreamSynchronize(s));
-  const long long m = hoff[1];
+  const long long m = host[1];
   long long* start = nullptr;
   long long used = 0;
   if ((rc = resolve_chain(s, sc, u, nu, prob, m, &start, &used))) return rc;
@@ -130,14 +121,14 @@ int pic_op_dsmc_reference(const double* x, const double* y, double* vx, double* 
   PIC_HIP(sc.get(&nc, 1));
   launch_fill_i32(s, self, n, -1);
   launch_fill_i32(s, lastw, n, -1);
-  PIC_HIP(hipMemsetAsync(nc, 0, sizeof(unsigned long long), s));
+  launch_fill_u64(s, nc, 1);
   launch_dsmc_reference(s, vx, vy, n, m, prob, u, start, cons, target, m1, m2, self, lastw, nc);
   PIC_HIP(hipGetLastError());
-  unsigned long long hn = 0;
-  PIC_HIP(hipMemcpyAsync(&hn, nc, sizeof(hn), hipMemcpyDeviceToHost, s));
+  PIC_HIP(hipMemcpyAsync(hn, nc, sizeof(*hn), hipMemcpyDeviceToHost, s));
   PIC_HIP(hipStreamSynchronize(s));
+  sc.done();
   *consumed = used;
-  if (ncoll) *ncoll = (int64_t)hn;
+  if (ncoll) *ncoll = (int64_t)*hn;
   return PIC_OK;
 }
 
