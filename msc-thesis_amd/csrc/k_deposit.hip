@@ -5,7 +5,7 @@
 // whatever the number of addresses, which bounded a deposit of four (FP64: eight) of them
 // per particle: 1.36 ms for 8,000,009 FP32 particles on 512^2.  The sums are integers, so the
 // particles can go in any order, and three forms give the same bits (8,000,009 FP32 particles
-// in random order on 512^2: 15.7 + 4.7 + 35.8 + 22.8 us in the last; whole call 1431 -> 152):
+// in random order on 512^2: 15.7 + 4.7 + 35.8 + 22.8 us in the last; whole call 1427 -> 89):
 //   direct   four global atomics per particle
 //   grid     each workgroup sums its share in an LDS copy of the whole grid, then adds the
 //            copy's non-zero words to the global one
@@ -300,12 +300,12 @@ inline int grid_for(long long n, int nt, int most) {
 }  // namespace
 
 // Lines measured as whole calls on one card, FP32 / FP64 where they differ (us):
-//   grid, 64^2, 65,536 positions: 24 / 28, direct 30 / 44; below 8 positions per node clearing
-//   and adding the copy costs what it saves (128^2 FP32: 39 against 31 at 65,536, 39 against 42
+//   grid, 64^2, 65,536 positions: 23 / 29, direct 30 / 43; below 8 positions per node clearing
+//   and adding the copy costs what it saves (128^2 FP32: 37 against 30 at 65,536, 37 against 41
 //   at 131,072)
-//   binned, 512^2: 93 / 98 against 97 / 168 direct at 262,144 positions, 99 against 123 (FP64)
-//   at 131,072; on larger grids the tiles' windows cost more (2048^2 FP32: 166 against 158 at
-//   524,288, 191 against 249 at 1,048,576)
+//   binned, 512^2: 36 / 41 against 41 / 66 direct at 131,072 positions, 39 / 43 against 30 / 44
+//   at 65,536; on larger grids the tiles' windows cost more (2048^2: 68 / 97 against 77 / 134 at
+//   262,144, 70 / 91 against 54 / 89 at 131,072)
 DepositPlan deposit_plan(int64_t n, int nx, int ny, int fp64, bool scratch) {
   DepositPlan p;
   const long long G = (long long)nx * ny, words = fp64 ? 2 : 1;
@@ -316,7 +316,7 @@ DepositPlan deposit_plan(int64_t n, int nx, int ny, int fp64, bool scratch) {
     if (n >= 8 * G) p.form = DEPOSIT_GRID;
     return p;
   }
-  if (!scratch || n * words < std::max(262144ll, G / 4) || n > 0x7fff0000) return p;
+  if (!scratch || n * words < std::max(131072ll, G / 16) || n > 0x7fff0000) return p;
   int lnx = 0, lny = 0;
   while ((1 << lnx) < nx) ++lnx;
   while ((1 << lny) < ny) ++lny;

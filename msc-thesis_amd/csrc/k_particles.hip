@@ -1133,28 +1133,31 @@ void launch_op_cell_keys(hipStream_t s, const R* x, const R* y, int64_t n, int n
 }
 
 // LDS: grids whose padded pairs leave two workgroups per CU.  Packed: enough particles to pay
-// for packing (an allocation, a launch, and 24 or 32 bytes per node).  Whole calls, random
-// order, node arrays -> new form, FP32 / FP64 (us):
-//   LDS, 64^2: 8,000,009 particles 145 / 155 -> 59 / 100, 1,048,576: 36 / 39 -> 29 / 33,
-//   524,288: 27 / 28 -> 27 / 31
-//   packed, 512^2: 8,000,009 particles 316 / 319 -> 171 / 238 (the kernel 269 -> 97 + 5 to
-//   pack, FP32), 4,194,304: 157 / 166 -> 92 / 145, 1,048,576: 56 / 60 -> 61 / 78
+// for packing (a launch, and 24 or 32 bytes per node).  Whole calls, random order, node arrays
+// -> new form, FP32 / FP64 (us):
+//   LDS, 64^2: 8,000,009 particles 145 / 155 -> 59 / 97, 1,048,576: 36 / 39 -> 25 / 28
+//   (32^2: 20 / 22 -> 20 / 21 at 262,144)
+//   packed, 512^2: 8,000,009 particles 281 / 319 -> 112 / 217 (with random velocities 316 ->
+//   148; the kernel 269 -> 97 + 5 to pack, FP32), 1,048,576: 56 / 60 -> 35 / 48, 524,288:
+//   36 / 38 -> 30 / 36, 262,144: 26 -> 27; 1024^2 at 524,288: 51 / 53 -> 40 / 47
 GatherPushPlan gather_push_plan(int64_t n, int nx, int ny, int fp64) {
   GatherPushPlan p;
   const long long G = (long long)nx * ny, pad = (long long)(nx + 1) * (ny + 1);
   const long long bytes = pad * (fp64 ? 16 : 8);
   p.pairs = 0;
   p.lds = 0;
-  if (bytes <= 72 * 1024 && n >= (1 << 20)) {
+  if (bytes <= 72 * 1024 && n >= std::max(262144ll, 256 * G)) {
     p.lds = (int)bytes;
-    const long long per = std::max<long long>(2 * GP_LDS_NT, 2 * G);
+    // four particles per thread, and at least as many as the fill has nodes
+    const long long per = std::max<long long>(4 * GP_LDS_NT, G);
     const long long b = (n + per - 1) / per;
     p.blocks = (int)(b > 512 ? 512 : b);
     return p;
   }
-  const long long b = (n + PIC_WG - 1) / PIC_WG;
+  if (n >= 524288 && n >= G / 8) p.pairs = pad;
+  const long long per = p.pairs ? 4 * PIC_WG : PIC_WG;
+  const long long b = (n + per - 1) / per;
   p.blocks = (int)(b < 1 ? 1 : (b > 4096 ? 4096 : b));
-  if (n >= (3 << 19) && n >= G && bytes < (64 << 20)) p.pairs = pad;
   return p;
 }
 
