@@ -150,11 +150,11 @@ Ctx::~Ctx() {
   F(d_runs); F(d_st);
   for (int i = 0; i < 2; ++i) { F(px[i]); F(pid[i]); }
   F(rho); F(rho_lo); F(E); F(S); F(Sx); F(Sy); F(phi); F(tw);
-  F(sb.keys); F(sb.rank); F(sb.perm); F(sb.counts); F(sb.offsets); F(sb.chunk_sums);
+  F(sb.keys); F(sb.rank); F(sb.rec); F(sb.counts); F(sb.offsets); F(sb.chunk_sums);
   F(sb.big_list); F(sb.big_count); F(sb.scratch); F(sb.table); F(sb.tchunk_sums);
   F(toffs[0]); F(toffs[1]); F(sb.ftable); F(sb.fchunk_sums); F(d_fscan_items);
   F(d_pitems); F(d_citems); F(d_rowpair); F(d_cols); F(d_rows); F(d_push);
-  F(d_segitems); F(d_tscan_items);
+  F(d_tscan_items);
   F(partials_push); F(partials_rows); F(diag);
   F(d_coll_counts); F(birth_count); F(birth_parent); F(birth_buf); F(gmax); F(flag);
   F(coll_list); F(coll_count); F(coll_partials);
@@ -178,7 +178,7 @@ int Ctx::upload_runs() {
 
 int Ctx::build_items() {
   pitems.clear(); citems.clear(); rowpair.clear(); cols.clear(); rows.clear(); push_items.clear();
-  segitems.clear(); tscan_items.clear(); rp_begin.clear(); col_begin.clear();
+  tscan_items.clear(); rp_begin.clear(); col_begin.clear();
   lds_push = 0;
   long long tsum = 0;
   toffsum = 0;
@@ -213,7 +213,6 @@ int Ctx::build_items() {
     d.cell_item_begin = (int)citems.size();
     for (int c = 0; c < d.nx * d.ny; c += PIC_CELL_CHUNK) citems.push_back(make_int2(r, c));
     d.cell_item_end = (int)citems.size();
-    for (int c = 0; c < d.nx * d.ny; c += PIC_SEG_CELLS) segitems.push_back(make_int2(r, c));
     push_items_for(r, nullptr);
     d.fchunks = 0;
     fft_groups(rows_total, d.nx, d.ny, &d.fft_pp, &d.fft_rf);
@@ -274,7 +273,6 @@ int Ctx::build_items() {
   if ((rc = up(cols, &d_cols))) return rc;
   if ((rc = up(rows, &d_rows))) return rc;
   if ((rc = up(push_items, &d_push))) return rc;
-  if ((rc = up(segitems, &d_segitems))) return rc;
   if ((rc = up(tscan_items, &d_tscan_items))) return rc;
   if ((rc = up(fscan_items, &d_fscan_items))) return rc;
   sb.fscan_items = d_fscan_items;
@@ -283,8 +281,6 @@ int Ctx::build_items() {
   PIC_HIP(dalloc(&sb.ftable, fused ? fsum : 1));
   if (sb.fchunk_sums) (void)hipFree(sb.fchunk_sums);
   PIC_HIP(dalloc(&sb.fchunk_sums, std::max<size_t>(1, fscan_items.size() * (size_t)maxb)));
-  sb.segitems = d_segitems;
-  sb.nsegitems = (int)segitems.size();
   sb.tscan_items = d_tscan_items;
   sb.ntscan_items = (int)tscan_items.size();
   sb.max_buckets = maxb;
@@ -338,7 +334,8 @@ int Ctx::alloc() {
   {
     long long maxcap = 0;
     for (auto& c : cfg) maxcap = std::max<long long>(maxcap, c.capacity);
-    const double need = (double)ptotal * (8.0 * rsize + 8 + 28) +
+    const double need = (double)ptotal * (8.0 * rsize + 8 + (any_dsmc ? 16 : 0) +
+                                          (any_mcc || any_dsmc ? 16 : 0)) +
                         (any_mcc ? 24.0 * maxcap : 0.0) + (double)gsum * (fp64 ? 40 : 24) +
                         (double)esum * 2 * rsize + 48.0 * ssum + 12.0 * ctotal;
     size_t free_b = 0, total_b = 0;
@@ -372,16 +369,18 @@ int Ctx::alloc() {
   PIC_HIP(dalloc(&Sy, ssum));
   PIC_HIP(dalloc(&phi, gsum));
   PIC_HIP(dalloc(&tw, PIC_FFT_MAX / 2));
-  PIC_HIP(dalloc(&sb.keys, ptotal));
-  PIC_HIP(dalloc(&sb.rank, ptotal));
-  PIC_HIP(dalloc(&sb.perm, ptotal));
+  if (any_dsmc) {
+    PIC_HIP(dalloc(&sb.keys, ptotal));
+    PIC_HIP(dalloc(&sb.rank, ptotal));
+    PIC_HIP(dalloc(&sb.rec, ptotal));
+  }
   PIC_HIP(dalloc(&sb.counts, ctotal));
   // the cell sorts keep the counts zero between sorts (their scan clears what it read)
   PIC_HIP(hipMemset(sb.counts, 0, sizeof(int) * (size_t)ctotal));
   PIC_HIP(dalloc(&sb.offsets, ctotal));
   PIC_HIP(dalloc(&sb.big_list, 2 * ctotal));
   PIC_HIP(dalloc(&sb.big_count, 1));
-  PIC_HIP(dalloc(&sb.scratch, 2 * ptotal));
+  if (any_mcc || any_dsmc) PIC_HIP(dalloc(&sb.scratch, 2 * ptotal));
   PIC_HIP(dalloc(&diag, (size_t)nruns * PIC_DIAG_CAP * 8));
   PIC_HIP(dalloc(&d_coll_counts, 4 * nruns));
   PIC_HIP(dalloc(&flag, 1));
@@ -492,13 +491,10 @@ int Ctx::launch_sort_stage() {
     cur ^= 1;
     return PIC_OK;
   }
-  // DSMC needs per-cell lists: full cell sort with tile-major cell numbering
-  if (fp64)
-    launch_sort<double>(stream, d_runs, d_st, nruns, bufs<double>(cur), bufs<double>(1 - cur), sb,
-                        d_pitems, (int)pitems.size(), d_citems, (int)citems.size(), ctotal, true);
-  else
-    launch_sort<float>(stream, d_runs, d_st, nruns, bufs<float>(cur), bufs<float>(1 - cur), sb,
-                       d_pitems, (int)pitems.size(), d_citems, (int)citems.size(), ctotal, true);
+  // DSMC needs per-cell lists: full cell sort with tile-major cell numbering (contexts with
+  // collisions hold FP32 particles)
+  launch_cell_sort(stream, d_runs, d_st, bufs<float>(cur), bufs<float>(1 - cur), sb, d_pitems,
+                   (int)pitems.size(), d_citems, (int)citems.size());
   cur ^= 1;
   return PIC_OK;
 }

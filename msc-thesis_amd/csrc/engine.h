@@ -108,12 +108,11 @@ struct Ctx {
   int* collide_count_table = nullptr;  // the count table while a count step's collision
                                        // stage runs (its births are counted; else NULL)
   bool fused = false;                  // sort fused into the push (see build_items)
-  std::vector<int2> pitems, citems, rowpair, cols, rows, segitems, tscan_items, fscan_items;
+  std::vector<int2> pitems, citems, rowpair, cols, rows, tscan_items, fscan_items;
   std::vector<int> rp_begin, col_begin;  // first row-pair and column item of each run
   std::vector<int4> push_items;
   int2 *d_pitems = nullptr, *d_citems = nullptr, *d_rowpair = nullptr, *d_cols = nullptr,
-       *d_rows = nullptr, *d_segitems = nullptr, *d_tscan_items = nullptr,
-       *d_fscan_items = nullptr;
+       *d_rows = nullptr, *d_tscan_items = nullptr, *d_fscan_items = nullptr;
   int4* d_push = nullptr;
   double* partials_push = nullptr;
   double* partials_rows = nullptr;

@@ -1,12 +1,10 @@
-// k_particles.hip -- particle-side kernels: cell sort, fused gather+push+deposit, outputs.
+// k_particles.hip -- particle-side kernels: tile sort, fused gather+push+deposit, outputs.
 //
 // Reference stages replaced (thesisCode/collisionless/double/src/pic.cu):
 //   currentCell        :69-87    -> cell key computed inside the sort and the push
 //   chargeAssignment   :99-138   -> deterministic fixed-point CIC deposit in LDS windows
 //   forceCalculation   :298-355  -> bilinear gather fused into the push
 //   positionUpdate     :372-420  -> leapfrog push, periodic wrap into [0, L)
-//   cellTrackerSetup   thesisCode/dsmcCollisions/cellTrackerAdvanced/src/pic.cu:419-445
-//                                -> stable counting sort by key cx*ny+cy (ties by id)
 #include <algorithm>
 #include <climits>
 #include <type_traits>
@@ -15,402 +13,6 @@
 #include "step_tail.h"
 
 namespace {
-
-// ========================================================================== sort
-#define HWIN 8192  // LDS histogram window (keys) of the rank kernel
-
-// Cell numbering of the engine's own sorts: tile-major (tile t = (cx/T)*tiles_y + cy/T,
-// then cx%T, cy%T), so that every tile and every cell is one contiguous range.  The
-// operator pic_op_sort sorts whatever keys it is given (k_radix.hip).
-// Tile sizes are powers of two and cells are clamped to >= 0: shifts and masks.
-__device__ __forceinline__ int engine_cell_key(int cx, int cy, const RunDesc& rd) {
-  const int sh = __builtin_ctz((unsigned)rd.tile), m = rd.tile - 1;
-  const int t = (cx >> sh) * rd.tiles_y + (cy >> sh);
-  return (((t << sh) + (cx & m)) << sh) + (cy & m);
-}
-
-template <typename R>
-__global__ __launch_bounds__(PIC_WG) void k_sort_rank(const RunDesc* __restrict__ runs,
-                                                      const RunState* __restrict__ st,
-                                                      const R* __restrict__ x,
-                                                      const R* __restrict__ y,
-                                                      int* __restrict__ keys,
-                                                      int* __restrict__ rank,
-                                                      int* __restrict__ counts,
-                                                      const int2* __restrict__ items) {
-  __shared__ int hist[HWIN];
-  __shared__ int red[8];
-  // slice blockIdx % PIC_SORT_SLICES of chunk item blockIdx / PIC_SORT_SLICES
-  const int2 it = items[blockIdx.x / PIC_SORT_SLICES];
-  const RunDesc rd = runs[it.x];
-  const int np = st[it.x].np;
-  const int p0 = it.y + (blockIdx.x % PIC_SORT_SLICES) * (PIC_CHUNK / PIC_SORT_SLICES);
-  const int p1 = min(p0 + PIC_CHUNK / PIC_SORT_SLICES, np);
-  if (p0 >= p1) return;  // uniform across the workgroup
-  const long long pb = rd.pbase;
-  const int nx = rd.nx, ny = rd.ny;
-  const R dxr = (R)rd.dx, dyr = (R)rd.dy;
-  int* cnt = counts + rd.cbase;
-  // a slice is RANK_U particles per thread: their loads go out together (lanes past p1 load
-  // particle p1 - 1, no branches) and their keys stay in registers for the later passes
-  constexpr int RANK_U = (PIC_CHUNK / PIC_SORT_SLICES) / PIC_WG;
-  static_assert(RANK_U * PIC_WG == PIC_CHUNK / PIC_SORT_SLICES, "slice = whole rounds");
-  int key[RANK_U];
-  bool act[RANK_U];
-  int kmin = INT_MAX, kmax = INT_MIN;
-  R xv[RANK_U], yv[RANK_U];
-#pragma unroll
-  for (int u = 0; u < RANK_U; ++u) {
-    const int p = p0 + threadIdx.x + u * PIC_WG;
-    act[u] = p < p1;
-    const int pl = act[u] ? p : p1 - 1;
-    xv[u] = x[pb + pl];
-    yv[u] = y[pb + pl];
-  }
-#pragma unroll
-  for (int u = 0; u < RANK_U; ++u) {
-    int cx, cy;
-    R f;
-    locate(xv[u], dxr, nx, cx, f);
-    locate(yv[u], dyr, ny, cy, f);
-    key[u] = engine_cell_key(cx, cy, rd);
-    if (act[u]) keys[pb + p0 + threadIdx.x + u * PIC_WG] = key[u];
-  }
-#pragma unroll
-  for (int u = 0; u < RANK_U; ++u)
-    if (act[u]) {
-      kmin = min(kmin, key[u]);
-      kmax = max(kmax, key[u]);
-    }
-  kmin = wave_min_i(kmin);
-  kmax = wave_max_i(kmax);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0) { red[w] = kmin; red[4 + w] = kmax; }
-  __syncthreads();
-  kmin = min(min(red[0], red[1]), min(red[2], red[3]));
-  kmax = max(max(red[4], red[5]), max(red[6], red[7]));
-  const long long span = (long long)kmax - kmin + 1;
-  if (span <= HWIN) {
-    for (int k = threadIdx.x; k < span; k += PIC_WG) hist[k] = 0;
-    __syncthreads();
-    int rk[RANK_U];
-#pragma unroll
-    for (int u = 0; u < RANK_U; ++u)
-      if (act[u]) rk[u] = atomicAdd(&hist[key[u] - kmin], 1);
-    __syncthreads();
-    for (int k = threadIdx.x; k < span; k += PIC_WG) {
-      int c = hist[k];
-      if (c) hist[k] = atomicAdd(&cnt[kmin + k], c);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < RANK_U; ++u)
-      if (act[u]) rank[pb + p0 + threadIdx.x + u * PIC_WG] = rk[u] + hist[key[u] - kmin];
-  } else {
-#pragma unroll
-    for (int u = 0; u < RANK_U; ++u)
-      if (act[u]) rank[pb + p0 + threadIdx.x + u * PIC_WG] = atomicAdd(&cnt[key[u]], 1);
-  }
-}
-
-// exclusive scan of the counts of one chunk of PIC_CELL_CHUNK cells; the counts are zeroed
-// once read (they are zero between sorts, so no fill launch precedes the rank kernel)
-__global__ __launch_bounds__(PIC_WG) void k_scan_local(const RunDesc* __restrict__ runs,
-                                                       int* __restrict__ counts,
-                                                       int* __restrict__ offsets,
-                                                       int* __restrict__ chunk_sums,
-                                                       const int2* __restrict__ items) {
-  __shared__ int wsum[4];
-  const int2 it = items[blockIdx.x];
-  const RunDesc rd = runs[it.x];
-  const int G = rd.nx * rd.ny;
-  const int c0 = it.y + threadIdx.x * 8;
-  int v[8], s = 0;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    int c = c0 + k;
-    v[k] = (c < G) ? counts[rd.cbase + c] : 0;
-    s += v[k];
-  }
-#pragma unroll
-  for (int k = 0; k < 8; ++k)
-    if (c0 + k < G) counts[rd.cbase + c0 + k] = 0;
-  // inclusive wave scan of per-thread totals
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int inc = s;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    int t = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += t;
-  }
-  if (lane == 63) wsum[w] = inc;
-  __syncthreads();
-  int wpre = 0;
-  for (int k = 0; k < w; ++k) wpre += wsum[k];
-  int ex = wpre + inc - s;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    int c = c0 + k;
-    if (c < G) offsets[rd.cbase + c] = ex;
-    ex += v[k];
-  }
-  if (threadIdx.x == PIC_WG - 1) chunk_sums[blockIdx.x] = wpre + inc;
-}
-
-// The chunk's base added to its offsets: the base is the sum of the run's chunk totals
-// before it (integer adds, so any order gives the same base), added up by the workgroup
-// itself, which saves a launch that scanned the chunk totals.  Also the tile offsets toff[t] =
-// offsets[t T^2] (the cell numbering is tile-major: tile t owns cells [t T^2, (t + 1) T^2)).  The run's last chunk writes the total: offsets[G], nsorted and the
-// closing tile offset; the first workgroup clears the count of cells too large for the
-// within-cell sort's small kernel (which appends to it next).
-__global__ __launch_bounds__(PIC_WG) void k_scan_add(const RunDesc* __restrict__ runs,
-                                                     RunState* __restrict__ st,
-                                                     int* __restrict__ offsets,
-                                                     const int* __restrict__ chunk_sums,
-                                                     const int2* __restrict__ items,
-                                                     int* __restrict__ toff,
-                                                     int* __restrict__ big_count) {
-  __shared__ int wsum[PIC_WG / 64];
-  const int2 it = items[blockIdx.x];
-  const RunDesc rd = runs[it.x];
-  const int G = rd.nx * rd.ny;
-  const int TT = rd.tile * rd.tile;
-  int part = 0;
-  for (int i = rd.cell_item_begin + (int)threadIdx.x; i < (int)blockIdx.x; i += PIC_WG)
-    part += chunk_sums[i];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
-  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = part;
-  __syncthreads();
-  int add = 0;
-#pragma unroll
-  for (int w = 0; w < PIC_WG / 64; ++w) add += wsum[w];
-  for (int k = threadIdx.x; k < PIC_CELL_CHUNK; k += PIC_WG) {
-    int c = it.y + k;
-    if (c < G) {
-      const int o = offsets[rd.cbase + c] + add;
-      offsets[rd.cbase + c] = o;
-      if (c % TT == 0) toff[rd.toffbase + c / TT] = o;
-    }
-  }
-  if (threadIdx.x == 0) {
-    if ((int)blockIdx.x == rd.cell_item_end - 1) {
-      const int total = add + chunk_sums[blockIdx.x];
-      offsets[rd.cbase + G] = total;
-      st[it.x].nsorted = total;
-      toff[rd.toffbase + rd.nbuckets] = total;
-    }
-    if (blockIdx.x == 0) *big_count = 0;
-  }
-}
-
-__global__ __launch_bounds__(PIC_WG) void k_sort_scatter(const RunDesc* __restrict__ runs,
-                                                         const RunState* __restrict__ st,
-                                                         const int* __restrict__ keys,
-                                                         const int* __restrict__ rank,
-                                                         const int* __restrict__ offsets,
-                                                         int* __restrict__ perm,
-                                                         const int2* __restrict__ items) {
-  const int2 it = items[blockIdx.x / PIC_SORT_SLICES];
-  const RunDesc rd = runs[it.x];
-  const int np = st[it.x].np;
-  const int p0 = it.y + (blockIdx.x % PIC_SORT_SLICES) * (PIC_CHUNK / PIC_SORT_SLICES);
-  const int p1 = min(p0 + PIC_CHUNK / PIC_SORT_SLICES, np);
-  for (int p = p0 + threadIdx.x; p < p1; p += PIC_WG) {
-    int d = offsets[rd.cbase + keys[rd.pbase + p]] + rank[rd.pbase + p];
-    perm[rd.pbase + d] = p;
-  }
-}
-
-__device__ __forceinline__ unsigned long long shfl_xor_u64(unsigned long long v, int m) {
-  unsigned lo = (unsigned)v, hi = (unsigned)(v >> 32);
-  lo = __shfl_xor(lo, m, 64);
-  hi = __shfl_xor(hi, m, 64);
-  return ((unsigned long long)hi << 32) | lo;
-}
-
-__device__ __forceinline__ unsigned long long seg_key(const int* id, long long pb, int slot) {
-  return ((unsigned long long)(unsigned)id[pb + slot] << 32) | (unsigned)slot;
-}
-
-// Canonical order inside each cell: ascending id.  One wavefront per cell: <= 64 entries by a bitonic
-// network across lanes, <= 256 entries by counting ranks (4 entries per lane, keys are
-// unique); larger cells are queued for k_segsort_big.  Items cover PIC_SEG_CELLS cells
-// (one per wave).
-// 65-256 entries of one cell, sorted by one wave: a bitonic network over 64 * NR keys held
-// NR per lane (key e at lane e % 64 of register e / 64; padding ~0 sorts last).  Distances of
-// 64 and more pair registers of one lane, shorter ones lanes of one register.  (Ranking each
-// key by counting the smaller ones took n steps per wave.)
-template <int NR>
-__device__ __forceinline__ void bitonic_regs(const int* __restrict__ id, int* __restrict__ perm,
-                                             long long pb, int b, int n, int lane) {
-  unsigned long long k4[NR];
-#pragma unroll
-  for (int k = 0; k < NR; ++k) {
-    const int j = lane + 64 * k;
-    k4[k] = (j < n) ? seg_key(id, pb, perm[pb + b + j]) : ~0ull;
-  }
-#pragma unroll
-  for (int size = 2; size <= 64 * NR; size <<= 1) {
-#pragma unroll
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      if (stride >= 64) {
-        const int sr = stride >> 6;
-#pragma unroll
-        for (int k = 0; k < NR; ++k) {
-          if (k & sr) continue;  // k is the lower element of the pair (k, k | sr)
-          const bool up = ((64 * k) & size) == 0;
-          const unsigned long long a0 = k4[k], a1 = k4[k | sr];
-          const unsigned long long mn = a0 < a1 ? a0 : a1, mx = a0 < a1 ? a1 : a0;
-          k4[k] = up ? mn : mx;
-          k4[k | sr] = up ? mx : mn;
-        }
-      } else {
-        const bool lower = (lane & stride) == 0;
-#pragma unroll
-        for (int k = 0; k < NR; ++k) {
-          const unsigned long long o = shfl_xor_u64(k4[k], stride);
-          const bool up = ((lane + 64 * k) & size) == 0;
-          const unsigned long long mn = k4[k] < o ? k4[k] : o, mx = k4[k] < o ? o : k4[k];
-          k4[k] = (lower == up) ? mn : mx;
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < NR; ++k)
-    if (lane + 64 * k < n) perm[pb + b + lane + 64 * k] = (int)(unsigned)(k4[k] & 0xffffffffull);
-}
-
-__global__ __launch_bounds__(PIC_WG) void k_segsort_small(const RunDesc* __restrict__ runs,
-                                                          const int* __restrict__ offsets,
-                                                          int* __restrict__ perm,
-                                                          const int* __restrict__ id,
-                                                          int* __restrict__ big_list,
-                                                          int* __restrict__ big_count,
-                                                          const int2* __restrict__ items) {
-  const int2 it = items[blockIdx.x];
-  const RunDesc rd = runs[it.x];
-  const int G = rd.nx * rd.ny;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int cend = min(it.y + PIC_SEG_CELLS, G);
-  const long long pb = rd.pbase;
-  for (int c = it.y + w; c < cend; c += 4) {
-    const int b = offsets[rd.cbase + c], e = offsets[rd.cbase + c + 1];
-    const int n = e - b;
-    if (n <= 1) continue;
-    if (n > 256) {
-      if (lane == 0) {
-        int slot = atomicAdd(big_count, 1);
-        big_list[2 * slot] = it.x;
-        big_list[2 * slot + 1] = c;
-      }
-      continue;
-    }
-    if (n > 128) {
-      bitonic_regs<4>(id, perm, pb, b, n, lane);
-      continue;
-    }
-    if (n > 64) {
-      bitonic_regs<2>(id, perm, pb, b, n, lane);
-      continue;
-    }
-    unsigned long long v = (lane < n) ? seg_key(id, pb, perm[pb + b + lane]) : ~0ull;
-    // the network over the first m = 2^ceil(log2 n) lanes only (the others hold padding)
-    const int m = 1 << (32 - __clz(n - 1));
-    for (int k = 2; k <= m; k <<= 1) {
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        unsigned long long o = shfl_xor_u64(v, j);
-        bool up = (lane & k) == 0;
-        bool lower = (lane & j) == 0;
-        unsigned long long mn = v < o ? v : o, mx = v < o ? o : v;
-        v = (lower == up) ? mn : mx;
-      }
-    }
-    if (lane < n) perm[pb + b + lane] = (int)(unsigned)(v & 0xffffffffull);
-  }
-}
-
-// Large cells: bitonic sort by one workgroup, in LDS up to 4096 entries, else in a
-// global scratch region [2*(pbase+b), 2*(pbase+b) + m) with m = next pow2 >= n (<= 2n).
-__global__ __launch_bounds__(PIC_WG) void k_segsort_big(const RunDesc* __restrict__ runs,
-                                                        const int* __restrict__ offsets,
-                                                        int* __restrict__ perm,
-                                                        const int* __restrict__ id,
-                                                        const int* __restrict__ big_list,
-                                                        const int* __restrict__ big_count,
-                                                        unsigned long long* __restrict__ scratch) {
-  __shared__ unsigned long long s[4096];
-  const int nbig = *big_count;
-  for (int q = blockIdx.x; q < nbig; q += gridDim.x) {
-    const int run = big_list[2 * q], c = big_list[2 * q + 1];
-    const RunDesc rd = runs[run];
-    const long long pb = rd.pbase;
-    const int b = offsets[rd.cbase + c], e = offsets[rd.cbase + c + 1];
-    const int n = e - b;
-    int m = 1;
-    while (m < n) m <<= 1;
-    unsigned long long* a = (m <= 4096) ? s : scratch + 2 * (pb + b);
-    for (int i = threadIdx.x; i < m; i += PIC_WG)
-      a[i] = (i < n) ? seg_key(id, pb, perm[pb + b + i]) : ~0ull;
-    __syncthreads();
-    for (int k = 2; k <= m; k <<= 1) {
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        for (int i = threadIdx.x; i < m; i += PIC_WG) {
-          int l = i ^ j;
-          if (l > i) {
-            unsigned long long u = a[i], v = a[l];
-            bool up = (i & k) == 0;
-            if ((u > v) == up) { a[i] = v; a[l] = u; }
-          }
-        }
-        __syncthreads();
-      }
-    }
-    for (int i = threadIdx.x; i < n; i += PIC_WG)
-      perm[pb + b + i] = (int)(unsigned)(a[i] & 0xffffffffull);
-    __syncthreads();
-  }
-}
-
-template <typename R>
-__global__ __launch_bounds__(PIC_WG) void k_sort_apply(const RunDesc* __restrict__ runs,
-                                                       const RunState* __restrict__ st,
-                                                       const int* __restrict__ perm,
-                                                       PartBufs<R> src, PartBufs<R> dst,
-                                                       const int2* __restrict__ items) {
-  const int2 it = items[blockIdx.x / PIC_SORT_SLICES];
-  const RunDesc rd = runs[it.x];
-  const int np = st[it.x].np;
-  const int d0 = it.y + (blockIdx.x % PIC_SORT_SLICES) * (PIC_CHUNK / PIC_SORT_SLICES);
-  const int p1 = min(d0 + PIC_CHUNK / PIC_SORT_SLICES, np);
-  const long long pb = rd.pbase;
-  // APPLY_U slots per thread per round, every load of a round issued before any store (one
-  // slot per thread and round waited for its permutation entry, then for its five reads);
-  // lanes past p1 read slot p1 - 1 (loads without branches) and store nothing
-  constexpr int APPLY_U = 4;
-  for (int d = d0 + threadIdx.x; d < p1; d += APPLY_U * PIC_WG) {
-    int sl[APPLY_U];
-#pragma unroll
-    for (int u = 0; u < APPLY_U; ++u) sl[u] = perm[pb + min(d + u * PIC_WG, p1 - 1)];
-    R x[APPLY_U], y[APPLY_U], vx[APPLY_U], vy[APPLY_U];
-    int idv[APPLY_U];
-#pragma unroll
-    for (int u = 0; u < APPLY_U; ++u) {
-      const long long s = pb + sl[u];
-      x[u] = src.x[s]; y[u] = src.y[s]; vx[u] = src.vx[s]; vy[u] = src.vy[s];
-      idv[u] = src.id[s];
-    }
-#pragma unroll
-    for (int u = 0; u < APPLY_U; ++u) {
-      const int dd = d + u * PIC_WG;
-      if (dd < p1) {
-        dst.x[pb + dd] = x[u]; dst.y[pb + dd] = y[u]; dst.vx[pb + dd] = vx[u];
-        dst.vy[pb + dd] = vy[u]; dst.id[pb + dd] = idv[u];
-      }
-    }
-  }
-}
 
 // ------------------------------------------------------------ tile sort of the step
 // Stable counting sort of the particles by tile (sort bucket):
@@ -1007,38 +609,6 @@ void launch_reduce_sum(hipStream_t s, const double* parts, int n, double* out) {
   k_reduce_sum<<<1, PIC_WG, 0, s>>>(parts, n, out);
 }
 
-static void sort_tail(hipStream_t s, const RunDesc* runs, RunState* st, const int* id,
-                      SortBufs sb, const int2* citems, int ncitems) {
-  k_segsort_small<<<sb.nsegitems, PIC_WG, 0, s>>>(runs, sb.offsets, sb.perm, id, sb.big_list,
-                                                  sb.big_count, sb.segitems);
-  k_segsort_big<<<256, PIC_WG, 0, s>>>(runs, sb.offsets, sb.perm, id, sb.big_list, sb.big_count,
-                                       sb.scratch);
-}
-
-static void sort_scan(hipStream_t s, const RunDesc* runs, RunState* st, int nruns, SortBufs sb,
-                      const int2* citems, int ncitems) {
-  k_scan_local<<<ncitems, PIC_WG, 0, s>>>(runs, sb.counts, sb.offsets, sb.chunk_sums, citems);
-  k_scan_add<<<ncitems, PIC_WG, 0, s>>>(runs, st, sb.offsets, sb.chunk_sums, citems, sb.toff,
-                                        sb.big_count);
-}
-
-template <typename R>
-void launch_sort(hipStream_t s, const RunDesc* runs, RunState* st, int nruns, PartBufs<R> src,
-                 PartBufs<R> dst, SortBufs sb, const int2* pitems, int npitems,
-                 const int2* citems, int ncitems, long long ctotal, bool move_data) {
-  // sb.counts is zero here: zeroed at allocation and by the scan of every sort since
-  (void)ctotal;
-  k_sort_rank<R><<<npitems * PIC_SORT_SLICES, PIC_WG, 0, s>>>(runs, st, src.x, src.y, sb.keys,
-                                                             sb.rank, sb.counts, pitems);
-  sort_scan(s, runs, st, nruns, sb, citems, ncitems);
-  k_sort_scatter<<<npitems * PIC_SORT_SLICES, PIC_WG, 0, s>>>(runs, st, sb.keys, sb.rank,
-                                                              sb.offsets, sb.perm, pitems);
-  sort_tail(s, runs, st, src.id, sb, citems, ncitems);
-  if (move_data)
-    k_sort_apply<R><<<npitems * PIC_SORT_SLICES, PIC_WG, 0, s>>>(runs, st, sb.perm, src, dst,
-                                                                 pitems);
-}
-
 template <typename R>
 void launch_tile_sort(hipStream_t s, const RunDesc* runs, RunState* st, int nruns,
                       PartBufs<R> src, PartBufs<R> dst, SortBufs sb, const int2* pitems,
@@ -1182,9 +752,6 @@ void launch_op_gather_push(hipStream_t s, const GatherPushPlan& p, R* x, R* y, R
 }
 
 #define PIC_INST(R)                                                                          \
-  template void launch_sort<R>(hipStream_t, const RunDesc*, RunState*, int, PartBufs<R>,    \
-                               PartBufs<R>, SortBufs, const int2*, int, const int2*, int,   \
-                               long long, bool);                                            \
   template void launch_tile_sort<R>(hipStream_t, const RunDesc*, RunState*, int, PartBufs<R>,\
                                     PartBufs<R>, SortBufs, const int2*, int);                 \
   template void launch_push<R>(hipStream_t, const PushArgs<R>&);                            \

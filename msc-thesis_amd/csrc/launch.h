@@ -9,25 +9,18 @@
 //   tile items   int4 {run, tx, ty, split}; tx < 0 marks a tail chunk (start in .z)
 //   row items    int2 {run, row}
 #define PIC_CELL_CHUNK 2048
-// cell sort: cells per item of the within-cell sort (one wave per cell, four waves per
-// workgroup), and the slices of a particle chunk item that the rank, scatter and apply
-// kernels give one workgroup each (more workgroups than chunks: the blob-like runs of the
-// collision stages need the latency hiding)
-#define PIC_SEG_CELLS 4
-#define PIC_SORT_SLICES 4
 
 struct SortBufs {
+  // cell sort (runs with DSMC)
   int* keys;        // [ptotal]
   int* rank;        // [ptotal]
-  int* perm;        // [ptotal]  run-local source index of sorted slot
+  unsigned long long* rec;      // [ptotal] (id << 32 | run-local source slot) by cell
   int* counts;      // [ctotal]
   int* offsets;     // [ctotal]
   int* chunk_sums;  // [n cell chunk items]
-  int* big_list;    // [ptotal] cells needing the workgroup segment sort (run, cell) pairs
+  int* big_list;    // [2*ctotal] cells that one workgroup sorts, (run, cell) pairs
   int* big_count;   // [1]
-  unsigned long long* scratch;  // [2*ptotal] power-of-two padded segments
-  const int2* segitems;         // {run, first cell} items of 64 cells (segment sort)
-  int nsegitems;
+  unsigned long long* scratch;  // [2*ptotal] power-of-two padded segments (also MCC births)
   // tile sort of the step
   int* table;                   // [sum nbuckets*nchunks] bucket-major count table
   int* tchunk_sums;             // [n table-scan items]
@@ -48,12 +41,13 @@ struct PartBufs {
   int* id;
 };
 
+// ---- cell sort (k_cellsort.hip): src in cell order, ascending id inside a cell, to dst; writes
+// sb.offsets, sb.toff and RunState::nsorted
+void launch_cell_sort(hipStream_t s, const RunDesc* runs, RunState* st, PartBufs<float> src,
+                      PartBufs<float> dst, SortBufs sb, const int2* pitems, int npitems,
+                      const int2* citems, int ncitems);
+
 // ---- particle kernels (k_particles.hip)
-template <typename R>
-void launch_sort(hipStream_t s, const RunDesc* runs, RunState* st, int nruns,
-                 PartBufs<R> src, PartBufs<R> dst, SortBufs sb,
-                 const int2* pitems, int npitems, const int2* citems, int ncitems,
-                 long long ctotal, bool move_data);
 // stable tile (bucket) sort of the step; writes sb.toff and RunState::nsorted
 // scan of the fused sort's count table and the new tile offsets (toff_new, nsorted)
 void launch_fused_scan(hipStream_t s, const RunDesc* runs, RunState* st, int nruns,
