@@ -76,21 +76,78 @@ double mcc_nu_max(const pic_config& c) {
   return best * 1.0001;  // margin so that no particle's total rate exceeds nu_max
 }
 
-static Tuning default_tuning(const pic_config& c, int tile, int halo, int splits) {
+// Steps a particle of unit speed takes to cross a cell, at most (thermal speeds and beams are
+// about 1 in the engine's units).
+static double cells_per_step(const pic_config& c) {
+  return c.dt / std::min(c.lx / c.nx, c.ly / c.ny);
+}
+
+// Sort cadence when none is asked for: every 8 steps was the fastest or within 3 % of it on
+// grids of 32^2 to 512^2, FP32 and FP64, up to 4 cells of drift per step (512^2, 4.2 M FP32
+// particles at 2: 61 us per step against 64 at every 4); beyond that half of a cycle's drift
+// outgrows the halo.
+static int default_cadence(const std::vector<pic_config>& cfg) {
+  for (const pic_config& c : cfg)
+    if (cells_per_step(c) > 4.0) return 4;
+  return 8;
+}
+
+// Tiling of a run whose share of the launch is `items` workgroups; nonzero values are kept.
+//   tile    the largest up to 32 that leaves half as many tiles as items (at most 128), 8 at
+//           least: a push workgroup pays for its windows, but a 64^2 grid in 16 tiles of 16^2 leaves most
+//           CUs idle (two-stream, 64^2, 409,600 FP64 particles: 46 us per step in 16 x 4
+//           workgroups, 26 in 64 x 4).  64 on FP32 grids that 32 leaves in more than 512 tiles
+//           (1024^2, 16 M particles: 375 us per step with 16, 259 with 32, 217 with 64)
+//   halo    16 where half a cycle's drift of 2.5 thermal speeds passes 8 cells, else 8
+//   splits  as many as make up the items, of 256 particles at least and 65,536 at most
+static Tuning default_tuning(const pic_config& c, int tile, int halo, int splits, int cadence,
+                             double items) {
   Tuning t;
   const int m = std::min(c.nx, c.ny);
-  t.tile = std::min(tile ? tile : 16, m / 2);
+  const long long n = std::max<long long>(c.capacity, 1);
+  if (tile) {
+    t.tile = std::min(tile, m / 2);
+  } else {
+    t.tile = std::min(32, m / 2);
+    while (t.tile > 8 && 2.0 * (c.nx / t.tile) * (c.ny / t.tile) < std::min(items, 256.0))
+      t.tile /= 2;
+    // above 512 tiles the sort leaves the push: FP32 windows of 64 cells still fit
+    if (c.precision == PIC_FP32 && (c.nx / t.tile) * (c.ny / t.tile) > 512 && m >= 128)
+      t.tile = 64;
+  }
   // at most 4096 tiles (the sort keeps one counter per tile in LDS)
   while ((c.nx / t.tile) * (c.ny / t.tile) > 4096 && t.tile < m / 2) t.tile *= 2;
   // the window (tile + 2 halo + 1 nodes) must not wrap onto itself: win <= min(nx, ny)
   const int hmax = std::max(0, (m - t.tile - 1) / 2);
-  t.halo = std::min(halo ? halo : 16, hmax);
+  if (!halo) halo = 2.5 * cells_per_step(c) * (0.5 * cadence + 1.0) > 8.0 ? 16 : 8;
+  t.halo = std::min(halo, hmax);
   const int ntiles = (c.nx / t.tile) * (c.ny / t.tile);
-  // about 8192 particles per 512-thread workgroup (1 to 64 workgroups per tile)
-  const long long per_tile = std::max<long long>(c.capacity, 1) / ntiles;
-  t.splits = splits ? splits : (int)std::max(1LL, std::min(64LL, (per_tile + 8191) / 8192));
+  const long long per_tile = n / ntiles;
+  if (splits) {
+    t.splits = splits;
+  } else {
+    long long s = (long long)(items / ntiles + 0.5);
+    s = std::min(s, per_tile / 256);
+    s = std::max(s, (per_tile + 65535) / 65536);
+    t.splits = (int)std::max(1LL, std::min(64LL, s));
+  }
   t.per_tile = splits == 0 && c.collide == PIC_COLLIDE_DSMC;
   return t;
+}
+
+// Tunings of all runs (values of 0: from_config takes the run's configured ones, then the
+// defaults).  A launch wants one workgroup per CU, two where two fit (FP32) and get 2048
+// particles each; a run of a batch has its share of them by particles.
+void Ctx::tune_runs(int tile, int halo, int splits, bool from_config) {
+  double total = 0;
+  for (const pic_config& c : cfg) total += (double)std::max<int64_t>(c.capacity, 1);
+  const double items = !fp64 && total >= 512.0 * 2048.0 ? 512.0 : 256.0;
+  tune.resize(nruns);
+  for (int r = 0; r < nruns; ++r)
+    tune[r] = default_tuning(cfg[r], from_config ? cfg[r].tile : tile,
+                             from_config ? cfg[r].halo : halo,
+                             from_config ? cfg[r].splits : splits, any_dsmc ? 1 : sort_every,
+                             items * std::max<int64_t>(cfg[r].capacity, 1) / total);
 }
 
 // Items (run, tile x, tile y, split | splits << 16) of run r: t.splits per tile, or with
@@ -411,9 +468,7 @@ int Ctx::alloc() {
   PIC_HIP(hipMemset(diag, 0, sizeof(double) * (size_t)nruns * PIC_DIAG_CAP * 8));
   PIC_HIP(hipMemset(d_coll_counts, 0, sizeof(long long) * 4 * nruns));
   PIC_HIP(hipMemset(E, 0, rs * 2 * esum));
-  tune.resize(nruns);
-  for (int r = 0; r < nruns; ++r)
-    tune[r] = default_tuning(cfg[r], cfg[r].tile, cfg[r].halo, cfg[r].splits);
+  tune_runs(0, 0, 0, true);
   int rc = build_items();
   if (rc) return rc;
   allocated = true;
@@ -744,7 +799,7 @@ static int create_impl(const pic_config* cfgs, int nruns, pic_ctx** out) {
   x.has_particles.assign(nruns, 0);
   int se = 0;
   for (auto& cc : x.cfg) se = std::max(se, cc.sort_every);
-  x.sort_every = se ? se : 4;
+  x.sort_every = se ? se : default_cadence(x.cfg);
   if (nruns > 1 || cfgs[0].capacity > 0) {
     int rc = x.alloc();
     if (rc) return rc;
@@ -1135,8 +1190,8 @@ int pic_set_tuning(pic_ctx* ctx, int tile, int halo, int splits, int sort_every)
       return fail(PIC_ERR_ARG, "tile must be a power of two <= min(nx, ny)/2 and <= 64");
   }
   PIC_HIP(hipStreamSynchronize(x.stream));
-  for (int r = 0; r < x.nruns; ++r) x.tune[r] = default_tuning(x.cfg[r], tile, halo, splits);
   if (sort_every) x.sort_every = sort_every;
+  x.tune_runs(tile, halo, splits, false);
   int rc = x.build_items();
   if (rc) return rc;
   // offsets must describe the current order for the new tiling: sort now
@@ -1228,8 +1283,8 @@ int pic_autotune(pic_ctx* ctx, int trial_steps, double* best_ms) {
           continue;
         rc = restore();
         if (rc) break;
-        for (int r = 0; r < x.nruns; ++r) x.tune[r] = default_tuning(x.cfg[r], ti, h, sp);
         x.sort_every = se;
+        x.tune_runs(ti, h, sp, false);
         if ((rc = x.build_items())) break;
         x.launch_sort_stage();
         x.steps_since_sort = 0;

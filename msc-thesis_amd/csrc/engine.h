@@ -137,6 +137,7 @@ struct Ctx {
 
   ~Ctx();
   int alloc();
+  void tune_runs(int tile, int halo, int splits, bool from_config);
   int build_items();
   void push_items_for(int r, const int* toff_h);
   int rebalance_push_items();
