@@ -27,14 +27,14 @@ __device__ __forceinline__ int fft_slot(int i) {
 // elements i0 + m h (h = 2^(s-1)) that those stages combine, applies the same butterflies
 // with the same twiddles in the same order as stage-by-stage radix-2 (so the result is
 // bit-identical to it), and stores them back.
-template <int K, int PAD>
+template <int K, int PAD, int NT>
 __device__ __forceinline__ void fft_lds_pass(double2* a, int rows, int n, int logn, int s,
                                              double ws, const double2* __restrict__ tw,
                                              int logtw) {
   const int h = 1 << (s - 1);
   const int gmask = (n >> K) - 1;
   const int total = rows * (n >> K);
-  for (int b = threadIdx.x; b < total; b += PIC_WG) {
+  for (int b = threadIdx.x; b < total; b += NT) {
     const int r = b >> (logn - K), g = b & gmask;
     const int j = g & (h - 1);
     const int e0 = r * n + ((g >> (s - 1)) << (s - 1 + K)) + j;
@@ -63,32 +63,33 @@ __device__ __forceinline__ void fft_lds_pass(double2* a, int rows, int n, int lo
 // global table (logtw = PIC_FFT_LOG) or a copy of the n-point twiddles in LDS
 // (fft_stage_twiddles, logtw = logn).  Radix-2 butterflies, three stages per pass in
 // registers (one barrier per pass), the groups of all rows spread over the workgroup.  All
-// threads of the workgroup (PIC_WG) must call it.  PAD: the buffer's layout (fft_slot).
-template <int PAD = 0>
+// threads of the workgroup (NT) must call it.  PAD: the buffer's layout (fft_slot).
+template <int PAD = 0, int NT = PIC_WG>
 __device__ __forceinline__ void fft_lds_rows(double2* a, int rows, int n, int logn, int sign,
                                              const double2* __restrict__ tw,
                                              int logtw = PIC_FFT_LOG) {
   const double ws = (sign < 0) ? 1.0 : -1.0;
   int s = 1;
   for (; s + 2 <= logn; s += 3) {
-    fft_lds_pass<3, PAD>(a, rows, n, logn, s, ws, tw, logtw);
+    fft_lds_pass<3, PAD, NT>(a, rows, n, logn, s, ws, tw, logtw);
     __syncthreads();
   }
   if (s + 1 == logn) {
-    fft_lds_pass<2, PAD>(a, rows, n, logn, s, ws, tw, logtw);
+    fft_lds_pass<2, PAD, NT>(a, rows, n, logn, s, ws, tw, logtw);
     __syncthreads();
   } else if (s == logn) {
-    fft_lds_pass<1, PAD>(a, rows, n, logn, s, ws, tw, logtw);
+    fft_lds_pass<1, PAD, NT>(a, rows, n, logn, s, ws, tw, logtw);
     __syncthreads();
   }
 }
 
 // the n/2 twiddles of an n-point transform, from the global table into LDS (twl[j] =
 // exp(-2 pi i j / n)); the caller synchronises before the transform
+template <int NT = PIC_WG>
 __device__ __forceinline__ void fft_stage_twiddles(double2* twl, int n,
                                                    const double2* __restrict__ tw) {
   const int st = PIC_FFT_MAX / n;
-  for (int j = threadIdx.x; j < n / 2; j += PIC_WG) twl[j] = tw[j * st];
+  for (int j = threadIdx.x; j < n / 2; j += NT) twl[j] = tw[j * st];
 }
 
 // one row

@@ -260,6 +260,84 @@ __global__ __launch_bounds__(PIC_WG) void k_fft_field(FieldArgs a) {
   if (threadIdx.x == 0) a.partials[item] = s;
 }
 
+// ---- phi of a small grid by one workgroup, the data in LDS throughout: one launch where the
+// passes are four (the call: 27 -> 18 us at 32^2, 28 -> 25 at 64^2, the largest; the same for
+// a step's E takes longer than the three passes above 32^2, as one CU's LDS holds it up).
+// Buffers (rows padded when PAD): A, the forward rows, then the inverse columns; X, the forward
+// columns, then the inverse rows, two real rows packed as one complex row at either end.  Per
+// value the arithmetic is that of the passes.
+#define PHI_ONE_NT 512
+template <int PAD>
+__global__ __launch_bounds__(PHI_ONE_NT) void k_phi_one(RunDesc rd,
+                                                        const double* __restrict__ rho,
+                                                        double* __restrict__ phi,
+                                                        const double2* __restrict__ tw) {
+  extern __shared__ double2 lds[];
+  constexpr int NT = PHI_ONE_NT;
+  const int nx = rd.nx, ny = rd.ny, lognx = rd.lognx, logny = rd.logny;
+  const int nc = ny / 2 + 1, nr = nx / 2;
+  const int half = max(nc * fft_slot<PAD>(nx), nr * fft_slot<PAD>(ny));
+  double2* A = lds;
+  double2* X = lds + half;
+  double2* twx = X + half;
+  double2* twy = twx + nx / 2;
+  fft_stage_twiddles<NT>(twx, nx, tw);
+  fft_stage_twiddles<NT>(twy, ny, tw);
+#pragma unroll 4
+  for (int t = threadIdx.x; t < nr * ny; t += NT) {
+    const int q = t >> logny, j = t & (ny - 1);
+    A[fft_slot<PAD>(q * ny + bitrev(j, logny))] =
+        make_double2(rho[2 * q * ny + j], rho[(2 * q + 1) * ny + j]);
+  }
+  __syncthreads();
+  fft_lds_rows<PAD, NT>(A, nr, ny, logny, -1, twy, logny);
+  for (int t = threadIdx.x; t < nc * nx; t += NT) {
+    const int i = t & (nx - 1), k = t >> lognx, q = i >> 1;
+    const double2 zk = A[fft_slot<PAD>(q * ny + k)];
+    const double2 zm = A[fft_slot<PAD>(q * ny + ((ny - k) & (ny - 1)))];
+    X[fft_slot<PAD>(k * nx + bitrev(i, lognx))] =
+        (i & 1) ? make_double2(0.5 * (zk.y + zm.y), -0.5 * (zk.x - zm.x))
+                : make_double2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
+  }
+  __syncthreads();
+  fft_lds_rows<PAD, NT>(X, nc, nx, lognx, -1, twx, lognx);
+  const double twopi = 6.283185307179586476925;
+  for (int t = threadIdx.x; t < nc * nx; t += NT) {
+    const int m = t & (nx - 1), k = t >> lognx;
+    const int kk = (2 * k < ny) ? k : k - ny, mm = (2 * m < nx) ? m : m - nx;
+    const double ky = twopi * kk / rd.ly, kx = twopi * mm / rd.lx;
+    const double k2 = kx * kx + ky * ky;
+    const double2 r = X[fft_slot<PAD>(k * nx + m)];
+    double2 ph = make_double2(0.0, 0.0);
+    if (m != 0 || k != 0) ph = make_double2(r.x / k2, r.y / k2);
+    A[fft_slot<PAD>(k * nx + bitrev(m, lognx))] = ph;
+  }
+  __syncthreads();
+  fft_lds_rows<PAD, NT>(A, nc, nx, lognx, +1, twx, lognx);
+  for (int t = threadIdx.x; t < nr * ny; t += NT) {
+    const int q = t & (nr - 1), k = t >> (lognx - 1);
+    const int ks = (2 * k <= ny) ? k : ny - k;
+    double2 u = A[fft_slot<PAD>(ks * nx + 2 * q)], v = A[fft_slot<PAD>(ks * nx + 2 * q + 1)];
+    if (2 * k > ny) {
+      u.y = -u.y;
+      v.y = -v.y;
+    } else if (k == 0 || 2 * k == ny) {
+      u.y = 0.0;
+      v.y = 0.0;
+    }
+    X[fft_slot<PAD>(q * ny + bitrev(k, logny))] = make_double2(u.x - v.y, u.y + v.x);
+  }
+  __syncthreads();
+  fft_lds_rows<PAD, NT>(X, nr, ny, logny, +1, twy, logny);
+  const double norm = 1.0 / ((double)nx * ny);
+  for (int t = threadIdx.x; t < nr * ny; t += NT) {
+    const int q = t >> logny, j = t & (ny - 1);
+    const double2 z = X[fft_slot<PAD>(q * ny + j)];
+    phi[2 * q * ny + j] = z.x * norm;
+    phi[(2 * q + 1) * ny + j] = z.y * norm;
+  }
+}
+
 __global__ __launch_bounds__(PIC_WG) void k_op_efield(const double* __restrict__ phi,
                                                       double* __restrict__ ex,
                                                       double* __restrict__ ey, int nx, int ny,
@@ -352,6 +430,19 @@ void launch_field(hipStream_t s, const FieldArgs& a, hipEvent_t* ev) {
     k_fft_field<float, 0><<<a.n_row_items + xfield, PIC_WG, lrow, s>>>(a);
   if (a.want_phi && a.phi) k_fft_field<float, 1><<<a.n_row_pair_items, PIC_WG, lrow, s>>>(a);
   if (ev) (void)hipEventRecord(ev[3], s);
+}
+
+bool launch_phi_one(hipStream_t s, const RunDesc& d, const double* rho, double* phi,
+                    const double2* tw) {
+  if ((long long)d.nx * d.ny > 4096) return false;
+  const bool pad = d.nx >= 8 && d.ny >= 8;
+  auto slot = [&](int n) { return pad ? n + n / 8 : n; };
+  const int half = std::max((d.ny / 2 + 1) * slot(d.nx), d.nx / 2 * slot(d.ny));
+  const size_t lds = sizeof(double2) * (2 * half + d.nx / 2 + d.ny / 2);
+  if (lds > 150 * 1024) return false;
+  if (pad) k_phi_one<1><<<1, PHI_ONE_NT, lds, s>>>(d, rho, phi, tw);
+  else k_phi_one<0><<<1, PHI_ONE_NT, lds, s>>>(d, rho, phi, tw);
+  return true;
 }
 
 void launch_op_setup(hipStream_t s, const RunDesc& d, RunDesc* dd, RunState* st, int2* rp,

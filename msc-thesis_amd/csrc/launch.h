@@ -248,6 +248,9 @@ void launch_field(hipStream_t s, const FieldArgs& a, hipEvent_t* ev /* 4 events 
 // one-grid descriptor, state and items into device memory (all of them read by launch_field)
 void launch_op_setup(hipStream_t s, const RunDesc& d, RunDesc* dd, RunState* st, int2* rp,
                      int nrp, int2* cl, int ncl);
+// phi of a small grid in one launch; false (and nothing launched) when the grid is too large
+bool launch_phi_one(hipStream_t s, const RunDesc& d, const double* rho, double* phi,
+                    const double2* tw);
 void launch_op_efield(hipStream_t s, const double* phi, double* ex, double* ey, int nx, int ny,
                       double lx, double ly);
 // copy padded E (float/double pairs) of one run out to two FP64 node arrays
