@@ -424,20 +424,24 @@ __global__ __launch_bounds__(PIC_WG) void k_op_cell_keys(const R* __restrict__ x
   }
 }
 
-// ---- gather + push of a caller's particles, in place and in any order.  Three sources of the
+// ---- gather + push of a caller's particles, in place and in any order.  Four sources of the
 // field give the same values (each is the node's FP64 field rounded to R):
 //   GP_NODES   the caller's two node arrays: eight 8-byte loads per particle
 //   GP_PACKED  (Ex, Ey) pairs on the padded (nx + 1) x (ny + 1) nodes, made by k_op_pack_E:
 //              a cell's two node rows are two contiguous pieces of two pairs
-//   GP_LDS     the same padded pairs of a small grid, in every workgroup's LDS
+//   GP_ROWS    the pairs with the two node rows of a cell interleaved, entry (i, j) = nodes
+//              (i, j), (i + 1, j): all four corners are one contiguous piece, for twice the
+//              memory.  The state is written past the caches, which then hold the pairs
+//   GP_LDS     the padded pairs of a small grid, in every workgroup's LDS
 // Random positions are bound by the vector L1: 64 lanes of a load meet up to 64 lines, so the
 // number of load instructions sets the time (launch_op_gather_push has the measurements).
-enum { GP_NODES, GP_PACKED, GP_LDS };
+enum { GP_NODES, GP_PACKED, GP_ROWS, GP_LDS };
 
+// rows: the interleaved form, nx rows of 2 * (ny + 1) entries
 template <typename R>
 __global__ __launch_bounds__(PIC_WG) void k_op_pack_E(const double* __restrict__ ex,
                                                       const double* __restrict__ ey, int nx,
-                                                      int ny,
+                                                      int ny, int rows,
                                                       typename EWin<R>::R2* __restrict__ E) {
   const int lny = __builtin_ctz((unsigned)ny);
   const int G = nx * ny;
@@ -446,6 +450,14 @@ __global__ __launch_bounds__(PIC_WG) void k_op_pack_E(const double* __restrict__
     typename EWin<R>::R2 v;
     v.x = (R)ex[q];
     v.y = (R)ey[q];
+    if (rows) {
+      // node (i, j): the first of entry (i, j), the second of entry (i - 1, j)
+      const long long a = 2ll * i * (ny + 1), b = 2ll * ((i ? i : nx) - 1) * (ny + 1) + 1;
+      E[a + 2 * j] = v;
+      E[b + 2 * j] = v;
+      if (j == 0) E[a + 2 * ny] = E[b + 2 * ny] = v;
+      continue;
+    }
     typename EWin<R>::R2* row = E + (long long)i * (ny + 1);
     row[j] = v;
     if (j == 0) row[ny] = v;
@@ -519,6 +531,10 @@ __global__ __launch_bounds__(SRC == GP_LDS ? GP_LDS_NT : PIC_WG) void k_op_gathe
       } else if (SRC == GP_LDS) {
         const int i0 = cx * ny1 + cy;
         e00[u] = el[i0]; e01[u] = el[i0 + 1]; e10[u] = el[i0 + ny1]; e11[u] = el[i0 + ny1 + 1];
+      } else if (SRC == GP_ROWS) {
+        R2 r[4];
+        __builtin_memcpy(r, E + 2 * ((long long)cx * ny1 + cy), sizeof(r));
+        e00[u] = r[0]; e10[u] = r[1]; e01[u] = r[2]; e11[u] = r[3];
       } else {
         // two neighbouring pairs as one piece (16 B in FP32, aligned to 8)
         R2 r0[2], r1[2];
@@ -544,10 +560,19 @@ __global__ __launch_bounds__(SRC == GP_LDS ? GP_LDS_NT : PIC_WG) void k_op_gathe
       const double vsy = (double)vyr[u] + skc * (double)epy;
       ke += vsx * vsx + vsy * vsy;
       const R wx = fmar(hk, epx, vxr[u]), wy = fmar(hk, epy, vyr[u]);
-      x[p] = wrap_pos(fmar(dtr, wx, xr[u]), g.Lx);
-      y[p] = wrap_pos(fmar(dtr, wy, yr[u]), g.Ly);
-      vx[p] = wx;
-      vy[p] = wy;
+      const R wxp = wrap_pos(fmar(dtr, wx, xr[u]), g.Lx);
+      const R wyp = wrap_pos(fmar(dtr, wy, yr[u]), g.Ly);
+      if (SRC == GP_ROWS) {
+        __builtin_nontemporal_store(wxp, x + p);
+        __builtin_nontemporal_store(wyp, y + p);
+        __builtin_nontemporal_store(wx, vx + p);
+        __builtin_nontemporal_store(wy, vy + p);
+      } else {
+        x[p] = wxp;
+        y[p] = wyp;
+        vx[p] = wx;
+        vy[p] = wy;
+      }
     }
   }
   if (!partials) return;  // uniform
@@ -710,11 +735,25 @@ void launch_op_cell_keys(hipStream_t s, const R* x, const R* y, int64_t n, int n
 //   packed, 512^2: 8,000,009 particles 281 / 319 -> 112 / 217 (with random velocities 316 ->
 //   148; the kernel 269 -> 97 + 5 to pack, FP32), 1,048,576: 56 / 60 -> 35 / 48, 524,288:
 //   36 / 38 -> 30 / 36, 262,144: 26 -> 27; 1024^2 at 524,288: 51 / 53 -> 40 / 47
+// Interleaved rows instead of packed: where they take little of an XCD's 4 MiB L2, where the
+// packed pairs do not fit it either, or where the state is a large part of the last-level
+// cache, whose lines then come from HBM anyway; enough particles to pay for packing twice the
+// memory.  Packed -> rows, the state in the last-level cache / in HBM at the start (us):
+//   FP32  128^2: 8,000,009 particles 98 / 155 -> 89 / 135, 1,048,576: 33 / 38 -> 30 / 36
+//         512^2: 20,000,003 334 / 376 -> 273 / 301, 8,000,009 114 / 166 -> 126 / 137,
+//         but 4,194,304 74 / 95 -> 82 / 88, 1,048,576 36 / 41 -> 41 / 41
+//         1024^2: 8,000,009 235 / 238 -> 195 / 199, 1,048,576 54 / 57 -> 52 / 57
+//         2048^2: 8,000,009 338 / 350 -> 233 / 251, 4,194,304 201 / 211 -> 146 / 162
+//   FP64  128^2: 8,000,009 150 / 235 -> 147 / 209
+//         256^2: 8,000,009 146 / 241 -> 163 / 215, but 4,194,304 88 / 133 -> 100 / 132
+//         1024^2: 8,000,009 353 / 353 -> 275 / 284, 1,048,576 68 / 73 -> 67 / 77
+//         2048^2: 4,194,304 243 / 260 -> 198 / 230, but 1,048,576 88 / 106 -> 84 / 119
 GatherPushPlan gather_push_plan(int64_t n, int nx, int ny, int fp64) {
   GatherPushPlan p;
   const long long G = (long long)nx * ny, pad = (long long)(nx + 1) * (ny + 1);
   const long long bytes = pad * (fp64 ? 16 : 8);
   p.pairs = 0;
+  p.rows = 0;
   p.lds = 0;
   if (bytes <= 72 * 1024 && n >= std::max(262144ll, 256 * G)) {
     p.lds = (int)bytes;
@@ -724,7 +763,12 @@ GatherPushPlan gather_push_plan(int64_t n, int nx, int ny, int fp64) {
     p.blocks = (int)(b > 512 ? 512 : b);
     return p;
   }
-  if (n >= 524288 && n >= G / 8) p.pairs = pad;
+  if (n >= 524288 && n >= G / 8) {
+    const long long state = n * (fp64 ? 32 : 16);
+    p.rows = n >= std::max(1048576ll, G) &&
+             (2 * bytes <= (4 << 20) / 3 || bytes > (6 << 20) || state >= (96ll << 20));
+    p.pairs = p.rows ? 2ll * nx * (ny + 1) : pad;
+  }
   const long long per = p.pairs ? 4 * PIC_WG : PIC_WG;
   const long long b = (n + per - 1) / per;
   p.blocks = (int)(b < 1 ? 1 : (b > 4096 ? 4096 : b));
@@ -742,9 +786,13 @@ void launch_op_gather_push(hipStream_t s, const GatherPushPlan& p, R* x, R* y, R
     k_op_gather_push<R, GP_LDS><<<p.blocks, GP_LDS_NT, p.lds, s>>>(
         x, y, vx, vy, n, ex, ey, nullptr, nx, ny, lx, ly, dt, qm, c, ke_partials);
   } else if (E) {
-    k_op_pack_E<R><<<grid_for((long long)nx * ny), PIC_WG, 0, s>>>(ex, ey, nx, ny, E);
-    k_op_gather_push<R, GP_PACKED><<<p.blocks, PIC_WG, 0, s>>>(
-        x, y, vx, vy, n, nullptr, nullptr, E, nx, ny, lx, ly, dt, qm, c, ke_partials);
+    k_op_pack_E<R><<<grid_for((long long)nx * ny), PIC_WG, 0, s>>>(ex, ey, nx, ny, p.rows, E);
+    if (p.rows)
+      k_op_gather_push<R, GP_ROWS><<<p.blocks, PIC_WG, 0, s>>>(
+          x, y, vx, vy, n, nullptr, nullptr, E, nx, ny, lx, ly, dt, qm, c, ke_partials);
+    else
+      k_op_gather_push<R, GP_PACKED><<<p.blocks, PIC_WG, 0, s>>>(
+          x, y, vx, vy, n, nullptr, nullptr, E, nx, ny, lx, ly, dt, qm, c, ke_partials);
   } else {
     k_op_gather_push<R, GP_NODES><<<p.blocks, PIC_WG, 0, s>>>(
         x, y, vx, vy, n, ex, ey, nullptr, nx, ny, lx, ly, dt, qm, c, ke_partials);

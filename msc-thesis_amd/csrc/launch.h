@@ -155,6 +155,7 @@ struct GatherPushPlan {
   int blocks;           // workgroups (and kinetic-energy partials)
   int lds;              // bytes of the padded field in LDS, 0: not there
   long long pairs;      // (Ex, Ey) pairs of the packed field, 0: not used
+  int rows;             // packed with the two node rows of a cell interleaved
 };
 GatherPushPlan gather_push_plan(int64_t n, int nx, int ny, int fp64);
 // pairs: memory for the plan's packed field, or NULL (then the node arrays are read)
