@@ -214,7 +214,7 @@ Ctx::~Ctx() {
   F(d_tscan_items);
   F(partials_push); F(partials_rows); F(diag);
   F(d_coll_counts); F(birth_count); F(birth_parent); F(birth_buf); F(gmax); F(flag);
-  F(coll_list); F(coll_count); F(coll_partials);
+  F(coll_list); F(coll_count); F(coll_partials); F(dsmc_slots);
   for (auto& e : ev) if (e) (void)hipEventDestroy(e);
   if (stream) (void)hipStreamDestroy(stream);
   workspace_trim(device);
@@ -454,7 +454,11 @@ int Ctx::alloc() {
     PIC_HIP(dalloc(&coll_count, PIC_MCC_BLOCKS));
     PIC_HIP(dalloc(&coll_partials, 4 * PIC_MCC_BLOCKS));
   }
-  if (any_dsmc) PIC_HIP(dalloc(&gmax, ctotal));
+  if (any_dsmc) {
+    PIC_HIP(dalloc(&gmax, ctotal));
+    PIC_HIP(dalloc(&dsmc_slots, DSMC_SLOTS * DSMC_SLOT_STRIDE));
+    PIC_HIP(hipMemset(dsmc_slots, 0, sizeof(*dsmc_slots) * DSMC_SLOTS * DSMC_SLOT_STRIDE));
+  }
   // twiddles exp(-2 pi i j / PIC_FFT_MAX)
   std::vector<double2> h(PIC_FFT_MAX / 2);
   for (int j = 0; j < PIC_FFT_MAX / 2; ++j) {
@@ -602,7 +606,7 @@ int Ctx::launch_collide_stage() {
       a.ncells = d.nx * d.ny; a.coeff = c.dsmc_coeff; a.seed = c.seed;
       // the cell sort numbers cells tile-major; gmax and the streams are row-major
       a.tile_shift = __builtin_ctz((unsigned)d.tile); a.tiles_y = d.tiles_y; a.ny = d.ny;
-      a.st = d_st + r; a.ncoll = d_coll_counts + 4 * r;
+      a.st = d_st + r; a.ncoll = d_coll_counts + 4 * r; a.slots = dsmc_slots;
       a.finish_after = finish_late() ? 1 : 0;
       a.diag = diag + d.dbase * 8;
       launch_dsmc(stream, a);

@@ -124,6 +124,7 @@ struct Ctx {
   int* coll_list = nullptr;   // MCC: slots that pass the null-collision test
   int* coll_count = nullptr;
   int* coll_partials = nullptr;
+  unsigned long long* dsmc_slots = nullptr;
   int* birth_parent = nullptr;
   float* birth_buf = nullptr;
   float* gmax = nullptr;               // per cell (ctotal)

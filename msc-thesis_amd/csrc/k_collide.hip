@@ -274,21 +274,23 @@ __device__ __forceinline__ uint32_t feistel_f(uint32_t r, uint32_t k, int half) 
   return h >> (32 - half);
 }
 
+__device__ __forceinline__ uint32_t pair_walk(uint32_t x, int half, const uint32_t key[4]) {
+  uint32_t l = x >> half, r = x & ((1u << half) - 1u);
+#pragma unroll
+  for (uint32_t i = 0; i < 12; ++i) {
+    const uint32_t f = feistel_f(r, key[i & 3] ^ (i * 0x632BE5ABu), half);
+    const uint32_t nl = r;
+    r = l ^ f;
+    l = nl;
+  }
+  return (l << half) | r;
+}
+
 __device__ __forceinline__ uint32_t pair_perm(uint32_t t, uint32_t n, int half,
                                               const uint32_t key[4]) {
-  const uint32_t mask = (1u << half) - 1u;
   uint32_t x = t;
-  do {
-    uint32_t l = x >> half, r = x & mask;
-#pragma unroll
-    for (uint32_t i = 0; i < 12; ++i) {
-      const uint32_t f = feistel_f(r, key[i & 3] ^ (i * 0x632BE5ABu), half);
-      const uint32_t nl = r;
-      r = l ^ f;
-      l = nl;
-    }
-    x = (l << half) | r;
-  } while (x >= n);
+  do x = pair_walk(x, half, key);
+  while (x >= n);
   return x;
 }
 
@@ -318,16 +320,13 @@ __device__ __forceinline__ int dsmc_cell_rm(int c, const DsmcArgs& a) {
   return cx * a.ny + cy;
 }
 
-// One candidate: the pair of slots (pi(2m), pi(2m+1)) of the cell's round permutation,
-// accepted when u gm < g with gm = max(gmax at the round's start, g); an accepted pair keeps
+// One candidate: the particles pi, pj at slots (pi(2m), pi(2m+1)) of the cell's round
+// permutation, accepted when u gm < g with gm = max(gmax at the round's start, g); an accepted pair keeps
 // its centre-of-mass velocity and turns its relative velocity to a uniform direction.
 // Returns g (for the round's new gmax); counts acceptances in acc.
-__device__ __forceinline__ double dsmc_candidate(const DsmcArgs& a, int b, uint32_t n,
-                                                 int half, const uint32_t key[4], int cr,
-                                                 uint32_t s32, long long k, uint32_t m,
-                                                 double gm, unsigned int& acc) {
-  const long long pi = b + (long long)pair_perm(2u * m, n, half, key);
-  const long long pj = b + (long long)pair_perm(2u * m + 1u, n, half, key);
+__device__ __forceinline__ double dsmc_candidate(const DsmcArgs& a, long long pi, long long pj,
+                                                 int cr, uint32_t s32, long long k, double gm,
+                                                 unsigned int& acc) {
   double w[4];
   draw4((uint32_t)cr, s32, (uint32_t)k, PIC_TAG_DSMC, a.seed, w);
   const double vix = a.vx[pi], viy = a.vy[pi], vjx = a.vx[pj], vjy = a.vy[pj];
@@ -353,15 +352,26 @@ __device__ __forceinline__ double dsmc_candidate(const DsmcArgs& a, int b, uint3
 // P = n/2 pairs; the pairs of a round are disjoint, so its candidates are independent.
 // After a round gmax = max(gmax, every g of the round) (a maximum: exact, order-free).
 //
-// One workgroup takes DSMC_CELLS consecutive cells: the per-cell set-up (offsets, gmax,
-// the draw of M, the first round's permutation key) runs a thread per cell, then the
-// first-round candidates of all its cells are dealt to the workgroup's threads together
+// One workgroup takes DSMC_CELLS cells, in pieces of 8 neighbours from all over the grid (dense
+// cells lie together, and a workgroup of them alone outlasts the rest): the per-cell set-up
+// (offsets, gmax, the draw of M, the first round's permutation key) runs a thread per cell, then
+// the first-round candidates of all its cells are dealt to the workgroup's threads together
 // (most cells need one round of a few candidates), and the few cells with more rounds go
 // on one at a time with the threads over the round's pairs.  Velocities are read and
 // written in HBM directly (only the candidates' particles are touched); a round that
 // follows another first waits for its stores (__syncthreads: workgroup-scope fence).
+//
+// Bound by the permutation: a slot takes up to four tries on average, each a chain of 24
+// dependent multiplications, and a dozen for the slowest lane of 64.  So the slots of the first
+// round come first, and a lane whose slot is found takes the workgroup's next one instead of
+// waiting for the others.  256^2 cells, 2,097,152 particles, a blob of 183 per cell at its
+// centre that spreads out over 280 steps: 33 us per launch with each candidate looking for its
+// two slots in turn, 64 consecutive cells per workgroup and an atomic per wave for the count of
+// accepted pairs, 22 now (of it the set-up 5, the pairs 9).
 #define DSMC_CELLS 64
-#define DSMC_THREADS 256
+#define DSMC_THREADS 128
+#define DSMC_PIECE_LOG 3
+#define DSMC_BATCH 1024  // first-round candidates whose slots are in LDS at once
 __global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
   __shared__ int s_b[DSMC_CELLS], s_n[DSMC_CELLS], s_cr[DSMC_CELLS], s_half[DSMC_CELLS];
   __shared__ int s_first[DSMC_CELLS + 1];
@@ -370,15 +380,21 @@ __global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
   __shared__ double s_gm[DSMC_CELLS];
   __shared__ unsigned long long s_gr[DSMC_CELLS];  // bits of the largest g (g >= 0: ordered)
   __shared__ unsigned long long s_more;
+  __shared__ unsigned int s_acc[DSMC_THREADS / 64];
+  __shared__ unsigned char s_cell[DSMC_BATCH];  // cell of a candidate
+  __shared__ uint32_t s_slot[2 * DSMC_BATCH];
   const int tid = threadIdx.x;
   const long long step = a.st ? a.st->step - (a.finish_after ? 0 : 1) : a.step;
   const uint32_t s32 = (uint32_t)step;
   const uint32_t sk0 = (uint32_t)a.seed, sk1 = (uint32_t)(a.seed >> 32);
   unsigned int acc = 0;
-  for (int c0 = blockIdx.x * DSMC_CELLS; c0 < a.ncells; c0 += gridDim.x * DSMC_CELLS) {
+  const int ngroups = (a.ncells + DSMC_CELLS - 1) / DSMC_CELLS;
+  for (int grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
     // ---- per-cell set-up, the first wave, a lane per cell
+    const int cell = ((tid >> DSMC_PIECE_LOG) * ngroups + grp) * (1 << DSMC_PIECE_LOG) +
+                     (tid & ((1 << DSMC_PIECE_LOG) - 1));
     if (tid < DSMC_CELLS) {
-      const int c = c0 + tid;
+      const int c = cell;
       int b = 0, n = 0, cr = 0;
       long long M = 0;
       double gm = 0.0;
@@ -425,18 +441,45 @@ __global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
     __syncthreads();
     // ---- first round of every cell, candidates dealt to the threads
     const int total = s_first[DSMC_CELLS];
-    for (int t = tid; t < total; t += DSMC_THREADS) {
-      int q = 0;  // cell of candidate t: s_first[q] <= t < s_first[q + 1]
+    for (int t0 = 0; t0 < total; t0 += DSMC_BATCH) {
+      const int nt = min(DSMC_BATCH, total - t0);
+      for (int t = tid; t < nt; t += DSMC_THREADS) {
+        int q = 0;  // cell of candidate t0 + t: s_first[q] <= t0 + t < s_first[q + 1]
 #pragma unroll
-      for (int w = DSMC_CELLS / 2; w > 0; w >>= 1)
-        if (s_first[q + w] <= t) q += w;
-      const uint32_t m = (uint32_t)(t - s_first[q]);
-      const uint32_t key[4] = {s_key[q][0], s_key[q][1], s_key[q][2], s_key[q][3]};
-      const double g = dsmc_candidate(a, s_b[q], (uint32_t)s_n[q], s_half[q], key, s_cr[q], s32,
-                                      (long long)m, m, s_gm[q], acc);
-      atomicMax(&s_gr[q], (unsigned long long)__double_as_longlong(g));
+        for (int w = DSMC_CELLS / 2; w > 0; w >>= 1)
+          if (s_first[q + w] <= t0 + t) q += w;
+        s_cell[t] = (unsigned char)q;
+      }
+      __syncthreads();
+      // slots: one walk per turn and lane
+      uint32_t x = 0, n = 0, key[4] = {0, 0, 0, 0};
+      int half = 1, i = tid - DSMC_THREADS;
+      bool next = true;
+      for (;;) {
+        if (next) {
+          i += DSMC_THREADS;
+          if (i >= 2 * nt) break;
+          const int q = s_cell[i >> 1];
+          x = (uint32_t)(2 * (t0 - s_first[q]) + i);  // slot 2 m or 2 m + 1 of its cell
+          n = (uint32_t)s_n[q];
+          half = s_half[q];
+          key[0] = s_key[q][0]; key[1] = s_key[q][1];
+          key[2] = s_key[q][2]; key[3] = s_key[q][3];
+        }
+        x = pair_walk(x, half, key);
+        next = x < n;
+        if (next) s_slot[i] = x;
+      }
+      __syncthreads();
+      for (int t = tid; t < nt; t += DSMC_THREADS) {
+        const int q = s_cell[t];
+        const double g = dsmc_candidate(a, s_b[q] + (long long)s_slot[2 * t],
+                                        s_b[q] + (long long)s_slot[2 * t + 1], s_cr[q], s32,
+                                        (long long)(t0 + t - s_first[q]), s_gm[q], acc);
+        atomicMax(&s_gr[q], (unsigned long long)__double_as_longlong(g));
+      }
+      __syncthreads();  // s_cell, s_slot are free
     }
-    __syncthreads();
     // ---- cells with further rounds, one at a time
     unsigned long long more = s_more;
     while (more) {
@@ -452,24 +495,42 @@ __global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
         const int npr = (int)((Mq - r0 < Pq) ? (Mq - r0) : Pq);
         __syncthreads();  // every thread has read s_gr[q] before it moves
         for (int m = tid; m < npr; m += DSMC_THREADS) {
-          const double g = dsmc_candidate(a, bq, (uint32_t)nq, hq, key, crq, s32, r0 + m,
-                                          (uint32_t)m, gq, acc);
+          const long long pi = bq + (long long)pair_perm(2u * m, (uint32_t)nq, hq, key);
+          const long long pj = bq + (long long)pair_perm(2u * m + 1u, (uint32_t)nq, hq, key);
+          const double g = dsmc_candidate(a, pi, pj, crq, s32, r0 + m, gq, acc);
           atomicMax(&s_gr[q], (unsigned long long)__double_as_longlong(g));
         }
         __syncthreads();
       }
     }
-    if (tid < DSMC_CELLS && c0 + tid < a.ncells && s_first[tid + 1] > s_first[tid])
+    if (tid < DSMC_CELLS && cell < a.ncells && s_first[tid + 1] > s_first[tid])
       a.gmax[s_cr[tid]] = (float)__longlong_as_double((long long)s_gr[tid]);
     __syncthreads();  // LDS reused by the next group of cells
   }
-  // accepted pairs: integer sum, order-free
+  // accepted pairs: integer sum, order-free.  Adds to one address take about 7 ns each, 7 us of a
+  // launch of 1024 workgroups: in the engine's runs a workgroup adds to one of DSMC_SLOTS
+  // counters (accepted pairs and, in the high bits, workgroups), and the last one of a counter
+  // passes its sum on and clears it.
   unsigned int t = acc;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-  if ((tid & 63) == 0 && t) {
-    if (a.ncoll) atomicAdd((unsigned long long*)a.ncoll, (unsigned long long)t);
-    if (a.diag) atomicAdd(&a.diag[(step % PIC_DIAG_CAP) * 8 + 6], (double)t);
+  if ((tid & 63) == 0) s_acc[tid >> 6] = t;
+  __syncthreads();
+  if (tid == 0) {
+    unsigned long long all = 0;
+    for (int w = 0; w < DSMC_THREADS / 64; ++w) all += s_acc[w];
+    if (a.slots) {
+      unsigned long long* c = a.slots + (blockIdx.x % DSMC_SLOTS) * DSMC_SLOT_STRIDE;
+      const int mine = (gridDim.x - 1 - blockIdx.x % DSMC_SLOTS) / DSMC_SLOTS + 1;
+      const unsigned long long v = atomicAdd(c, all + (1ull << 48)) + all + (1ull << 48);
+      all = 0;
+      if ((v >> 48) == (unsigned long long)mine) {
+        all = v & ((1ull << 48) - 1);
+        atomicExch(c, 0ull);
+      }
+    }
+    if (all && a.ncoll) atomicAdd((unsigned long long*)a.ncoll, all);
+    if (all && a.diag) atomicAdd(&a.diag[(step % PIC_DIAG_CAP) * 8 + 6], (double)all);
   }
 }
 

@@ -300,6 +300,8 @@ void launch_mcc(hipStream_t s, const MccArgs& a, int n_upper);
 void launch_mcc_births(hipStream_t s, const MccArgs& a, unsigned long long* scratch,
                        unsigned long long* rho, long long gsum, const RunDesc* runs, int run,
                        int n_upper);
+#define DSMC_SLOTS 32         // counters of accepted pairs
+#define DSMC_SLOT_STRIDE 16   // a cache line apart
 struct DsmcArgs {
   float *vx, *vy;
   const int* offsets;             // [ncells + 1] cell ranges in the sort's numbering
@@ -315,6 +317,7 @@ struct DsmcArgs {
   int finish_after;               // 1: the step's end runs after this stage (st->step is this
                                   // step's index; else its + 1)
   long long* ncoll;
+  unsigned long long* slots;      // [DSMC_SLOTS * DSMC_SLOT_STRIDE] zero between launches, or NULL
   double* diag;                   // the run's diagnostics rows (may be NULL)
 };
 void launch_dsmc(hipStream_t s, const DsmcArgs& a);
