@@ -132,6 +132,9 @@ static Tuning default_tuning(const pic_config& c, int tile, int halo, int splits
     t.splits = (int)std::max(1LL, std::min(64LL, s));
   }
   t.per_tile = splits == 0 && c.collide == PIC_COLLIDE_DSMC;
+  // (steps of 256^2 in 256 tiles, spread out / a blob: 100 particles per cell 345 / 634 us per
+  // tile, 332 / 615 in shares, 32: 142 / 166 and 126 / 157, 12: 89 / 104 and 93 / 105)
+  t.shares = t.per_tile && per_tile >= 6400 ? (int)(items + 0.5) : 0;
   return t;
 }
 
@@ -152,13 +155,14 @@ void Ctx::tune_runs(int tile, int halo, int splits, bool from_config) {
 
 // Items (run, tile x, tile y, split | splits << 16) of run r: t.splits per tile, or with
 // per-tile splits (and the tile offsets of the current order on the host) one split per
-// PUSH_SPLIT_TARGET particles of the tile, 1 to 64.
+// PUSH_SPLIT_TARGET particles of the tile, 1 to 64; or shares (run, -2, share, shares).
 void Ctx::push_items_for(int r, const int* toff_h) {
   RunDesc& d = rd[r];
   const Tuning& t = tune[r];
   constexpr long long PUSH_SPLIT_TARGET = 4096;
   d.push_item_begin = (int)push_items.size();
-  for (int tx = 0; tx < d.tiles_x; ++tx)
+  for (int s = 0; s < t.shares; ++s) push_items.push_back(make_int4(r, -2, s, t.shares));
+  for (int tx = 0; tx < d.tiles_x && !t.shares; ++tx)
     for (int ty = 0; ty < d.tiles_y; ++ty) {
       int S = t.splits;
       if (t.per_tile && toff_h) {
@@ -183,7 +187,7 @@ void Ctx::push_items_for(int r, const int* toff_h) {
 // sequences change.
 int Ctx::rebalance_push_items() {
   bool any = false;
-  for (int r = 0; r < nruns; ++r) any = any || (tune[r].per_tile && has_particles[r]);
+  for (int r = 0; r < nruns; ++r) any = any || (tune[r].per_tile && !tune[r].shares && has_particles[r]);
   if (!any) return PIC_OK;
   PIC_HIP(hipStreamSynchronize(stream));
   std::vector<int> toff_h((size_t)toffsum);
@@ -510,6 +514,11 @@ PushArgs<R> Ctx::push_args(int mode, int sort_mode) const {
   a.items = d_push; a.nitems = (int)push_items.size();
   a.nruns = nruns;
   a.partials = partials_push;
+  // cell order matters to the push from about 16 particles per cell on (steps of 256^2 with 32
+  // per cell 143 -> 132 us, 512^2 with 12 188 -> 182, but 64^2 with 2 or 6 55 -> 56, 58 -> 59)
+  bool shares = false;
+  for (const Tuning& t : tune) shares = shares || t.shares;
+  a.by_cell = shares || (any_dsmc && ptotal >= 16 * gsum);
   a.mode = mode; a.lds_bytes = lds_push;
   a.sort_mode = fused ? sort_mode : 0;
   a.ftable = sb.ftable;

@@ -65,6 +65,9 @@ struct Tuning {
   // splits per tile from each tile's particle count (DSMC runs asked for splits 0: the
   // blob-like densities of the collision workloads leave uniform splits unbalanced)
   bool per_tile = false;
+  // push items of equal particles whatever the tiles, 0: not (DSMC runs asked for splits 0 that
+  // have enough particles per tile)
+  int shares = 0;
 };
 
 struct Ctx {

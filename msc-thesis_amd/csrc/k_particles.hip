@@ -676,7 +676,13 @@ void launch_step_finish(hipStream_t s, const RunDesc* runs, RunState* st, int nr
 template <typename R>
 void launch_push(hipStream_t s, const PushArgs<R>& a) {
   if (a.nitems <= 0) return;
-  if (a.mode != 0)
+  if (a.by_cell) {
+    // FP32 only, and without the fused sort
+    if constexpr (sizeof(R) == 4) {
+      if (a.mode != 0) k_push<R, 1, 0, 1><<<a.nitems, PUSH_NT, a.lds_bytes, s>>>(a);
+      else k_push<R, 0, 0, 1><<<a.nitems, PUSH_NT, a.lds_bytes, s>>>(a);
+    }
+  } else if (a.mode != 0)
     k_push<R, 1, 0><<<a.nitems, PUSH_NT, a.lds_bytes, s>>>(a);
   else if (a.sort_mode == 1)
     k_push<R, 0, 1><<<a.nitems, PUSH_NT, a.lds_bytes, s>>>(a);

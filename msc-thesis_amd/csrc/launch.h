@@ -119,6 +119,8 @@ struct PushArgs {
   int nruns;
   double* partials;             // [nitems*3] per-workgroup kinetic energy, px, py
   int mode;                     // 0: gather+push+deposit, 1: deposit only
+  int by_cell;                  // the particles are in cell order, many per cell (DSMC); items
+                                // may be shares
   int lds_bytes;
   // sort fused into the push (mode 0, tile items): 0 off; 1 count the tiles of the new
   // positions per item into its row of ftable; 2 scatter the particles tile-major (by their
