@@ -70,14 +70,10 @@ __device__ __forceinline__ int bucket_lead_code(R x, R y, R vx, R vy, const Geo<
   locate_w(y, g.idy, g.ny, cy, f);
   const int sh = __builtin_ctz((unsigned)rd.tile);
   const int kx = cx >> sh, ky = cy >> sh;
-  int dx = kx - tx, dy = ky - ty;
-  if (dx > 1) dx -= rd.tiles_x;
-  else if (dx < -1) dx += rd.tiles_x;
-  if (dy > 1) dy -= rd.tiles_y;
-  else if (dy < -1) dy += rd.tiles_y;
-  const bool near = rd.tiles_x >= 3 && rd.tiles_y >= 3 && dx >= -1 && dx <= 1 && dy >= -1 &&
-                    dy <= 1;
-  const int code = near ? (dx + 1) * 3 + (dy + 1) : PUSH_NCODES;
+  // tiles per axis: a power of two
+  const int dx = pwrap(kx - tx + 1, rd.tiles_x), dy = pwrap(ky - ty + 1, rd.tiles_y);
+  const bool near = rd.tiles_x >= 3 && rd.tiles_y >= 3 && dx <= 2 && dy <= 2;
+  const int code = near ? dx * 3 + dy : PUSH_NCODES;
   return (kx * rd.tiles_y + ky) | (code << 16);
 }
 
