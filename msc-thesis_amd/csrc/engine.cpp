@@ -218,7 +218,7 @@ Ctx::~Ctx() {
   F(d_tscan_items);
   F(partials_push); F(partials_rows); F(diag);
   F(d_coll_counts); F(birth_count); F(birth_parent); F(birth_buf); F(gmax); F(flag);
-  F(coll_list); F(coll_count); F(coll_partials); F(dsmc_slots);
+  F(coll_list); F(coll_partials); F(dsmc_slots);
   for (auto& e : ev) if (e) (void)hipEventDestroy(e);
   if (stream) (void)hipStreamDestroy(stream);
   workspace_trim(device);
@@ -455,7 +455,6 @@ int Ctx::alloc() {
     int lb, lp;
     mcc_list_layout(maxcap, &lb, &lp);
     PIC_HIP(dalloc(&coll_list, (size_t)lb * lp));
-    PIC_HIP(dalloc(&coll_count, PIC_MCC_BLOCKS));
     PIC_HIP(dalloc(&coll_partials, 4 * PIC_MCC_BLOCKS));
   }
   if (any_dsmc) {
@@ -587,12 +586,12 @@ int Ctx::launch_collide_stage() {
       a.ng_vunit_dtphys = c.mcc_ng * c.mcc_v_unit * c.mcc_dt_phys * c.dt;
       const double numax_dt = numax_dt_of(r);
       a.nu_max_dt = numax_dt;
-      a.p_coll = 1.0 - std::exp(-numax_dt);
+      mcc_null_range(1.0 - std::exp(-numax_dt), &a.null_any, &a.null_last);
       a.mass_ratio2 = 2.0 * kMe / c.mcc_neutral_mass;
       a.seed = c.seed;
       a.counts = d_coll_counts + 4 * r;
       a.birth_count = birth_count; a.birth_parent = birth_parent; a.birth_buf = birth_buf;
-      a.coll_list = coll_list; a.coll_count = coll_count; a.coll_partials = coll_partials;
+      a.coll_list = coll_list; a.coll_partials = coll_partials;
       a.count_table = collide_count_table;
       a.from_state_step = 1;
       a.finish_after = finish_late() ? 1 : 0;

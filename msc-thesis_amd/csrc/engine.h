@@ -125,7 +125,6 @@ struct Ctx {
   long long* d_coll_counts = nullptr;  // [nruns*4]
   int* birth_count = nullptr;
   int* coll_list = nullptr;   // MCC: slots that pass the null-collision test
-  int* coll_count = nullptr;
   int* coll_partials = nullptr;
   unsigned long long* dsmc_slots = nullptr;
   int* birth_parent = nullptr;

@@ -9,6 +9,7 @@
 // with NTC hard-sphere like-particle collisions on the cell-sorted arrays, candidates in
 // rounds of disjoint pairs.
 // Random streams: counter {particle id | cell, step, draw, tag}, key = seed.
+#include <cmath>
 #include "launch.h"
 
 namespace {
@@ -19,20 +20,28 @@ __device__ __forceinline__ void cross_sections(double e, double& sel, double& se
   siz = (e > 15.8) ? 3e-20 * log_own(e / 15.8) / e : 0.0;
 }
 
+// One workgroup's share of the step's collisions, in two parts.
+//
 // Null-collision test, every particle: word 0 of Philox2x32-10 with counter (id, step) and
 // key seed_lo ^ seed_hi ^ 'MCC1'; the particles whose uniform falls below p_coll = 1 -
-// exp(-nu_max dt) (about 1 in 100) go to the step's collision list.  (A Philox4x32-10 block
-// per particle, of which the test used one word, made the kernel VALU-bound at ~100
-// instructions per particle.)  Workgroup b appends its hits to its own region
-// [b * per_block, (b + 1) * per_block) of the list through an LDS counter (one LDS atomic per
-// wave; one global counter for all of them serialised ~60k atomics per step on a single
-// address) and stores its count.  The collisions run on the list in a second launch, so the
-// waves do not carry the ~1 % of lanes through the long FP64 collision branch while the
-// other 63 wait.
+// exp(-nu_max dt) (about 1 in 100) go to the workgroup's region [b * per_block,
+// (b + 1) * per_block) of the collision list through an LDS counter (one LDS atomic per wave
+// and hit).  The uniform (c + 1/2) / 2^32 of word c is below p_coll for the words up to
+// null_last: an integer comparison.  Bound by the generator's ten multiplications (a
+// Philox4x32-10 block per particle, of which the test used one word, took twice as long).
+//
+// Then the collisions on the list, so that the waves do not carry the ~1 % of lanes through the
+// long FP64 branch while the other 63 wait: a Philox4x32-10 block keyed by (id, step), the
+// process chosen by u1 nu_max dt against the cumulative nu_k(E) dt, isotropic scattering in the
+// velocity plane; an ionisation appends a birth (ordered by parent id afterwards).  A few waves
+// per workgroup have work here, which the other workgroups' tests hide (8,388,608 particles:
+// 20 us; a launch of its own for the collisions 16.4 + 9.9).
 #define MCC_NULL_U 8
-__global__ __launch_bounds__(PIC_WG) void k_mcc_null(MccArgs a, int n_upper, int per_block) {
+__global__ __launch_bounds__(PIC_WG) void k_mcc(MccArgs a, int n_upper, int per_block) {
   __shared__ int s_cnt;
+  __shared__ int cnt[4];
   if (threadIdx.x == 0) s_cnt = 0;
+  if (threadIdx.x < 4) cnt[threadIdx.x] = 0;
   __syncthreads();
   const int np = min(a.st->np, n_upper);
   const long long step = a.from_state_step ? a.st->step - (a.finish_after ? 0 : 1) : a.step;
@@ -54,7 +63,7 @@ __global__ __launch_bounds__(PIC_WG) void k_mcc_null(MccArgs a, int n_upper, int
       const int q = q0 + j * stride;
       uint32_t ctr[2] = {idv[j], s32};
       philox2x32_10(ctr, nk);
-      const bool hit = q < np && u01(ctr[0]) < a.p_coll;
+      const bool hit = q < np && a.null_any && ctr[0] <= a.null_last;
       const unsigned long long mask = __ballot(hit);
       if (mask) {
         const int leader = __builtin_ctzll(mask);
@@ -66,21 +75,7 @@ __global__ __launch_bounds__(PIC_WG) void k_mcc_null(MccArgs a, int n_upper, int
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0) a.coll_count[blockIdx.x] = s_cnt;
-}
-
-// The collisions of the step's list (workgroup b takes region b of the null test): a
-// Philox4x32-10 block keyed by (id, step), the process chosen by u1 nu_max dt against
-// the cumulative nu_k(E) dt, isotropic scattering in the velocity plane; an ionisation
-// appends a birth (ordered by parent id afterwards).
-__global__ __launch_bounds__(PIC_WG) void k_mcc(MccArgs a, int per_block) {
-  __shared__ int cnt[4];
-  if (threadIdx.x < 4) cnt[threadIdx.x] = 0;
-  __syncthreads();
-  const int ncand = a.coll_count[blockIdx.x];
-  const int* list = a.coll_list + (long long)blockIdx.x * per_block;
-  const long long step = a.from_state_step ? a.st->step - (a.finish_after ? 0 : 1) : a.step;
-  const uint32_t s32 = (uint32_t)step;
+  const int ncand = s_cnt;
   for (int k = threadIdx.x; k < ncand; k += PIC_WG) {
     const long long i = a.pbase + list[k];
     const uint32_t pid = (uint32_t)a.id[i];
@@ -536,6 +531,13 @@ __global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
 
 }  // namespace
 
+void mcc_null_range(double p_coll, int* any, unsigned* last) {
+  // the words c with (c + 0.5) 2^-32 < p_coll: c < 2^32 p_coll - 0.5, all of it exact
+  const double n = std::ceil(p_coll * 4294967296.0 - 0.5);
+  *any = n >= 1.0;
+  *last = n >= 4294967296.0 ? 0xffffffffu : n >= 1.0 ? (unsigned)(n - 1.0) : 0u;
+}
+
 void mcc_list_layout(long long n_upper, int* blocks, int* per_block) {
   long long b = (n_upper + PIC_WG - 1) / PIC_WG;
   b = b < 1 ? 1 : (b > PIC_MCC_BLOCKS ? PIC_MCC_BLOCKS : b);
@@ -547,8 +549,7 @@ void mcc_list_layout(long long n_upper, int* blocks, int* per_block) {
 void launch_mcc(hipStream_t s, const MccArgs& a, int n_upper) {
   int blocks, per_block;
   mcc_list_layout(n_upper, &blocks, &per_block);
-  k_mcc_null<<<blocks, PIC_WG, 0, s>>>(a, n_upper, per_block);
-  k_mcc<<<blocks, PIC_WG, 0, s>>>(a, per_block);
+  k_mcc<<<blocks, PIC_WG, 0, s>>>(a, n_upper, per_block);
 }
 
 void launch_mcc_births(hipStream_t s, const MccArgs& a, unsigned long long* scratch,

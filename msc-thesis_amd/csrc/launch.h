@@ -272,7 +272,8 @@ struct MccArgs {
   int cap;
   double v_unit2_half_me_over_e;  // E[eV] = this * |v|^2
   double ng_vunit_dtphys;         // nu*dt = this * sigma(E) * |v|
-  double p_coll;                  // 1 - exp(-nu_max dt)
+  int null_any;                   // random words 0 .. null_last pass the null-collision test
+  unsigned null_last;             // (mcc_null_range)
   double nu_max_dt;               // nu_max * dt_phys
   double mass_ratio2;             // 2 m_e / M
   uint64_t seed;
@@ -288,15 +289,16 @@ struct MccArgs {
                                   // collisions are added to column PIC_DIAG_NCOLL
   int* coll_list;                 // slots that pass the null-collision test, a region of
                                   // per_block entries per workgroup (mcc_list_layout)
-  int* coll_count;                // [blocks] entries of each region
   int* coll_partials;             // [blocks][4] collision counts of each k_mcc workgroup
   int* count_table;               // sort fused into the push, after its count step: the
                                   // count table, to which the births add their tiles (in
                                   // the row of the tail item that will push them); else NULL
 };
-// MCC collision list layout for n_upper particles: the null-test grid and the list region
+// MCC collision list layout for n_upper particles: the grid of k_mcc and the list region
 // of each workgroup (its grid-stride share); the list needs blocks * per_block entries
 #define PIC_MCC_BLOCKS 2048
+// the random words that pass a null-collision test of probability p_coll
+void mcc_null_range(double p_coll, int* any, unsigned* last);
 void mcc_list_layout(long long n_upper, int* blocks, int* per_block);
 void launch_mcc(hipStream_t s, const MccArgs& a, int n_upper);
 void launch_mcc_births(hipStream_t s, const MccArgs& a, unsigned long long* scratch,

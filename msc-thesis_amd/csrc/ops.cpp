@@ -334,7 +334,7 @@ int pic_op_mcc(float* x, float* y, float* vx, float* vy, int32_t* id, int64_t* n
   Workspace m;
   RunState* st;
   RunDesc* dd;
-  int *bc, *bp, *cl, *cc, *cp;
+  int *bc, *bp, *cl, *cp;
   float* bb;
   unsigned long long *scratch, *rho;
   PIC_HIP(m.get(&st, 1));
@@ -345,7 +345,6 @@ int pic_op_mcc(float* x, float* y, float* vx, float* vy, int32_t* id, int64_t* n
   int lb, lp;
   mcc_list_layout(std::max<int64_t>(*n_io, 1), &lb, &lp);
   PIC_HIP(m.get(&cl, (size_t)lb * lp));
-  PIC_HIP(m.get(&cc, PIC_MCC_BLOCKS));
   PIC_HIP(m.get(&cp, 4 * PIC_MCC_BLOCKS));
   PIC_HIP(m.get(&scratch, 2 * std::max<int64_t>(cap, 1)));
   PIC_HIP(m.get(&rho, 2 * (size_t)c.nx * c.ny));
@@ -369,12 +368,12 @@ int pic_op_mcc(float* x, float* y, float* vx, float* vy, int32_t* id, int64_t* n
   a.ng_vunit_dtphys = c.mcc_ng * c.mcc_v_unit * c.mcc_dt_phys * c.dt;
   const double numax_dt = mcc_nu_max(c) * c.mcc_dt_phys * c.dt;
   a.nu_max_dt = numax_dt;
-  a.p_coll = 1.0 - std::exp(-numax_dt);
+  mcc_null_range(1.0 - std::exp(-numax_dt), &a.null_any, &a.null_last);
   a.mass_ratio2 = 2.0 * kMe / c.mcc_neutral_mass;
   a.seed = c.seed;
   a.counts = (long long*)counts;
   a.birth_count = bc; a.birth_parent = bp; a.birth_buf = bb;
-  a.coll_list = cl; a.coll_count = cc; a.coll_partials = cp;
+  a.coll_list = cl; a.coll_partials = cp;
   a.from_state_step = 0;
   a.step = step;
   launch_mcc(s, a, (int)*n_io);

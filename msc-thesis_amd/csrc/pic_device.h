@@ -137,6 +137,10 @@ __device__ __forceinline__ int qweight(R f) {
   return (int)rint(f * (R)(double)(1 << Fix<R>::QB));
 }
 
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);  // one instruction
+}
+
 // ------------------------------------------------------------- Philox4x32-10
 // Each round's two 32 x 32 -> 64-bit products are one v_mad_u64_u32 each (the high and low
 // words written separately cost a v_mul_hi_u32 and a v_mul_lo_u32 apiece).
@@ -148,7 +152,7 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32
     const uint64_t p1 = (uint64_t)c[2] * 0xCD9E8D57u;
     const uint32_t lo0 = (uint32_t)p0, hi0 = (uint32_t)(p0 >> 32);
     const uint32_t lo1 = (uint32_t)p1, hi1 = (uint32_t)(p1 >> 32);
-    uint32_t n0 = hi1 ^ c[1] ^ k0, n2 = hi0 ^ c[3] ^ k1;
+    uint32_t n0 = xor3(hi1, c[1], k0), n2 = xor3(hi0, c[3], k1);
     c[0] = n0; c[1] = lo1; c[2] = n2; c[3] = lo0;
   }
 }
@@ -160,7 +164,7 @@ __device__ __forceinline__ void philox2x32_10(uint32_t c[2], uint32_t k) {
   for (int r = 0; r < 10; ++r) {
     if (r > 0) k += 0x9E3779B9u;
     const uint64_t p = (uint64_t)c[0] * 0xD256D193u;
-    const uint32_t n0 = (uint32_t)(p >> 32) ^ k ^ c[1];
+    const uint32_t n0 = xor3((uint32_t)(p >> 32), k, c[1]);
     c[1] = (uint32_t)p;
     c[0] = n0;
   }
