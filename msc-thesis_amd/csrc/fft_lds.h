@@ -62,7 +62,11 @@ __device__ __forceinline__ void fft_lds_pass(double2* a, int rows, int n, int lo
 // (unnormalised).  tw[j] = exp(-2 pi i j / 2^logtw), j < 2^logtw / 2, logtw >= logn: the
 // global table (logtw = PIC_FFT_LOG) or a copy of the n-point twiddles in LDS
 // (fft_stage_twiddles, logtw = logn).  Radix-2 butterflies, three stages per pass in
-// registers (one barrier per pass), the groups of all rows spread over the workgroup.  All
+// registers (one barrier per pass), the groups of all rows spread over the workgroup; two stages
+// per pass up to 256 points, where eight values per thread leave most threads without work and
+// one thread's chain of butterflies is the pass (64 steps on 64^2: 1955 -> 1888 us, a gradient at
+// 128^2 6398 -> 6002, the 256^2 runs with collisions 0.3-0.6 %; at 512 and 1024 points two stages
+// cost 0.7 % and 3 %).  All
 // threads of the workgroup (NT) must call it.  PAD: the buffer's layout (fft_slot).
 template <int PAD = 0, int NT = PIC_WG>
 __device__ __forceinline__ void fft_lds_rows(double2* a, int rows, int n, int logn, int sign,
@@ -70,6 +74,12 @@ __device__ __forceinline__ void fft_lds_rows(double2* a, int rows, int n, int lo
                                              int logtw = PIC_FFT_LOG) {
   const double ws = (sign < 0) ? 1.0 : -1.0;
   int s = 1;
+  if (n <= 256) {
+    for (; s + 1 <= logn; s += 2) {
+      fft_lds_pass<2, PAD, NT>(a, rows, n, logn, s, ws, tw, logtw);
+      __syncthreads();
+    }
+  }
   for (; s + 2 <= logn; s += 3) {
     fft_lds_pass<3, PAD, NT>(a, rows, n, logn, s, ws, tw, logtw);
     __syncthreads();
