@@ -128,7 +128,7 @@ void record_forward(pic_adjoint& a) {
       PartBufs<R> dst{ck, ck + n, ck + 2 * n, ck + 3 * n, a.ids + (size_t)seg * n};
       SortBufs sb = a.sb;
       sb.toff = a.toffs + (size_t)seg * (a.nb + 1);
-      launch_tile_sort<R>(a.s, a.dd, a.st, 1, src, dst, sb, a.pitems, a.npitems);
+      launch_tile_sort<R>(a.s, a.dd, a.st, 1, src, dst, sb, a.pitems, a.npitems, PIC_CHUNK_SMALL);
       for (int q = 0; q < 4; ++q) in[q] = ck + q * n;
     }
     if (k == 0) {  // the initial charge, deposited once the particles are sorted
@@ -354,7 +354,7 @@ int pic_adjoint_create(const pic_config* cfg, const double* xl, const double* yl
     d.tile = T; d.halo = g.halo; d.tiles_x = g.nx / T; d.tiles_y = g.tiles_y;
     d.win = g.win; d.splits = g.splits; d.nbuckets = A.nb;
     // sort chunks of 1024 particles: the adjoint's runs are small (config 5: 512 chunks)
-    d.schunk = 1024;
+    d.schunk = PIC_CHUNK_SMALL;
     // tiles of the positions half a segment on: the drift of a segment is half of it either
     // way, so fewer nodes of the windows are touched (each costs an item's flush an atomic)
     d.sort_lead = 0.5 * std::min(A.K, nsteps) * cfg->dt;

@@ -551,10 +551,10 @@ int Ctx::launch_sort_stage() {
     // tile sort: the step only needs tiles to be contiguous
     if (fp64)
       launch_tile_sort<double>(stream, d_runs, d_st, nruns, bufs<double>(cur),
-                               bufs<double>(1 - cur), sb, d_pitems, (int)pitems.size());
+                               bufs<double>(1 - cur), sb, d_pitems, (int)pitems.size(), PIC_CHUNK);
     else
       launch_tile_sort<float>(stream, d_runs, d_st, nruns, bufs<float>(cur), bufs<float>(1 - cur),
-                              sb, d_pitems, (int)pitems.size());
+                              sb, d_pitems, (int)pitems.size(), PIC_CHUNK);
     cur ^= 1;
     return PIC_OK;
   }

@@ -18,7 +18,7 @@ namespace {
 // Stable counting sort of the particles by tile (sort bucket):
 //   1. k_tile_hist    per chunk of schunk particles: count of each bucket -> table[b][chunk]
 //   2. k_tscan_*      exclusive scan of the table in bucket-major order (per run)
-//   3. k_tile_scatter one wavefront per chunk walks its particles in index order; lanes
+//   3. k_tile_scatter the waves of a workgroup walk a chunk's quarters in index order; lanes
 //                     with equal buckets get consecutive slots (ballot ranks), so the
 //                     order inside a bucket is the previous order: deterministic and
 //                     stable without any per-cell sort.
@@ -213,78 +213,95 @@ __global__ __launch_bounds__(PIC_WG) void k_fscan_rows(const RunDesc* __restrict
   fscan_rows(runs, table, part, stride, items, blockIdx.x);
 }
 
-template <typename R>
-__global__ __launch_bounds__(64) void k_tile_scatter(const RunDesc* __restrict__ runs,
-                                                     RunState* __restrict__ st,
-                                                     PartBufs<R> src, PartBufs<R> dst,
-                                                     const int* __restrict__ table,
-                                                     int* __restrict__ toff,
-                                                     const int2* __restrict__ items) {
-  extern __shared__ int base[];
+// A workgroup per chunk of G * TILE_SCAT_NT particles, all of them in registers, an equal part
+// per wave in index order, in groups of 64.  Lanes with equal buckets are found by one ballot per
+// bucket bit, whatever the order, and the first lane of each bucket counts for all of them, so no
+// two lanes meet at a counter.  16,777,216 FP32 particles in no order: 169 us (40 bytes each
+// take 132 at the rate of a copy); a ballot per distinct bucket by one wave per chunk 224, the
+// state read again for the move 228, moved in the chunk's sorted order 236.  524,288 in order in
+// chunks of 1024: 24.6 -> 9.6.
+#define TILE_SCAT_NT 512
+template <typename R, int G>
+__global__ __launch_bounds__(TILE_SCAT_NT) void k_tile_scatter(const RunDesc* __restrict__ runs,
+                                                               RunState* __restrict__ st,
+                                                               PartBufs<R> src, PartBufs<R> dst,
+                                                               const int* __restrict__ table,
+                                                               int* __restrict__ toff,
+                                                               const int2* __restrict__ items) {
+  extern __shared__ int base[];  // [waves][nb]: counts, then the next slots
+  constexpr int NT = TILE_SCAT_NT, NW = NT / 64;
   const int2 it = items[blockIdx.x];
   const RunDesc rd = runs[it.x];
   const Geo<R> g = make_geo<R>(rd.nx, rd.ny, rd.lx, rd.ly);
   const int np = st[it.x].np;
   const int nb = rd.nbuckets;
-  const int chunk = it.y / rd.schunk;
-  const int lane = threadIdx.x;
-  for (int b = lane; b < nb; b += 64) {
-    const int v = table[rd.tbase + (long long)b * rd.nchunks + chunk];
-    base[b] = v;
-    if (chunk == 0) toff[rd.toffbase + b] = v;
+  const int chunk = it.y / (G * NT);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const long long pb = rd.pbase;
+  const int p1 = min(it.y + G * NT, np);
+  const int q0 = it.y + w * 64 * G + lane;  // this lane's particles: q0, q0 + 64, ...
+  R x[G], y[G], vx[G], vy[G];
+  int id[G];
+#pragma unroll
+  for (int i = 0; i < G; ++i) {
+    // lanes past p1 load the run's first particle
+    const int p = q0 + i * 64;
+    const long long pl = pb + (p < p1 ? p : 0);
+    x[i] = src.x[pl];
+    y[i] = src.y[pl];
+    vx[i] = src.vx[pl];
+    vy[i] = src.vy[pl];
+    id[i] = src.id[pl];
   }
-  if (chunk == 0 && lane == 0) {
+  for (int i = threadIdx.x; i < NW * nb; i += NT) base[i] = 0;
+  if (chunk == 0 && threadIdx.x == 0) {
     toff[rd.toffbase + nb] = np;
     st[it.x].nsorted = np;
   }
   __syncthreads();
-  const long long pb = rd.pbase;
-  const int p1 = min(it.y + rd.schunk, np);
-  // SCAT_U groups of 64 particles per pass: all their loads are issued first (the wave's
-  // memory latency is paid once per pass), then the groups are ranked in index order
-  constexpr int SCAT_U = 4;
-  for (int q0 = it.y; q0 < p1; q0 += 64 * SCAT_U) {
-    R vx[SCAT_U], vy[SCAT_U], vvx[SCAT_U], vvy[SCAT_U];
-    int vid[SCAT_U], key[SCAT_U];
+  const int nbits = nb > 1 ? 32 - __builtin_clz((unsigned)(nb - 1)) : 0;
+  int* __restrict__ wb = base + w * nb;
+  // bucket (bits 0-12), rank among the group's lanes of the bucket (13-18), their number (19-25)
+  unsigned at[G];
 #pragma unroll
-    for (int u = 0; u < SCAT_U; ++u) {
-      // lanes past p1 load particle p1 - 1 (p1 > q0 here): loads without branches
-      const int p = q0 + 64 * u + lane;
-      const int pl = p < p1 ? p : p1 - 1;
-      vx[u] = src.x[pb + pl];
-      vy[u] = src.y[pb + pl];
-      vvx[u] = src.vx[pb + pl];
-      vvy[u] = src.vy[pb + pl];
-      vid[u] = src.id[pb + pl];
+  for (int i = 0; i < G; ++i) {
+    const bool act = q0 + i * 64 < p1;
+    const unsigned key = (unsigned)bucket_lead<R>(x[i], y[i], vx[i], vy[i], g, rd);
+    unsigned long long m = __ballot(act);
+    for (int k = 0; k < nbits; ++k) {
+      const bool bit = (key >> k) & 1;
+      const unsigned long long ones = __ballot(bit);
+      m &= bit ? ones : ~ones;
     }
+    const unsigned r = (unsigned)lanes_below(m), c = (unsigned)__popcll(m);
+    if (act && r == 0) atomicAdd(&wb[key], (int)c);
+    at[i] = key | r << 13 | c << 19;
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < nb; b += NT) {
+    int v = table[rd.tbase + (long long)b * rd.nchunks + chunk];
+    if (chunk == 0) toff[rd.toffbase + b] = v;
 #pragma unroll
-    for (int u = 0; u < SCAT_U; ++u) {
-      const int p = q0 + 64 * u + lane;
-      key[u] = (p < p1) ? bucket_lead<R>(vx[u], vy[u], vvx[u], vvy[u], g, rd) : -1;
+    for (int k = 0; k < NW; ++k) {
+      const int c = base[k * nb + b];
+      base[k * nb + b] = v;
+      v += c;
     }
+  }
+  __syncthreads();
 #pragma unroll
-    for (int u = 0; u < SCAT_U; ++u) {
-      const int p = q0 + 64 * u + lane;
-      const bool act = p < p1;
-      unsigned long long rem = __ballot(act);
-      int d = 0;
-      while (rem) {
-        const int leader = __ffsll((long long)rem) - 1;
-        const int lk = __builtin_amdgcn_readlane(key[u], leader);
-        const unsigned long long m = __ballot(act && key[u] == lk);
-        const int b0 = base[lk];
-        if (act && key[u] == lk) d = b0 + __popcll(m & ((1ull << lane) - 1ull));
-        __syncthreads();
-        if (lane == leader) base[lk] = b0 + __popcll(m);
-        __syncthreads();
-        rem &= ~m;
-      }
-      if (act) {
-        dst.x[pb + d] = vx[u]; dst.y[pb + d] = vy[u]; dst.vx[pb + d] = vvx[u];
-        dst.vy[pb + d] = vvy[u];
-        dst.id[pb + d] = vid[u];
-      }
-    }
+  for (int i = 0; i < G; ++i) {
+    if (q0 + i * 64 >= p1) continue;
+    const unsigned key = at[i] & 8191u, r = (at[i] >> 13) & 63u;
+    const int b = wb[key];
+    const long long d = pb + b + (int)r;
+    // the group's lanes have read their slots before one of them moves the bucket's on, and
+    // the next group reads it after (one wave: program order)
+    __builtin_amdgcn_wave_barrier();
+    if (r == 0) wb[key] = b + (int)(at[i] >> 19);
+    __builtin_amdgcn_wave_barrier();
+    dst.x[d] = x[i]; dst.y[d] = y[i]; dst.vx[d] = vx[i]; dst.vy[d] = vy[i];
+    dst.id[d] = id[i];
   }
 }
 
@@ -633,7 +650,7 @@ void launch_reduce_sum(hipStream_t s, const double* parts, int n, double* out) {
 template <typename R>
 void launch_tile_sort(hipStream_t s, const RunDesc* runs, RunState* st, int nruns,
                       PartBufs<R> src, PartBufs<R> dst, SortBufs sb, const int2* pitems,
-                      int npitems) {
+                      int npitems, int schunk) {
   const size_t lds = sizeof(int) * (size_t)sb.max_buckets;
   k_tile_hist<R><<<npitems, PIC_WG, lds, s>>>(runs, st, src.x, src.y, src.vx, src.vy, sb.table,
                                                pitems);
@@ -642,7 +659,13 @@ void launch_tile_sort(hipStream_t s, const RunDesc* runs, RunState* st, int nrun
   k_tscan_chunks<<<nruns, PIC_WG, 0, s>>>(runs, sb.tchunk_sums);
   k_tscan_add<<<sb.ntscan_items, PIC_WG, 0, s>>>(runs, sb.table, sb.tchunk_sums,
                                                  sb.tscan_items);
-  k_tile_scatter<R><<<npitems, 64, lds, s>>>(runs, st, src, dst, sb.table, sb.toff, pitems);
+  const size_t scat = TILE_SCAT_NT / 64 * lds;
+  if (schunk == PIC_CHUNK)
+    k_tile_scatter<R, PIC_CHUNK / TILE_SCAT_NT><<<npitems, TILE_SCAT_NT, scat, s>>>(
+        runs, st, src, dst, sb.table, sb.toff, pitems);
+  else
+    k_tile_scatter<R, PIC_CHUNK_SMALL / TILE_SCAT_NT><<<npitems, TILE_SCAT_NT, scat, s>>>(
+        runs, st, src, dst, sb.table, sb.toff, pitems);
 }
 
 void launch_fused_scan(hipStream_t s, const RunDesc* runs, RunState* st, int nruns,
@@ -803,7 +826,7 @@ void launch_op_gather_push(hipStream_t s, const GatherPushPlan& p, R* x, R* y, R
 
 #define PIC_INST(R)                                                                          \
   template void launch_tile_sort<R>(hipStream_t, const RunDesc*, RunState*, int, PartBufs<R>,\
-                                    PartBufs<R>, SortBufs, const int2*, int);                 \
+                                    PartBufs<R>, SortBufs, const int2*, int, int);            \
   template void launch_push<R>(hipStream_t, const PushArgs<R>&);                            \
   template void launch_out_particles<R>(hipStream_t, const RunDesc*, RunState*, int, int,   \
                                         PartBufs<R>, const R*, void*, R*, R*, R*, R*);      \

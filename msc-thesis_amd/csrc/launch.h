@@ -55,7 +55,7 @@ void launch_fused_scan(hipStream_t s, const RunDesc* runs, RunState* st, int nru
 template <typename R>
 void launch_tile_sort(hipStream_t s, const RunDesc* runs, RunState* st, int nruns,
                       PartBufs<R> src, PartBufs<R> dst, SortBufs sb, const int2* pitems,
-                      int npitems);
+                      int npitems, int schunk);
 
 // ---- deposit of particles in any order (k_deposit.hip)
 enum { DEPOSIT_DIRECT, DEPOSIT_GRID, DEPOSIT_BINNED };
