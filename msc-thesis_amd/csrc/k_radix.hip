@@ -14,22 +14,24 @@
 // sort this replaced took one returning global atomic per particle (127 us for 3,000,017 in
 // 65,536 cells, random order) and then ordered each cell by index, a cell above 256
 // particles by one workgroup's bitonic network (2.9 ms for the 2-cell sort of 100,003).
-// Whole calls, before -> now: 434 -> 239 us (keys and sort of the 3,000,017), 7.0 -> 1.1 ms
-// (the reference's DSMC collide of 100,003 particles, which sorts twice).
+// Whole calls, counting sort -> this one: 434 -> 88 us (keys and sort of the 3,000,017); with the
+// other steps of it, 7.0 -> 0.21 ms (the reference's DSMC collide of 100,003 particles, which
+// sorts twice).
 #include "launch.h"
 
 namespace {
 
 #define RADIX_MAX 256            // digits per pass
-#define RADIX_NW (PIC_WG / 64)
+#define RADIX_NT 512             // threads of the scatter
 
 __device__ __forceinline__ int radix_lanes_below(unsigned long long m) {
   return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                         __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
 
-// Exclusive scan over the 256 threads of a workgroup; *total (every thread) the sum.  The
-// caller synchronises before wsum is used again.
+// Exclusive scan over the threads of a workgroup of NW waves; *total (every thread) the sum.
+// The caller synchronises before wsum is used again.
+template <int NW>
 __device__ __forceinline__ int wg_exclusive(int v, int* wsum, int* total) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   int inc = v;
@@ -42,7 +44,7 @@ __device__ __forceinline__ int wg_exclusive(int v, int* wsum, int* total) {
   __syncthreads();
   int pre = 0, sum = 0;
 #pragma unroll
-  for (int k = 0; k < RADIX_NW; ++k) {
+  for (int k = 0; k < NW; ++k) {
     if (k < w) pre += wsum[k];
     sum += wsum[k];
   }
@@ -82,7 +84,8 @@ __global__ __launch_bounds__(PIC_WG) void k_radix_hist(const int* __restrict__ k
 __global__ __launch_bounds__(PIC_WG) void k_radix_rows(int* __restrict__ table, int ntiles,
                                                        int* __restrict__ totals,
                                                        const int* __restrict__ flag) {
-  __shared__ int wsum[RADIX_NW];
+  constexpr int NW = PIC_WG / 64;
+  __shared__ int wsum[NW];
   if (flag && *flag) return;
   int* row = table + (long long)blockIdx.x * ntiles;
   int carry = 0;
@@ -94,7 +97,7 @@ __global__ __launch_bounds__(PIC_WG) void k_radix_rows(int* __restrict__ table, 
       v[k] = (i + k < ntiles) ? row[i + k] : 0;
       s += v[k];
     }
-    int ex = carry + wg_exclusive(s, wsum, &total);
+    int ex = carry + wg_exclusive<NW>(s, wsum, &total);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       if (i + k < ntiles) row[i + k] = ex;
@@ -108,20 +111,23 @@ __global__ __launch_bounds__(PIC_WG) void k_radix_rows(int* __restrict__ table, 
 
 // Items of a tile go by (wave, u, lane), which is their order in the input.  A wave ranks
 // its 64 items of one u by their digit with one ballot per digit bit (the lanes that agree
-// in every bit), on top of its running count of the digit in LDS.
+// in every bit), on top of its running count of the digit in LDS: a chain over the wave's items,
+// so tiles are spread over eight waves (us per pass with four, eight and sixteen: 3,000,017 items
+// in tiles of 4096 20.2, 19.7, 26; 100,003 in tiles of 1024 5.8, 5.0, 5.0).
 template <int IT, bool FIRST>
-__global__ __launch_bounds__(PIC_WG) void k_radix_scatter(
+__global__ __launch_bounds__(RADIX_NT) void k_radix_scatter(
     const int* __restrict__ keys, const int* __restrict__ idx, int n, int shift, int bits,
     int ntiles, const int* __restrict__ table, const int* __restrict__ totals,
     int* __restrict__ keys_out, int* __restrict__ idx_out, const int* __restrict__ flag) {
-  __shared__ int wh[RADIX_NW][RADIX_MAX];  // per-wave digit counts, then their prefix
+  constexpr int NT = RADIX_NT, NW = NT / 64;
+  __shared__ int wh[NW][RADIX_MAX];  // per-wave digit counts, then their prefix
   __shared__ int lstart[RADIX_MAX], gstart[RADIX_MAX];
-  __shared__ int wsum[2][RADIX_NW];
-  __shared__ int skey[IT * PIC_WG], sidx[IT * PIC_WG];
+  __shared__ int wsum[2][NW];
+  __shared__ int skey[IT * NT], sidx[IT * NT];
   if (*flag) return;
   const int nd = 1 << bits, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int tile0 = blockIdx.x * (IT * PIC_WG);
-  const int count = min(IT * PIC_WG, n - tile0);
+  const int tile0 = blockIdx.x * (IT * NT);
+  const int count = min(IT * NT, n - tile0);
   const int q0 = w * (IT * 64) + lane;
   int k[IT], ix[IT], rk[IT];
 #pragma unroll
@@ -131,7 +137,7 @@ __global__ __launch_bounds__(PIC_WG) void k_radix_scatter(
     ix[u] = FIRST ? p : idx[p];
   }
 #pragma unroll
-  for (int q = 0; q < RADIX_NW; ++q)
+  for (int q = 0; q < NW; ++q)
     if (threadIdx.x < nd) wh[q][threadIdx.x] = 0;
   __syncthreads();
 #pragma unroll
@@ -155,19 +161,19 @@ __global__ __launch_bounds__(PIC_WG) void k_radix_scatter(
   __syncthreads();
   {
     const int d = threadIdx.x;
-    int c[RADIX_NW], mine = 0;
+    int c[NW], mine = 0;
 #pragma unroll
-    for (int q = 0; q < RADIX_NW; ++q) {
+    for (int q = 0; q < NW; ++q) {
       c[q] = (d < nd) ? wh[q][d] : 0;
       mine += c[q];
     }
     int sum;
-    const int ls = wg_exclusive(mine, wsum[0], &sum);
-    const int gb = wg_exclusive(d < nd ? totals[d] : 0, wsum[1], &sum);
+    const int ls = wg_exclusive<NW>(mine, wsum[0], &sum);
+    const int gb = wg_exclusive<NW>(d < nd ? totals[d] : 0, wsum[1], &sum);
     if (d < nd) {
       int run = 0;
 #pragma unroll
-      for (int q = 0; q < RADIX_NW; ++q) {
+      for (int q = 0; q < NW; ++q) {
         wh[q][d] = run;
         run += c[q];
       }
@@ -185,7 +191,7 @@ __global__ __launch_bounds__(PIC_WG) void k_radix_scatter(
     sidx[lp] = ix[u];
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < count; i += PIC_WG) {
+  for (int i = threadIdx.x; i < count; i += NT) {
     const int key = skey[i];
     const int dst = gstart[((unsigned)key >> shift) & (nd - 1)] + i;
     keys_out[dst] = key;
@@ -193,30 +199,53 @@ __global__ __launch_bounds__(PIC_WG) void k_radix_scatter(
   }
 }
 
-__device__ __forceinline__ int lower_bound_i(const int* __restrict__ a, int n, int v) {
-  int lo = 0, hi = n;
+// lower bound of v in a[lo, hi), a quarter of the range per step (three loads at once)
+__device__ __forceinline__ int lower_bound_i(const int* __restrict__ a, int lo, int hi, int v) {
   while (lo < hi) {
-    const int mid = lo + ((hi - lo) >> 1);
-    if (a[mid] < v) lo = mid + 1;
-    else hi = mid;
+    const int len = hi - lo;
+    const int m1 = lo + len / 4, m2 = lo + len / 2, m3 = m2 + len / 4;  // all below hi
+    const bool b1 = a[m1] < v, b2 = a[m2] < v, b3 = a[m3] < v;
+    const int l = b3 ? m3 + 1 : b2 ? m2 + 1 : b1 ? m1 + 1 : lo;
+    hi = !b1 ? m1 : !b2 ? m2 : !b3 ? m3 : hi;
+    lo = l;
   }
   return lo;
 }
 
-// A search per cell (log2 n loads, the first of them shared by all cells) costs the same for
-// any gaps between the occupied cells; a cell's end is its right neighbour's search.
+// A search per cell costs the same for any gaps between the occupied cells; a cell's end is its
+// right neighbour's search.  The chain of its loads is the kernel's time, so it starts from the
+// range of the cell's last digit (the totals of the last pass; NULL: no items) and takes three
+// loads per step (3,000,017 items, 65,536 cells: 9 us; from the whole array, one load per step 12).
 __global__ __launch_bounds__(PIC_WG) void k_radix_offsets(const int* __restrict__ sorted, int n,
-                                                          int ncells, int* __restrict__ counts,
+                                                          int ncells, int shift, int bits,
+                                                          const int* __restrict__ totals,
+                                                          int* __restrict__ counts,
                                                           int* __restrict__ offsets,
                                                           const int* __restrict__ flag) {
+  constexpr int NW = PIC_WG / 64;
+  static_assert(RADIX_MAX == PIC_WG, "a digit per thread");
+  __shared__ int start[RADIX_MAX + 1];
+  __shared__ int wsum[NW];
   if (*flag) return;
+  {
+    int sum;
+    const int d = threadIdx.x;
+    start[d] = wg_exclusive<NW>(totals && d < (1 << bits) ? totals[d] : 0, wsum, &sum);
+    if (d == 0) start[RADIX_MAX] = sum;
+  }
+  __syncthreads();
   const int lane = threadIdx.x & 63;
+  auto search = [&](long long c) {
+    if (c >= ncells || n == 0) return n;
+    const int d = (int)c >> shift;
+    return lower_bound_i(sorted, start[d], start[d + 1], (int)c);
+  };
   for (long long c0 = blockIdx.x * (long long)PIC_WG + threadIdx.x - lane; c0 < ncells;
        c0 += (long long)gridDim.x * PIC_WG) {
     const long long c = c0 + lane;
-    const int b = lower_bound_i(sorted, n, (int)min(c, (long long)ncells));
+    const int b = search(c);
     int e = __shfl_down(b, 1, 64);
-    if (lane == 63) e = lower_bound_i(sorted, n, (int)min(c + 1, (long long)ncells));
+    if (lane == 63) e = search(c + 1);
     if (c < ncells) {
       offsets[c] = b;
       counts[c] = e - b;
@@ -228,6 +257,7 @@ __global__ __launch_bounds__(PIC_WG) void k_radix_offsets(const int* __restrict_
 template <int IT>
 void radix_passes(hipStream_t s, const int* keys, int n, int ncells, const RadixPlan& p,
                   RadixBufs b, int* perm, int* counts, int* offsets) {
+  constexpr int SIT = IT * PIC_WG / RADIX_NT;
   const int* kin = keys;
   const int* iin = nullptr;
   for (int q = 0; q < p.passes && n > 0; ++q) {
@@ -242,19 +272,18 @@ void radix_passes(hipStream_t s, const int* keys, int n, int ncells, const Radix
                                                          b.table, b.flag);
     launch_scan_rows(s, b.table, 1 << p.bits, p.tiles, b.totals, b.flag);
     if (q == 0)
-      k_radix_scatter<IT, true><<<p.tiles, PIC_WG, 0, s>>>(kin, iin, n, shift, p.bits, p.tiles,
-                                                           b.table, b.totals, kout, iout, b.flag);
+      k_radix_scatter<SIT, true><<<p.tiles, RADIX_NT, 0, s>>>(
+          kin, iin, n, shift, p.bits, p.tiles, b.table, b.totals, kout, iout, b.flag);
     else
-      k_radix_scatter<IT, false><<<p.tiles, PIC_WG, 0, s>>>(kin, iin, n, shift, p.bits, p.tiles,
-                                                            b.table, b.totals, kout, iout,
-                                                            b.flag);
+      k_radix_scatter<SIT, false><<<p.tiles, RADIX_NT, 0, s>>>(
+          kin, iin, n, shift, p.bits, p.tiles, b.table, b.totals, kout, iout, b.flag);
     kin = kout;
     iin = iout;
   }
   const long long blocks = ((long long)ncells + PIC_WG - 1) / PIC_WG;
-  k_radix_offsets<<<(int)(blocks > 16384 ? 16384 : blocks), PIC_WG, 0, s>>>(kin, n, ncells,
-                                                                           counts, offsets,
-                                                                           b.flag);
+  k_radix_offsets<<<(int)(blocks > 16384 ? 16384 : blocks), PIC_WG, 0, s>>>(
+      kin, n, ncells, (p.passes - 1) * p.bits, p.bits, n > 0 ? b.totals : nullptr, counts, offsets,
+      b.flag);
 }
 
 }  // namespace
