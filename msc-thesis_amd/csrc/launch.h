@@ -175,29 +175,33 @@ void launch_fill_u64(hipStream_t s, unsigned long long* p, long long n);
 void launch_reduce_sum(hipStream_t s, const double* parts, int n, double* out);
 
 // ---- field kernels (k_field.hip)
-// Row passes work on groups of consecutive rows (at most about 4096 complex values of LDS),
+// Row passes work on groups of consecutive rows (at most about 2048 complex values of LDS),
 // so the transposed spectra S[k][x] are read and written in contiguous runs along x.
 // Forward rows are packed in pairs (two real rows = one complex FFT).
 __host__ __device__ inline int fft_row_pairs_per_block(int nx, int ny) {
-  int p = 4096 / ny;
+  int p = 2048 / ny;
   p = p < 1 ? 1 : (p > 8 ? 8 : p);
   return p > nx / 2 ? nx / 2 : p;
 }
 __host__ __device__ inline int fft_rows_per_block(int nx, int ny) {
-  int r = 4096 / ny;
+  int r = 2048 / ny;
   r = r < 1 ? 1 : (r > 16 ? 16 : r);
   return r > nx ? nx : r;
 }
-// Group sizes used by a launch: about one workgroup per CU (256) over all runs' rows, never
-// above the per-grid limits.  A single large grid keeps one pair / row per workgroup (its
-// rows alone fill the chip); many small grids get grouped rows.
+// Group sizes used by a launch: from about one workgroup per CU (256) of rows, two of pairs, over
+// all runs' rows, never above the per-grid limits.  A single grid of 512 rows keeps one pair and
+// two rows per workgroup (one row: the field pass 9.0 -> 9.4 us); many small grids get grouped
+// rows.  Groups of half the values as before hold less LDS, so more of a CU's workgroups hide
+// each other's latency: 48 runs of 64^2 to 256^2 rows 12.3 -> 9.2 us, field 16.3 -> 12.9 (groups
+// of 1024 12.1, but the step of 1024^2 69.4 -> 73.4), the step of 2048^2 with few particles 248
+// -> 232 us (FP64 369 -> 341).
 inline int pow2_floor(long long v) {
   int p = 1;
   while ((long long)p * 2 <= v) p *= 2;
   return p;
 }
 inline void fft_groups(long long rows_total, int nx, int ny, int* pp, int* rf) {
-  const long long t = rows_total / 256, tp = rows_total / 512;
+  const long long t = rows_total / 256, tp = rows_total / 1024;
   const int gr = t >= 1 ? pow2_floor(t) : 1, gp = tp >= 1 ? pow2_floor(tp) : 1;
   *rf = fft_rows_per_block(nx, ny) < gr ? fft_rows_per_block(nx, ny) : gr;
   *pp = fft_row_pairs_per_block(nx, ny) < gp ? fft_row_pairs_per_block(nx, ny) : gp;
