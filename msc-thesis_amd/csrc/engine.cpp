@@ -182,6 +182,22 @@ void Ctx::push_items_for(int r, const int* toff_h) {
   d.push_item_end = (int)push_items.size();
 }
 
+// The runs in the order of their push items, the largest items first: a long item that starts
+// last is the end of the launch alone (48 runs of 16,384 to 1,769,472 particles, in the order of
+// the runs: 153 us per plain push, 288 per sort step; largest first 132, 233).
+std::vector<int> Ctx::push_order() const {
+  std::vector<int> order(nruns);
+  std::vector<double> per(nruns);
+  for (int r = 0; r < nruns; ++r) {
+    order[r] = r;
+    const Tuning& t = tune[r];
+    per[r] = (double)cfg[r].capacity /
+             (t.shares ? t.shares : (double)rd[r].tiles_x * rd[r].tiles_y * t.splits);
+  }
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return per[a] > per[b]; });
+  return order;
+}
+
 // Per-tile splits follow the tile counts of the current order: rebuilt from them (after a
 // sort) when a run asks for them.  Only the push items, their partials and the captured
 // sequences change.
@@ -193,7 +209,7 @@ int Ctx::rebalance_push_items() {
   std::vector<int> toff_h((size_t)toffsum);
   PIC_HIP(hipMemcpy(toff_h.data(), toffs[cur], sizeof(int) * toffsum, hipMemcpyDeviceToHost));
   push_items.clear();
-  for (int r = 0; r < nruns; ++r) push_items_for(r, has_particles[r] ? toff_h.data() : nullptr);
+  for (int r : push_order()) push_items_for(r, has_particles[r] ? toff_h.data() : nullptr);
   if (d_push) (void)hipFree(d_push);
   PIC_HIP(dalloc(&d_push, push_items.size()));
   PIC_HIP(hipMemcpy(d_push, push_items.data(), sizeof(int4) * push_items.size(),
@@ -274,7 +290,6 @@ int Ctx::build_items() {
     d.cell_item_begin = (int)citems.size();
     for (int c = 0; c < d.nx * d.ny; c += PIC_CELL_CHUNK) citems.push_back(make_int2(r, c));
     d.cell_item_end = (int)citems.size();
-    push_items_for(r, nullptr);
     d.fchunks = 0;
     fft_groups(rows_total, d.nx, d.ny, &d.fft_pp, &d.fft_rf);
     rp_begin.push_back((int)rowpair.size());
@@ -287,6 +302,7 @@ int Ctx::build_items() {
   }
   rp_begin.push_back((int)rowpair.size());
   col_begin.push_back((int)cols.size());
+  for (int r : push_order()) push_items_for(r, nullptr);
   if (lds_push > 160 * 1024) return fail(PIC_ERR_INVALID_CONFIG, "deposit window exceeds LDS");
   // Sort fused into the push: needs no cell lists (no DSMC), a cadence of at least two
   // steps (the count is taken one step ahead), and room in LDS for one counter per tile

@@ -142,6 +142,7 @@ struct Ctx {
   int alloc();
   void tune_runs(int tile, int halo, int splits, bool from_config);
   int build_items();
+  std::vector<int> push_order() const;
   void push_items_for(int r, const int* toff_h);
   int rebalance_push_items();
   int upload_runs();
