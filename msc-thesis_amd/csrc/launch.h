@@ -298,11 +298,11 @@ struct MccArgs {
                                   // count table, to which the births add their tiles (in
                                   // the row of the tail item that will push them); else NULL
 };
+// the random words that pass a null-collision test of probability p_coll
+void mcc_null_range(double p_coll, int* any, unsigned* last);
 // MCC collision list layout for n_upper particles: the grid of k_mcc and the list region
 // of each workgroup (its grid-stride share); the list needs blocks * per_block entries
 #define PIC_MCC_BLOCKS 2048
-// the random words that pass a null-collision test of probability p_coll
-void mcc_null_range(double p_coll, int* any, unsigned* last);
 void mcc_list_layout(long long n_upper, int* blocks, int* per_block);
 void launch_mcc(hipStream_t s, const MccArgs& a, int n_upper);
 void launch_mcc_births(hipStream_t s, const MccArgs& a, unsigned long long* scratch,
