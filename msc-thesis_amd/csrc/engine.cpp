@@ -132,9 +132,7 @@ static Tuning default_tuning(const pic_config& c, int tile, int halo, int splits
     t.splits = (int)std::max(1LL, std::min(64LL, s));
   }
   t.per_tile = splits == 0 && c.collide == PIC_COLLIDE_DSMC;
-  // (steps of 256^2 in 256 tiles, spread out / a blob: 100 particles per cell 345 / 634 us per
-  // tile, 332 / 615 in shares, 32: 142 / 166 and 126 / 157, 12: 89 / 104 and 93 / 105)
-  t.shares = t.per_tile && per_tile >= 6400 ? (int)(items + 0.5) : 0;
+  t.max_shares = t.per_tile ? (int)std::max(1.0, items + 0.5) : 0;
   return t;
 }
 
@@ -203,11 +201,18 @@ std::vector<int> Ctx::push_order() const {
 // sequences change.
 int Ctx::rebalance_push_items() {
   bool any = false;
-  for (int r = 0; r < nruns; ++r) any = any || (tune[r].per_tile && !tune[r].shares && has_particles[r]);
+  for (int r = 0; r < nruns; ++r) any = any || (tune[r].per_tile && has_particles[r]);
   if (!any) return PIC_OK;
   PIC_HIP(hipStreamSynchronize(stream));
   std::vector<int> toff_h((size_t)toffsum);
   PIC_HIP(hipMemcpy(toff_h.data(), toffs[cur], sizeof(int) * toffsum, hipMemcpyDeviceToHost));
+  // Equal shares from 6400 particles per tile on (steps of 256^2 in 256 tiles, spread out / a
+  // blob: 100 particles per cell 345 / 634 us per tile, 332 / 615 in shares, 32: 142 / 166 and
+  // 126 / 157, 12: 89 / 104 and 93 / 105)
+  for (int r = 0; r < nruns; ++r) {
+    const long long np = has_particles[r] ? toff_h[rd[r].toffbase + rd[r].nbuckets] : 0;
+    tune[r].shares = np >= 6400ll * rd[r].nbuckets ? tune[r].max_shares : 0;
+  }
   push_items.clear();
   for (int r : push_order()) push_items_for(r, has_particles[r] ? toff_h.data() : nullptr);
   if (d_push) (void)hipFree(d_push);

@@ -65,9 +65,9 @@ struct Tuning {
   // splits per tile from each tile's particle count (DSMC runs asked for splits 0: the
   // blob-like densities of the collision workloads leave uniform splits unbalanced)
   bool per_tile = false;
-  // push items of equal particles whatever the tiles, 0: not (DSMC runs asked for splits 0 that
-  // have enough particles per tile)
-  int shares = 0;
+  // push items of equal particles whatever the tiles, 0: not; and as many as there would be (DSMC
+  // runs asked for splits 0, by the particles they hold per tile)
+  int shares = 0, max_shares = 0;
 };
 
 struct Ctx {
