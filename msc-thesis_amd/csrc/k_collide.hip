@@ -295,9 +295,12 @@ __device__ __forceinline__ int pair_half_bits(uint32_t n) {
   return b >> 1;
 }
 
-__device__ __forceinline__ double wave_max_f64(double v) {
+__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned long long w = __shfl_xor(v, o, 64);
+    v = w > v ? w : v;
+  }
   return v;
 }
 
@@ -362,12 +365,14 @@ __device__ __forceinline__ double dsmc_candidate(const DsmcArgs& a, long long pi
 // waiting for the others.  256^2 cells, 2,097,152 particles, a blob of 183 per cell at its
 // centre that spreads out over 280 steps: 33 us per launch with each candidate looking for its
 // two slots in turn, 64 consecutive cells per workgroup and an atomic per wave for the count of
-// accepted pairs, 22 now (of it the set-up 5, the pairs 9).
+// accepted pairs, 22 now (of it the set-up 5, the pairs 9).  Further rounds deal their slots the
+// same way (1024 cells of 1500 particles, 4 to 6 rounds: 22.6 ms with the slots in turn and 256
+// threads, 46.5 with 128, 12.7 now; launch_dsmc chooses NT).
 #define DSMC_CELLS 64
-#define DSMC_THREADS 128
 #define DSMC_PIECE_LOG 3
 #define DSMC_BATCH 1024  // first-round candidates whose slots are in LDS at once
-__global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
+template <int NT>
+__global__ __launch_bounds__(NT) void k_dsmc(DsmcArgs a) {
   __shared__ int s_b[DSMC_CELLS], s_n[DSMC_CELLS], s_cr[DSMC_CELLS], s_half[DSMC_CELLS];
   __shared__ int s_first[DSMC_CELLS + 1];
   __shared__ long long s_M[DSMC_CELLS];
@@ -375,7 +380,7 @@ __global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
   __shared__ double s_gm[DSMC_CELLS];
   __shared__ unsigned long long s_gr[DSMC_CELLS];  // bits of the largest g (g >= 0: ordered)
   __shared__ unsigned long long s_more;
-  __shared__ unsigned int s_acc[DSMC_THREADS / 64];
+  __shared__ unsigned int s_acc[NT / 64];
   __shared__ unsigned char s_cell[DSMC_BATCH];  // cell of a candidate
   __shared__ uint32_t s_slot[2 * DSMC_BATCH];
   const int tid = threadIdx.x;
@@ -438,7 +443,7 @@ __global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
     const int total = s_first[DSMC_CELLS];
     for (int t0 = 0; t0 < total; t0 += DSMC_BATCH) {
       const int nt = min(DSMC_BATCH, total - t0);
-      for (int t = tid; t < nt; t += DSMC_THREADS) {
+      for (int t = tid; t < nt; t += NT) {
         int q = 0;  // cell of candidate t0 + t: s_first[q] <= t0 + t < s_first[q + 1]
 #pragma unroll
         for (int w = DSMC_CELLS / 2; w > 0; w >>= 1)
@@ -448,11 +453,11 @@ __global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
       __syncthreads();
       // slots: one walk per turn and lane
       uint32_t x = 0, n = 0, key[4] = {0, 0, 0, 0};
-      int half = 1, i = tid - DSMC_THREADS;
+      int half = 1, i = tid - NT;
       bool next = true;
       for (;;) {
         if (next) {
-          i += DSMC_THREADS;
+          i += NT;
           if (i >= 2 * nt) break;
           const int q = s_cell[i >> 1];
           x = (uint32_t)(2 * (t0 - s_first[q]) + i);  // slot 2 m or 2 m + 1 of its cell
@@ -466,7 +471,7 @@ __global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
         if (next) s_slot[i] = x;
       }
       __syncthreads();
-      for (int t = tid; t < nt; t += DSMC_THREADS) {
+      for (int t = tid; t < nt; t += NT) {
         const int q = s_cell[t];
         const double g = dsmc_candidate(a, s_b[q] + (long long)s_slot[2 * t],
                                         s_b[q] + (long long)s_slot[2 * t + 1], s_cr[q], s32,
@@ -488,13 +493,34 @@ __global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
         uint32_t key[4] = {(uint32_t)crq, s32, 0x80000000u | (uint32_t)(r0 / Pq), PIC_TAG_DSMP};
         philox4x32_10(key, sk0, sk1);
         const int npr = (int)((Mq - r0 < Pq) ? (Mq - r0) : Pq);
-        __syncthreads();  // every thread has read s_gr[q] before it moves
-        for (int m = tid; m < npr; m += DSMC_THREADS) {
-          const long long pi = bq + (long long)pair_perm(2u * m, (uint32_t)nq, hq, key);
-          const long long pj = bq + (long long)pair_perm(2u * m + 1u, (uint32_t)nq, hq, key);
-          const double g = dsmc_candidate(a, pi, pj, crq, s32, r0 + m, gq, acc);
-          atomicMax(&s_gr[q], (unsigned long long)__double_as_longlong(g));
+        // the slots first, dealt to the lanes as in the first round; the round's largest g by
+        // its bits (g >= 0, a NaN stays the largest) in a register per thread, then one LDS
+        // atomic per wave: atomics of every candidate on the cell's one word held the round up
+        unsigned long long gl = 0;
+        for (int m0 = 0; m0 < npr; m0 += DSMC_BATCH) {
+          const int nt = min(DSMC_BATCH, npr - m0);
+          int i = tid;
+          uint32_t x = (uint32_t)(2 * m0 + i);
+          while (i < 2 * nt) {
+            x = pair_walk(x, hq, key);
+            if (x < (uint32_t)nq) {
+              s_slot[i] = x;
+              i += NT;
+              x = (uint32_t)(2 * m0 + i);
+            }
+          }
+          __syncthreads();  // (and every thread has read s_gr[q] before it moves)
+          for (int t = tid; t < nt; t += NT) {
+            const double g = dsmc_candidate(a, bq + (long long)s_slot[2 * t],
+                                            bq + (long long)s_slot[2 * t + 1], crq, s32,
+                                            r0 + m0 + t, gq, acc);
+            const unsigned long long gb = (unsigned long long)__double_as_longlong(g);
+            gl = gb > gl ? gb : gl;
+          }
+          if (m0 + DSMC_BATCH < npr) __syncthreads();  // s_slot is free
         }
+        gl = wave_max_u64(gl);
+        if ((tid & 63) == 0) atomicMax(&s_gr[q], gl);
         __syncthreads();
       }
     }
@@ -513,7 +539,7 @@ __global__ __launch_bounds__(DSMC_THREADS) void k_dsmc(DsmcArgs a) {
   __syncthreads();
   if (tid == 0) {
     unsigned long long all = 0;
-    for (int w = 0; w < DSMC_THREADS / 64; ++w) all += s_acc[w];
+    for (int w = 0; w < NT / 64; ++w) all += s_acc[w];
     if (a.slots) {
       unsigned long long* c = a.slots + (blockIdx.x % DSMC_SLOTS) * DSMC_SLOT_STRIDE;
       const int mine = (gridDim.x - 1 - blockIdx.x % DSMC_SLOTS) / DSMC_SLOTS + 1;
@@ -563,5 +589,11 @@ void launch_mcc_births(hipStream_t s, const MccArgs& a, unsigned long long* scra
 void launch_dsmc(hipStream_t s, const DsmcArgs& a) {
   int blocks = (a.ncells + DSMC_CELLS - 1) / DSMC_CELLS;
   blocks = blocks < 1 ? 1 : (blocks > 65536 ? 65536 : blocks);
-  k_dsmc<<<blocks, DSMC_THREADS, 0, s>>>(a);
+  // Up to two workgroups per CU the threads of one are the time, above it how many workgroups
+  // fit a CU (95 registers: ten of 128 threads, five of 256).  128 / 256 threads, whole calls (us),
+  // 100 particles per cell, half a round and four: 8192 cells 91 / 65 and 1620 / 1585, 32,768
+  // 119 / 85 and 2183 / 2145, 65,536 129 / 122 but 2411 / 2829, 131,072 193 / 209 and 8669 / 11244
+  // (eight rounds).
+  if (blocks <= 512) k_dsmc<256><<<blocks, 256, 0, s>>>(a);
+  else k_dsmc<128><<<blocks, 128, 0, s>>>(a);
 }
