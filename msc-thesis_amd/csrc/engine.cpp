@@ -92,12 +92,22 @@ static int default_cadence(const std::vector<pic_config>& cfg) {
   return 8;
 }
 
+// LDS of a push workgroup's windows: the charge (one or two int64 words per node, padded to 16 B)
+// and the field.
+static int push_window_lds(int win, bool fp64) {
+  const int nwin = win * win * (fp64 ? 2 : 1);
+  return ((nwin + 1) & ~1) * 8 + win * win * (fp64 ? 16 : 8);
+}
+static const int PUSH_LDS_MAX = 160 * 1024;
+
 // Tiling of a run whose share of the launch is `items` workgroups; nonzero values are kept.
 //   tile    the largest up to 32 that leaves half as many tiles as items (at most 128), 8 at
 //           least: a push workgroup pays for its windows, but a 64^2 grid in 16 tiles of 16^2 leaves most
 //           CUs idle (two-stream, 64^2, 409,600 FP64 particles: 46 us per step in 16 x 4
 //           workgroups, 26 in 64 x 4).  64 on FP32 grids that 32 leaves in more than 512 tiles
 //           (1024^2, 16 M particles: 375 us per step with 16, 259 with 32, 217 with 64)
+//           A halo the caller gives may not fit such tiles (1024^2 FP32, halo 24: 204 KB with 64,
+//           68 KB with 16): they are halved to 16 cells until the window fits
 //   halo    16 where half a cycle's drift of 2.5 thermal speeds passes 8 cells, else 8
 //   splits  as many as make up the items, of 256 particles at least and 65,536 at most
 static Tuning default_tuning(const pic_config& c, int tile, int halo, int splits, int cadence,
@@ -105,6 +115,9 @@ static Tuning default_tuning(const pic_config& c, int tile, int halo, int splits
   Tuning t;
   const int m = std::min(c.nx, c.ny);
   const long long n = std::max<long long>(c.capacity, 1);
+  if (!halo) halo = 2.5 * cells_per_step(c) * (0.5 * cadence + 1.0) > 8.0 ? 16 : 8;
+  // the window (tile + 2 halo + 1 nodes) must not wrap onto itself: win <= min(nx, ny)
+  auto halo_of = [&](int side) { return std::min(halo, std::max(0, (m - side - 1) / 2)); };
   if (tile) {
     t.tile = std::min(tile, m / 2);
   } else {
@@ -114,13 +127,13 @@ static Tuning default_tuning(const pic_config& c, int tile, int halo, int splits
     // above 512 tiles the sort leaves the push: FP32 windows of 64 cells still fit
     if (c.precision == PIC_FP32 && (c.nx / t.tile) * (c.ny / t.tile) > 512 && m >= 128)
       t.tile = 64;
+    while (t.tile > 16 && push_window_lds(t.tile + 2 * halo_of(t.tile) + 1,
+                                          c.precision == PIC_FP64) > PUSH_LDS_MAX)
+      t.tile /= 2;
   }
   // at most 4096 tiles (the sort keeps one counter per tile in LDS)
   while ((c.nx / t.tile) * (c.ny / t.tile) > 4096 && t.tile < m / 2) t.tile *= 2;
-  // the window (tile + 2 halo + 1 nodes) must not wrap onto itself: win <= min(nx, ny)
-  const int hmax = std::max(0, (m - t.tile - 1) / 2);
-  if (!halo) halo = 2.5 * cells_per_step(c) * (0.5 * cadence + 1.0) > 8.0 ? 16 : 8;
-  t.halo = std::min(halo, hmax);
+  t.halo = halo_of(t.tile);
   const int ntiles = (c.nx / t.tile) * (c.ny / t.tile);
   const long long per_tile = n / ntiles;
   if (splits) {
@@ -273,9 +286,7 @@ int Ctx::build_items() {
     d.tile = t.tile; d.halo = t.halo; d.splits = t.splits;
     d.tiles_x = d.nx / t.tile; d.tiles_y = d.ny / t.tile;
     d.win = t.tile + 2 * t.halo + 1;
-    // LDS: charge window (1 or 2 int64 words per node, padded to 16 B) + field window
-    const int nwin = d.win * d.win * (fp64 ? 2 : 1);
-    lds_push = std::max(lds_push, ((nwin + 1) & ~1) * 8 + d.win * d.win * (fp64 ? 16 : 8));
+    lds_push = std::max(lds_push, push_window_lds(d.win, fp64));
     const long long preg = round_up(std::max<long long>(d.pcap, 1), PIC_CHUNK);
     d.nbuckets = d.tiles_x * d.tiles_y;
     d.nchunks = (int)(preg / PIC_CHUNK);
@@ -308,7 +319,7 @@ int Ctx::build_items() {
   rp_begin.push_back((int)rowpair.size());
   col_begin.push_back((int)cols.size());
   for (int r : push_order()) push_items_for(r, nullptr);
-  if (lds_push > 160 * 1024) return fail(PIC_ERR_INVALID_CONFIG, "deposit window exceeds LDS");
+  if (lds_push > PUSH_LDS_MAX) return fail(PIC_ERR_INVALID_CONFIG, "deposit window exceeds LDS");
   // Sort fused into the push: needs no cell lists (no DSMC), a cadence of at least two
   // steps (the count is taken one step ahead), and room in LDS for one counter per tile
   // (int) and two per tile and wave (16-bit pass counts).  MCC births join it through the
@@ -316,7 +327,7 @@ int Ctx::build_items() {
   // appended).
   const int fused_lds = (PUSH_NW + 1) * maxb * (int)sizeof(int);
   fused = !any_dsmc && sort_every >= 2 && maxb <= 512 &&
-          lds_push + fused_lds <= 160 * 1024;
+          lds_push + fused_lds <= PUSH_LDS_MAX;
   fscan_items.clear();
   long long fsum = 0;
   for (int r = 0; r < nruns && fused; ++r) {
