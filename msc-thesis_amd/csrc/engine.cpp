@@ -271,7 +271,24 @@ int Ctx::upload_runs() {
   return PIC_OK;
 }
 
+// The tunings as build_items will use them: an error, and nothing changed, when it cannot.
+int Ctx::check_tunings() const {
+  for (int r = 0; r < nruns; ++r) {
+    const Tuning& t = tune[r];
+    const long long nb = (long long)(rd[r].nx / t.tile) * (rd[r].ny / t.tile);
+    const long long nchunks = round_up(std::max<long long>(rd[r].pcap, 1), PIC_CHUNK) / PIC_CHUNK;
+    if (push_window_lds(t.tile + 2 * t.halo + 1, fp64) > PUSH_LDS_MAX)
+      return fail(PIC_ERR_INVALID_CONFIG, "deposit window exceeds LDS");
+    if (nb > 4096) return fail(PIC_ERR_INVALID_CONFIG, "more than 4096 tiles: use a larger tile");
+    if (nb * nchunks >= (1ll << 31))
+      return fail(PIC_ERR_INVALID_CONFIG, "tile table too large: use a larger tile");
+  }
+  return PIC_OK;
+}
+
 int Ctx::build_items() {
+  int rc = check_tunings();
+  if (rc) return rc;
   pitems.clear(); citems.clear(); rowpair.clear(); cols.clear(); rows.clear(); push_items.clear();
   tscan_items.clear(); rp_begin.clear(); col_begin.clear();
   lds_push = 0;
@@ -291,9 +308,6 @@ int Ctx::build_items() {
     d.nbuckets = d.tiles_x * d.tiles_y;
     d.nchunks = (int)(preg / PIC_CHUNK);
     d.schunk = PIC_CHUNK;
-    if (d.nbuckets > 4096) return fail(PIC_ERR_INVALID_CONFIG, "more than 4096 tiles: use a larger tile");
-    if ((long long)d.nbuckets * d.nchunks >= (1ll << 31))
-      return fail(PIC_ERR_INVALID_CONFIG, "tile table too large: use a larger tile");
     maxb = std::max(maxb, d.nbuckets);
     d.tbase = tsum; tsum += (long long)d.nbuckets * d.nchunks;
     d.toffbase = toffsum; toffsum += d.nbuckets + 1;
@@ -319,7 +333,6 @@ int Ctx::build_items() {
   rp_begin.push_back((int)rowpair.size());
   col_begin.push_back((int)cols.size());
   for (int r : push_order()) push_items_for(r, nullptr);
-  if (lds_push > PUSH_LDS_MAX) return fail(PIC_ERR_INVALID_CONFIG, "deposit window exceeds LDS");
   // Sort fused into the push: needs no cell lists (no DSMC), a cadence of at least two
   // steps (the count is taken one step ahead), and room in LDS for one counter per tile
   // (int) and two per tile and wave (16-bit pass counts).  MCC births join it through the
@@ -359,7 +372,6 @@ int Ctx::build_items() {
       PIC_HIP(hipMemcpy(*dptr, vec.data(), sizeof(T) * vec.size(), hipMemcpyHostToDevice));
     return PIC_OK;
   };
-  int rc;
   if ((rc = up(pitems, &d_pitems))) return rc;
   if ((rc = up(citems, &d_citems))) return rc;
   if ((rc = up(rowpair, &d_rowpair))) return rc;
@@ -1234,10 +1246,17 @@ int pic_set_tuning(pic_ctx* ctx, int tile, int halo, int splits, int sort_every)
       return fail(PIC_ERR_ARG, "tile must be a power of two <= min(nx, ny)/2 and <= 64");
   }
   PIC_HIP(hipStreamSynchronize(x.stream));
+  const std::vector<Tuning> was = x.tune;
+  const int was_every = x.sort_every;
   if (sort_every) x.sort_every = sort_every;
   x.tune_runs(tile, halo, splits, false);
-  int rc = x.build_items();
-  if (rc) return rc;
+  int rc = x.check_tunings();
+  if (rc) {  // refused: the tuning in force stays
+    x.tune = was;
+    x.sort_every = was_every;
+    return rc;
+  }
+  if ((rc = x.build_items())) return rc;
   // offsets must describe the current order for the new tiling: sort now
   bool any = false;
   for (int r = 0; r < x.nruns; ++r) any |= x.has_particles[r] != 0;

@@ -141,6 +141,7 @@ struct Ctx {
   ~Ctx();
   int alloc();
   void tune_runs(int tile, int halo, int splits, bool from_config);
+  int check_tunings() const;
   int build_items();
   std::vector<int> push_order() const;
   void push_items_for(int r, const int* toff_h);
