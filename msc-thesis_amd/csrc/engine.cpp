@@ -98,7 +98,8 @@ static int push_window_lds(int win, bool fp64) {
   const int nwin = win * win * (fp64 ? 2 : 1);
   return ((nwin + 1) & ~1) * 8 + win * win * (fp64 ? 16 : 8);
 }
-static const int PUSH_LDS_MAX = 160 * 1024;
+// what the windows and the fused sort's counters may take: k_push's own sums (196 B) come on top
+static const int PUSH_LDS_MAX = 160 * 1024 - 256;
 
 // Tiling of a run whose share of the launch is `items` workgroups; nonzero values are kept.
 //   tile    the largest up to 32 that leaves half as many tiles as items (at most 128), 8 at
