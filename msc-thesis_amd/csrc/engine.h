@@ -159,7 +159,7 @@ struct Ctx {
   template <typename R> PushArgs<R> push_args(int mode, int sort_mode = 0) const;
 
   // launches (no synchronisation)
-  int launch_field_run(int run, int want_phi);  // the field of one run's current positions
+  int launch_field_run(int run, int want_phi);  // E or phi of one run's current positions
   int launch_push_stage(int mode, int sort_mode = 0);
   int launch_sort_stage();
   int launch_collide_stage();

@@ -13,9 +13,10 @@
 //   field   : Ex + i Ey from one inverse complex row FFT per row (groups of rows per
 //             workgroup); writes the padded (Ex, Ey) node array and the field energy
 //             (fixed-order reduction)
-// A solve that wants phi alone (pic_op_poisson) transforms one output per column instead of
-// three and skips the field pass: at 1024^2 the column pass took 42 us (four rows of a column
-// left room for one workgroup per CU) and takes 16.5, the field pass took 20.
+// A solve that wants phi (pic_op_poisson, pic_get_grid) leaves E as it was: it transforms one
+// output per column instead of three and skips the field pass.  At 1024^2 the column pass took
+// 42 us (four rows of a column left room for one workgroup per CU) and takes 16.5, the field pass
+// took 20; at nx = 2048 four rows and the pass's own sums do not fit the LDS at all.
 // Inside a captured sequence of steps the three kernels also run the previous step's
 // end-of-step work in extra workgroups after their own items (step_tail.h): its
 // diagnostics row (rows) and step counter (columns), and on the step after a count step
@@ -111,15 +112,13 @@ __device__ __forceinline__ void fft_col_item(const FieldArgs& a, double2* lds) {
   const RunDesc rd = a.runs[it.x];
   const int nx = rd.nx, ny = rd.ny, lognx = rd.lognx;
   const int k = it.y;
-  // nxp slots per row; the outputs back to back (row r of a buffer starts at slot r nxp): Ex,
-  // Ey and, when wanted, phi, or phi alone
+  // nxp slots per row; the outputs back to back (row r of a buffer starts at slot r nxp): Ex and
+  // Ey, or phi alone
   const int nxp = fft_slot<PAD>(nx), mxp = a.max_nx + (a.max_nx >> 3);
-  const bool want_E = !a.phi_only;
-  const int nout = want_E ? (a.want_phi ? 3 : 2) : 1;
+  const int nout = a.want_phi ? 1 : 2;
   double2* col = lds;
   double2* A = lds + nxp;
   double2* B = lds + 2 * nxp;
-  double2* C = lds + nout * nxp;
   double2* twl = lds + (1 + nout) * mxp;
   double2* S = a.S + rd.sbase + (long long)k * nx;
   fft_stage_twiddles(twl, nx, a.tw);
@@ -151,12 +150,13 @@ __device__ __forceinline__ void fft_col_item(const FieldArgs& a, double2* lds) {
     double2 ph = make_double2(0.0, 0.0);
     if (m != 0 || k != 0) ph = make_double2(r.x / k2, r.y / k2);
     const int br = fft_slot<PAD>(bitrev(m, lognx));
-    if (want_E) {
+    if (a.want_phi) {
+      A[br] = ph;
+    } else {
       const double sx = sin2pi_frac(m, nx, twl, lognx) / rd.dx;
       A[br] = make_double2(sx * ph.y, -sx * ph.x);
       B[br] = make_double2(sy * ph.y, -sy * ph.x);
     }
-    if (a.want_phi) C[br] = ph;
   }
   __syncthreads();
   fft_lds_rows<PAD>(A, nout, nx, lognx, +1, twl, lognx);  // the outputs, consecutive rows
@@ -164,11 +164,12 @@ __device__ __forceinline__ void fft_col_item(const FieldArgs& a, double2* lds) {
   double2* Sy = a.Sy + rd.sbase + (long long)k * nx;
   for (int i = threadIdx.x; i < nx; i += PIC_WG) {
     const int q = fft_slot<PAD>(i);
-    if (want_E) {
+    if (a.want_phi) {
+      S[i] = A[q];
+    } else {
       Sx[i] = A[q];
       Sy[i] = B[q];
     }
-    if (a.want_phi) S[i] = C[q];
   }
 }
 
@@ -412,7 +413,7 @@ void launch_field(hipStream_t s, const FieldArgs& a, hipEvent_t* ev) {
   // data, then the n/2 twiddles of the transform length
   const size_t lrow = ((size_t)a.row_lds + a.max_ny / 2) * sizeof(double2);
   const size_t lcol = (size_t)(a.max_nx + a.max_nx / 8) * sizeof(double2) *
-                          (a.phi_only ? 2 : (a.want_phi ? 4 : 3)) +
+                          (a.want_phi ? 2 : 3) +
                       (size_t)(a.max_nx / 2) * sizeof(double2);
   // extra workgroups of the folded end-of-step work
   const int xrows = (a.fold_finish ? a.nruns : 0) + (a.fold_scan ? a.nfscan_items : 0);
@@ -422,13 +423,12 @@ void launch_field(hipStream_t s, const FieldArgs& a, hipEvent_t* ev) {
   if (ev) (void)hipEventRecord(ev[1], s);
   k_fft_cols<<<a.n_col_items + xcols, PIC_WG, lcol, s>>>(a);
   if (ev) (void)hipEventRecord(ev[2], s);
-  if (a.phi_only)
-    ;  // the caller wants no E
+  if (a.want_phi)
+    k_fft_field<float, 1><<<a.n_row_pair_items, PIC_WG, lrow, s>>>(a);
   else if (a.fp64)
     k_fft_field<double, 0><<<a.n_row_items + xfield, PIC_WG, lrow, s>>>(a);
   else
     k_fft_field<float, 0><<<a.n_row_items + xfield, PIC_WG, lrow, s>>>(a);
-  if (a.want_phi && a.phi) k_fft_field<float, 1><<<a.n_row_pair_items, PIC_WG, lrow, s>>>(a);
   if (ev) (void)hipEventRecord(ev[3], s);
 }
 

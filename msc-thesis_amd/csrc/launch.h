@@ -228,8 +228,7 @@ struct FieldArgs {
   double* diag;
   int nruns;
   int fp64;                          // particle precision (E type, rho words)
-  int want_phi;
-  int phi_only;                      // 1 (with want_phi): no Ex, Ey transforms, E untouched
+  int want_phi;                      // 1: phi instead of E (which stays as it was)
   int max_nx, max_ny;                // largest grid of the context (LDS sizing)
   int row_lds;                       // complex values per row-pass workgroup: the largest
                                      // max(fft_pp, fft_rf) * ny over the runs

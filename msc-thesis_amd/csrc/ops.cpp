@@ -271,7 +271,7 @@ int pic_op_poisson(const double* rho, double* phi, const pic_grid* g, void* stre
   a.S = S; a.phi = phi; a.tw = tw;
   a.row_pair_items = items; a.n_row_pair_items = nrp;
   a.col_items = items + nrp; a.n_col_items = ncl;
-  a.nruns = 1; a.fp64 = 0; a.want_phi = 1; a.phi_only = 1; a.max_nx = nx; a.max_ny = ny;
+  a.nruns = 1; a.fp64 = 0; a.want_phi = 1; a.max_nx = nx; a.max_ny = ny;
   a.row_lds = d.fft_pp * ny;
   a.rho_in = rho;
   launch_field(s, a, nullptr);
