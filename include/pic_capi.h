@@ -161,7 +161,8 @@ int pic_set_tuning(pic_ctx* ctx, int tile, int halo, int splits, int sort_every)
  * included); 0 when it runs as separate kernels (DSMC runs, sort_every < 2, or too many
  * tiles for the LDS). */
 int pic_sort_fused(pic_ctx* ctx, int* fused);
-/* Time candidate tilings for `trial_steps` each and keep the fastest (restores state). */
+/* Time the tuning in use and candidate tilings for `trial_steps` each and keep the fastest
+ * (restores state). */
 int pic_autotune(pic_ctx* ctx, int trial_steps, double* best_ms_per_step);
 /* Run nsteps eagerly with hipEvents around every kernel; out_ms[PIC_NSTAGES] receives the
  * mean duration per step of each stage (ms). */

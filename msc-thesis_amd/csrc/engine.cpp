@@ -239,6 +239,20 @@ int Ctx::rebalance_push_items() {
   return upload_runs();
 }
 
+// The tunings in force laid out on the device, and the particles sorted under them.
+int Ctx::retile() {
+  int rc = build_items();
+  if (rc) return rc;
+  bool any = false;
+  for (int r = 0; r < nruns; ++r) any |= has_particles[r] != 0;
+  if (any) {  // the offsets must describe the current order under the new tiles: sort now
+    launch_sort_stage();
+    steps_since_sort = 0;
+    PIC_HIP(hipStreamSynchronize(stream));
+  }
+  return rebalance_push_items();
+}
+
 Ctx::~Ctx() {
   if (device >= 0) (void)hipSetDevice(device);
   free_graphs();
@@ -1257,21 +1271,13 @@ int pic_set_tuning(pic_ctx* ctx, int tile, int halo, int splits, int sort_every)
     x.sort_every = was_every;
     return rc;
   }
-  if ((rc = x.build_items())) return rc;
-  // offsets must describe the current order for the new tiling: sort now
-  bool any = false;
-  for (int r = 0; r < x.nruns; ++r) any |= x.has_particles[r] != 0;
-  if (any) {
-    x.launch_sort_stage();
-    x.steps_since_sort = 0;
-    PIC_HIP(hipStreamSynchronize(x.stream));
-  }
-  return x.rebalance_push_items();
+  return x.retile();
 }
 
-// Project autotuner: times (tile, halo, sort cadence) candidates on the live state and
-// keeps the fastest.  The particle state, charge, counters and diagnostics are restored
-// afterwards, so tuning does not advance the simulation.
+// Project autotuner: times the tuning in force and (tile, halo, splits, sort cadence) candidates
+// on the live state and keeps the fastest; a tuning that no candidate beats stays.  The particle
+// state, charge, counters and diagnostics are restored afterwards, so tuning does not advance the
+// simulation.
 int pic_autotune(pic_ctx* ctx, int trial_steps, double* best_ms) {
   CTX_CHECK(ctx);
   Ctx& x = ctx->impl;
@@ -1326,56 +1332,61 @@ int pic_autotune(pic_ctx* ctx, int trial_steps, double* best_ms) {
   };
   int mn = PIC_FFT_MAX;
   for (auto& c : x.cfg) mn = std::min(mn, std::min(c.nx, c.ny));
-  double best = 1e30;
-  int bt = 0, bh = 0, bs = 0;
-  const int tiles[3] = {8, 16, 32}, halos[2] = {8, 16}, cad[5] = {1, 2, 4, 6, 8};
+  // the tuning set in x: one warm cycle (captures graphs), then the timed cycles
+  auto trial = [&](double* per) -> int {
+    int rc = restore();
+    if (rc) return rc;
+    if ((rc = x.retile())) return rc;
+    const int ml = x.macro_len();
+    if ((rc = x.step(ml))) return rc;
+    const int n = std::max(trial_steps / ml, 1) * ml;
+    PIC_HIP(hipEventRecord(x.ev[0], x.stream));
+    if ((rc = x.step(n))) return rc;
+    PIC_HIP(hipEventRecord(x.ev[1], x.stream));
+    PIC_HIP(hipEventSynchronize(x.ev[1]));
+    float ms = 0.f;
+    PIC_HIP(hipEventElapsedTime(&ms, x.ev[0], x.ev[1]));
+    *per = ms / n;
+    return PIC_OK;
+  };
+  // 64 where the windows fit (FP32) and the grid has two such tiles a side
+  const int tiles[4] = {8, 16, 32, 64}, halos[2] = {8, 16}, cad[5] = {1, 2, 4, 6, 8};
   // splits: 0 = sized by particles per tile (the only choice for ragged batches); the
   // larger counts fill the GPU on small grids (a 64^2 run has 16 tiles of 16^2 cells)
   const int splitc[6] = {0, 1, 2, 4, 8, 16};
-  int rc = PIC_OK;
-  int bsp = 0;
+  std::vector<Tuning> best_tune = orig;
+  int best_se = orig_se;
+  double best = 0.0;
+  int rc = trial(&best);
   for (int ti : tiles) {
-    if (ti > mn || ti > 64) continue;
+    if (ti > mn || (ti == 64 && mn < 128)) continue;
     for (int h : halos) {
       for (int se : cad)
       for (int sp : splitc) {
+        if (rc) break;
         if (x.any_dsmc && se != 1) continue;
         if (sp && x.nruns > 1) continue;
         // at least ~1k particles per workgroup for the larger split counts
         if (sp > 2 && (long long)x.cfg[0].capacity <
                           1024LL * sp * (x.cfg[0].nx / ti) * (x.cfg[0].ny / ti))
           continue;
-        rc = restore();
-        if (rc) break;
         x.sort_every = se;
         x.tune_runs(ti, h, sp, false);
-        if ((rc = x.build_items())) break;
-        x.launch_sort_stage();
-        x.steps_since_sort = 0;
-        if ((rc = x.rebalance_push_items())) break;
-        // one warm cycle (captures graphs), then the timed cycles
-        const int ml = x.macro_len();
-        if ((rc = x.step(ml))) break;
-        const int n = std::max(trial_steps / ml, 1) * ml;
-        PIC_HIP(hipEventRecord(x.ev[0], x.stream));
-        if ((rc = x.step(n))) break;
-        PIC_HIP(hipEventRecord(x.ev[1], x.stream));
-        PIC_HIP(hipEventSynchronize(x.ev[1]));
-        float ms = 0.f;
-        PIC_HIP(hipEventElapsedTime(&ms, x.ev[0], x.ev[1]));
-        const double per = ms / n;
-        if (per < best) { best = per; bt = ti; bh = h; bs = se; bsp = sp; }
+        if (x.check_tunings()) continue;  // its windows do not fit
+        double per = 0.0;
+        if ((rc = trial(&per))) break;
+        if (per < best) { best = per; best_tune = x.tune; best_se = se; }
       }
-      if (rc) break;
     }
-    if (rc) break;
   }
-  int rc2 = restore();
+  x.tune = rc ? orig : best_tune;
+  x.sort_every = rc ? orig_se : best_se;
+  const int rc2 = restore();
   release();
-  if (rc) { x.tune = orig; x.sort_every = orig_se; x.build_items(); return rc; }
-  if (rc2) return rc2;
+  const int rc3 = x.retile();
+  if (rc || rc2 || rc3) return rc ? rc : rc2 ? rc2 : rc3;
   if (best_ms) *best_ms = best;
-  return pic_set_tuning(ctx, bt, bh, bsp, bs);
+  return PIC_OK;
 }
 
 int pic_stage_times(pic_ctx* ctx, int nsteps, double* out) {

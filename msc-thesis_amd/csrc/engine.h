@@ -146,6 +146,7 @@ struct Ctx {
   std::vector<int> push_order() const;
   void push_items_for(int r, const int* toff_h);
   int rebalance_push_items();
+  int retile();
   int upload_runs();
   void free_graphs();
 
