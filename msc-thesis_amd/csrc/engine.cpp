@@ -76,19 +76,36 @@ double mcc_nu_max(const pic_config& c) {
   return best * 1.0001;  // margin so that no particle's total rate exceeds nu_max
 }
 
-// Steps a particle of unit speed takes to cross a cell, at most (thermal speeds and beams are
-// about 1 in the engine's units).
-static double cells_per_step(const pic_config& c) {
+// Cells a particle of unit speed crosses per step, at most.
+static double unit_drift(const pic_config& c) {
   return c.dt / std::min(c.lx / c.nx, c.ly / c.ny);
 }
 
-// Sort cadence when none is asked for: every 8 steps was the fastest or within 3 % of it on
-// grids of 32^2 to 512^2, FP32 and FP64, up to 4 cells of drift per step (512^2, 4.2 M FP32
-// particles at 2: 61 us per step against 64 at every 4); beyond that half of a cycle's drift
-// outgrows the halo.
-static int default_cadence(const std::vector<pic_config>& cfg) {
-  for (const pic_config& c : cfg)
-    if (cells_per_step(c) > 4.0) return 4;
+// Cells a thermal particle crosses per step, from the speeds a run holds: m8 are the means of
+// vx^8 and vy^8, whose eighth root is 105^(1/8) = 1.79 thermal speeds of a Maxwellian and the speed
+// itself of cold beams (which have no tail, so need that much less halo).  At least that of beams
+// of unit speed, the engine's units: cold particles do not stay cold.
+static double held_drift(const pic_config& c, const double m8[2]) {
+  const double q = std::pow(105.0, -0.125);
+  const double d = q * c.dt * std::max(std::pow(m8[0], 0.125) / (c.lx / c.nx),
+                                       std::pow(m8[1], 0.125) / (c.ly / c.ny));
+  return std::max(q * unit_drift(c), d);
+}
+
+// Steps from the positions that a sort keys on to the last deposit under it: half a cycle either
+// side where the keys are led (sort_lead), the whole cycle with MCC.
+static double key_reach(const pic_config& c, int cadence) {
+  return (c.collide == PIC_COLLIDE_MCC ? cadence : 0.5 * cadence) + 1.0;
+}
+
+// Sort cadence when none is asked for: every 8 steps while the thermal drift from the keys is 13
+// cells or less (2.6 per step, with MCC 1.4), else every 4.  Steps sorted every 8 / 4 (us), 512^2
+// FP32 with 16 particles per cell: thermal speeds of 2 cells per step 60 / 64, 4 84 / 66, 6 137 / 73,
+// beams of 4 60 / 63, 6 85 / 64, 10 184 / 81; 256^2 FP64: thermal 2 42 / 44, 3 50 / 45, beams of 3
+// 40 / 43, 5 51 / 44, 10 142 / 65; 256^2 with MCC, thermal 1 68 / 70, 1.5 97 / 71, 2.5 194 / 101.
+int Ctx::default_cadence() const {
+  for (int r = 0; r < nruns; ++r)
+    if (!(drift[r] * key_reach(cfg[r], 8) <= 13.0)) return 4;
   return 8;
 }
 
@@ -109,14 +126,14 @@ static const int PUSH_LDS_MAX = 160 * 1024 - 256;
 //           (1024^2, 16 M particles: 375 us per step with 16, 259 with 32, 217 with 64)
 //           A halo the caller gives may not fit such tiles (1024^2 FP32, halo 24: 204 KB with 64,
 //           68 KB with 16): they are halved to 16 cells until the window fits
-//   halo    16 where half a cycle's drift of 2.5 thermal speeds passes 8 cells, else 8
+//   halo    16 where the drift of 2.5 thermal speeds from the sort's keys passes 8 cells, else 8
 //   splits  as many as make up the items, of 256 particles at least and 65,536 at most
 static Tuning default_tuning(const pic_config& c, int tile, int halo, int splits, int cadence,
-                             double items) {
+                             double items, double drift) {
   Tuning t;
   const int m = std::min(c.nx, c.ny);
   const long long n = std::max<long long>(c.capacity, 1);
-  if (!halo) halo = 2.5 * cells_per_step(c) * (0.5 * cadence + 1.0) > 8.0 ? 16 : 8;
+  if (!halo) halo = 2.5 * drift * key_reach(c, cadence) <= 8.0 ? 8 : 16;
   // the window (tile + 2 halo + 1 nodes) must not wrap onto itself: win <= min(nx, ny)
   auto halo_of = [&](int side) { return std::min(halo, std::max(0, (m - side - 1) / 2)); };
   if (tile) {
@@ -150,19 +167,46 @@ static Tuning default_tuning(const pic_config& c, int tile, int halo, int splits
   return t;
 }
 
-// Tunings of all runs (values of 0: from_config takes the run's configured ones, then the
-// defaults).  A launch wants one workgroup per CU, two where two fit (FP32) and get 2048
-// particles each; a run of a batch has its share of them by particles.
-void Ctx::tune_runs(int tile, int halo, int splits, bool from_config) {
+// Tunings of all runs by what is asked for.  A launch wants one workgroup per CU, two where two
+// fit (FP32) and get 2048 particles each; a run of a batch has its share of them by particles.
+void Ctx::tune_runs() {
   double total = 0;
   for (const pic_config& c : cfg) total += (double)std::max<int64_t>(c.capacity, 1);
   const double items = !fp64 && total >= 512.0 * 2048.0 ? 512.0 : 256.0;
+  sort_every = ask.sort_every ? ask.sort_every : default_cadence();
   tune.resize(nruns);
   for (int r = 0; r < nruns; ++r)
-    tune[r] = default_tuning(cfg[r], from_config ? cfg[r].tile : tile,
-                             from_config ? cfg[r].halo : halo,
-                             from_config ? cfg[r].splits : splits, any_dsmc ? 1 : sort_every,
-                             items * std::max<int64_t>(cfg[r].capacity, 1) / total);
+    tune[r] = default_tuning(cfg[r], ask.from_config ? cfg[r].tile : ask.tile,
+                             ask.from_config ? cfg[r].halo : ask.halo,
+                             ask.from_config ? cfg[r].splits : ask.splits,
+                             any_dsmc ? 1 : sort_every,
+                             items * std::max<int64_t>(cfg[r].capacity, 1) / total, drift[r]);
+}
+
+// A run has new particles: the defaults that go by their speeds follow them.  Lays the tunings
+// out again when one of them changes (the caller sorts).
+int Ctx::retune_for_speeds(int run, int64_t n) {
+  if (ask.sort_every && (ask.from_config ? cfg[run].halo : ask.halo)) return PIC_OK;
+  if (fp64) launch_speed8<double>(stream, bufs<double>(cur), rd[run].pbase, n, speed_part);
+  else launch_speed8<float>(stream, bufs<float>(cur), rd[run].pbase, n, speed_part);
+  PIC_HIP(hipGetLastError());
+  PIC_HIP(hipStreamSynchronize(stream));
+  std::vector<double> h(2 * SPEED_BLOCKS);
+  PIC_HIP(hipMemcpy(h.data(), speed_part, sizeof(double) * h.size(), hipMemcpyDeviceToHost));
+  double m8[2] = {0.0, 0.0};
+  for (int b = 0; b < 2 * SPEED_BLOCKS; ++b) m8[b & 1] += h[b] / (double)n;
+  const std::vector<Tuning> was = tune;
+  const int was_every = sort_every;
+  drift[run] = held_drift(cfg[run], m8);
+  tune_runs();
+  bool same = sort_every == was_every;
+  for (int r = 0; r < nruns; ++r) same = same && tune[r].same_layout(was[r]);
+  if (same || check_tunings()) {
+    tune = was;
+    sort_every = was_every;
+    return PIC_OK;
+  }
+  return build_items();
 }
 
 // Items (run, tile x, tile y, split | splits << 16) of run r: t.splits per tile, or with
@@ -266,7 +310,7 @@ Ctx::~Ctx() {
   F(d_pitems); F(d_citems); F(d_rowpair); F(d_cols); F(d_rows); F(d_push);
   F(d_tscan_items);
   F(partials_push); F(partials_rows); F(diag);
-  F(d_coll_counts); F(birth_count); F(birth_parent); F(birth_buf); F(gmax); F(flag);
+  F(d_coll_counts); F(birth_count); F(birth_parent); F(birth_buf); F(gmax); F(flag); F(speed_part);
   F(coll_list); F(coll_partials); F(dsmc_slots);
   for (auto& e : ev) if (e) (void)hipEventDestroy(e);
   if (stream) (void)hipStreamDestroy(stream);
@@ -504,6 +548,7 @@ int Ctx::alloc() {
   PIC_HIP(dalloc(&diag, (size_t)nruns * PIC_DIAG_CAP * 8));
   PIC_HIP(dalloc(&d_coll_counts, 4 * nruns));
   PIC_HIP(dalloc(&flag, 1));
+  PIC_HIP(dalloc(&speed_part, 2 * SPEED_BLOCKS));
   if (any_mcc) {
     long long maxcap = 0;
     for (auto& c : cfg) maxcap = std::max<long long>(maxcap, c.capacity);
@@ -534,7 +579,9 @@ int Ctx::alloc() {
   PIC_HIP(hipMemset(diag, 0, sizeof(double) * (size_t)nruns * PIC_DIAG_CAP * 8));
   PIC_HIP(hipMemset(d_coll_counts, 0, sizeof(long long) * 4 * nruns));
   PIC_HIP(hipMemset(E, 0, rs * 2 * esum));
-  tune_runs(0, 0, 0, true);
+  drift.resize(nruns);
+  for (int r = 0; r < nruns; ++r) drift[r] = unit_drift(cfg[r]);
+  tune_runs();
   int rc = build_items();
   if (rc) return rc;
   allocated = true;
@@ -868,9 +915,7 @@ static int create_impl(const pic_config* cfgs, int nruns, pic_ctx** out) {
   x.cfg.assign(cfgs, cfgs + nruns);
   x.rd.resize(nruns);
   x.has_particles.assign(nruns, 0);
-  int se = 0;
-  for (auto& cc : x.cfg) se = std::max(se, cc.sort_every);
-  x.sort_every = se ? se : default_cadence(x.cfg);
+  for (auto& cc : x.cfg) x.ask.sort_every = std::max(x.ask.sort_every, cc.sort_every);
   if (nruns > 1 || cfgs[0].capacity > 0) {
     int rc = x.alloc();
     if (rc) return rc;
@@ -958,6 +1003,7 @@ int set_particles_impl(pic_ctx* ctx, int run, const void* px_, const void* py_,
     s.next_id = restore->next_id;
   }
   PIC_HIP(hipMemcpy(x.d_st + run, &s, sizeof(s), hipMemcpyHostToDevice));
+  if ((rc = x.retune_for_speeds(run, n))) return rc;
   const long long G = (long long)d.nx * d.ny;
   for (int p = 0; p < 2; ++p) {
     launch_fill_u64(x.stream, x.rho + p * x.gsum + d.gbase, G);
@@ -1262,12 +1308,14 @@ int pic_set_tuning(pic_ctx* ctx, int tile, int halo, int splits, int sort_every)
   }
   PIC_HIP(hipStreamSynchronize(x.stream));
   const std::vector<Tuning> was = x.tune;
+  const TuningAsk was_ask = x.ask;
   const int was_every = x.sort_every;
-  if (sort_every) x.sort_every = sort_every;
-  x.tune_runs(tile, halo, splits, false);
+  x.ask = {tile, halo, splits, sort_every ? sort_every : was_ask.sort_every, false};
+  x.tune_runs();
   int rc = x.check_tunings();
   if (rc) {  // refused: the tuning in force stays
     x.tune = was;
+    x.ask = was_ask;
     x.sort_every = was_every;
     return rc;
   }
@@ -1313,6 +1361,7 @@ int pic_autotune(pic_ctx* ctx, int trial_steps, double* best_ms) {
     return fail(PIC_ERR_OOM, "autotune snapshot allocation failed");
   }
   const std::vector<Tuning> orig = x.tune;
+  const TuningAsk orig_ask = x.ask;
   const int orig_se = x.sort_every;
   auto restore = [&]() -> int {
     const int c = x.cur;
@@ -1355,6 +1404,7 @@ int pic_autotune(pic_ctx* ctx, int trial_steps, double* best_ms) {
   // larger counts fill the GPU on small grids (a 64^2 run has 16 tiles of 16^2 cells)
   const int splitc[6] = {0, 1, 2, 4, 8, 16};
   std::vector<Tuning> best_tune = orig;
+  TuningAsk best_ask = orig_ask;
   int best_se = orig_se;
   double best = 0.0;
   int rc = trial(&best);
@@ -1370,16 +1420,17 @@ int pic_autotune(pic_ctx* ctx, int trial_steps, double* best_ms) {
         if (sp > 2 && (long long)x.cfg[0].capacity <
                           1024LL * sp * (x.cfg[0].nx / ti) * (x.cfg[0].ny / ti))
           continue;
-        x.sort_every = se;
-        x.tune_runs(ti, h, sp, false);
+        x.ask = {ti, h, sp, se, false};
+        x.tune_runs();
         if (x.check_tunings()) continue;  // its windows do not fit
         double per = 0.0;
         if ((rc = trial(&per))) break;
-        if (per < best) { best = per; best_tune = x.tune; best_se = se; }
+        if (per < best) { best = per; best_tune = x.tune; best_ask = x.ask; best_se = se; }
       }
     }
   }
   x.tune = rc ? orig : best_tune;
+  x.ask = rc ? orig_ask : best_ask;
   x.sort_every = rc ? orig_se : best_se;
   const int rc2 = restore();
   release();

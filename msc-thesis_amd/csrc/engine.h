@@ -68,6 +68,17 @@ struct Tuning {
   // push items of equal particles whatever the tiles, 0: not; and as many as there would be (DSMC
   // runs asked for splits 0, by the particles they hold per tile)
   int shares = 0, max_shares = 0;
+  bool same_layout(const Tuning& o) const {
+    return tile == o.tile && halo == o.halo && splits == o.splits && per_tile == o.per_tile &&
+           max_shares == o.max_shares;
+  }
+};
+
+// What the caller asks of the tunings; 0: the default.  from_config: tile, halo and splits are the
+// runs' configured ones (a run each) instead of these.
+struct TuningAsk {
+  int tile = 0, halo = 0, splits = 0, sort_every = 0;
+  bool from_config = true;
 };
 
 struct Ctx {
@@ -79,6 +90,8 @@ struct Ctx {
   std::vector<pic_config> cfg;
   std::vector<RunDesc> rd;
   std::vector<Tuning> tune;
+  TuningAsk ask;
+  std::vector<double> drift;  // cells that a run's thermal particles cross per step
   std::vector<int> has_particles;
   std::vector<double> numax_dt;     // MCC nu_max * dt_phys * dt per run
   int sort_every = 4;
@@ -129,6 +142,7 @@ struct Ctx {
   unsigned long long* dsmc_slots = nullptr;
   int* birth_parent = nullptr;
   float* birth_buf = nullptr;
+  double* speed_part = nullptr;        // [2 * SPEED_BLOCKS]
   float* gmax = nullptr;               // per cell (ctotal)
   // output scratch
   int* flag = nullptr;
@@ -140,7 +154,9 @@ struct Ctx {
 
   ~Ctx();
   int alloc();
-  void tune_runs(int tile, int halo, int splits, bool from_config);
+  int default_cadence() const;
+  void tune_runs();
+  int retune_for_speeds(int run, int64_t n);
   int check_tunings() const;
   int build_items();
   std::vector<int> push_order() const;

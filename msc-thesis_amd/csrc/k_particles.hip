@@ -621,6 +621,26 @@ __global__ void k_reduce_sum(const double* parts, int n, double* out) {
   if (threadIdx.x == 0) *out = v;
 }
 
+template <typename R>
+__global__ __launch_bounds__(PIC_WG) void k_speed8(const R* __restrict__ vx,
+                                                   const R* __restrict__ vy, int64_t n,
+                                                   double* __restrict__ part) {
+  __shared__ double red[4];
+  double sx = 0.0, sy = 0.0;
+  for (int64_t p = blockIdx.x * (int64_t)PIC_WG + threadIdx.x; p < n;
+       p += (int64_t)SPEED_BLOCKS * PIC_WG) {
+    const double a = (double)vx[p] * (double)vx[p], b = (double)vy[p] * (double)vy[p];
+    sx += (a * a) * (a * a);
+    sy += (b * b) * (b * b);
+  }
+  sx = block_sum(sx, red);
+  sy = block_sum(sy, red);
+  if (threadIdx.x == 0) {
+    part[2 * blockIdx.x] = sx;
+    part[2 * blockIdx.x + 1] = sy;
+  }
+}
+
 inline int grid_for(long long n) {
   long long b = (n + PIC_WG - 1) / PIC_WG;
   return (int)(b < 1 ? 1 : (b > 8192 ? 8192 : b));
@@ -645,6 +665,11 @@ void launch_op_fixed_to_double(hipStream_t s, const unsigned long long* hi,
 }
 void launch_reduce_sum(hipStream_t s, const double* parts, int n, double* out) {
   k_reduce_sum<<<1, PIC_WG, 0, s>>>(parts, n, out);
+}
+
+template <typename R>
+void launch_speed8(hipStream_t s, PartBufs<R> p, long long base, int64_t n, double* part) {
+  k_speed8<R><<<SPEED_BLOCKS, PIC_WG, 0, s>>>(p.vx + base, p.vy + base, n, part);
 }
 
 template <typename R>
@@ -825,6 +850,7 @@ void launch_op_gather_push(hipStream_t s, const GatherPushPlan& p, R* x, R* y, R
 }
 
 #define PIC_INST(R)                                                                          \
+  template void launch_speed8<R>(hipStream_t, PartBufs<R>, long long, int64_t, double*);     \
   template void launch_tile_sort<R>(hipStream_t, const RunDesc*, RunState*, int, PartBufs<R>,\
                                     PartBufs<R>, SortBufs, const int2*, int, int);            \
   template void launch_push<R>(hipStream_t, const PushArgs<R>&);                            \
