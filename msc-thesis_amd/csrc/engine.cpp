@@ -606,6 +606,17 @@ FieldArgs Ctx::field_args(int want_phi) const {
   return a;
 }
 
+// Cell order matters to the push from about 16 particles per cell on, of those held (steps of
+// 256^2 with 32 per cell 143 -> 132 us, 512^2 with 12 188 -> 182, but 64^2 with 2 or 6 55 -> 56,
+// 58 -> 59); shares need it.
+bool Ctx::by_cell() const {
+  for (const Tuning& t : tune)
+    if (t.shares) return true;
+  long long n = 0;
+  for (int64_t h : held) n += h;
+  return any_dsmc && n >= 16 * gsum;
+}
+
 template <typename R>
 PushArgs<R> Ctx::push_args(int mode, int sort_mode) const {
   PushArgs<R> a;
@@ -619,11 +630,7 @@ PushArgs<R> Ctx::push_args(int mode, int sort_mode) const {
   a.items = d_push; a.nitems = (int)push_items.size();
   a.nruns = nruns;
   a.partials = partials_push;
-  // cell order matters to the push from about 16 particles per cell on (steps of 256^2 with 32
-  // per cell 143 -> 132 us, 512^2 with 12 188 -> 182, but 64^2 with 2 or 6 55 -> 56, 58 -> 59)
-  bool shares = false;
-  for (const Tuning& t : tune) shares = shares || t.shares;
-  a.by_cell = shares || (any_dsmc && ptotal >= 16 * gsum);
+  a.by_cell = by_cell();
   a.mode = mode; a.lds_bytes = lds_push;
   a.sort_mode = fused ? sort_mode : 0;
   a.ftable = sb.ftable;
@@ -915,6 +922,7 @@ static int create_impl(const pic_config* cfgs, int nruns, pic_ctx** out) {
   x.cfg.assign(cfgs, cfgs + nruns);
   x.rd.resize(nruns);
   x.has_particles.assign(nruns, 0);
+  x.held.assign(nruns, 0);
   for (auto& cc : x.cfg) x.ask.sort_every = std::max(x.ask.sort_every, cc.sort_every);
   if (nruns > 1 || cfgs[0].capacity > 0) {
     int rc = x.alloc();
@@ -1024,7 +1032,10 @@ int set_particles_impl(pic_ctx* ctx, int run, const void* px_, const void* py_,
   x.launch_sort_stage();
   x.steps_since_sort = 0;
   x.has_particles[run] = 1;
+  const bool was_by_cell = x.by_cell();
+  x.held[run] = n;
   if ((rc = x.rebalance_push_items())) return rc;
+  if (x.by_cell() != was_by_cell) x.free_graphs();  // they hold the other form of the push
   // deposit the initial charge of this run only
   if (x.fp64) {
     PushArgs<double> a = x.push_args<double>(1);

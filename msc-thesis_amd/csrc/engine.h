@@ -93,6 +93,7 @@ struct Ctx {
   TuningAsk ask;
   std::vector<double> drift;  // cells that a run's thermal particles cross per step
   std::vector<int> has_particles;
+  std::vector<int64_t> held;           // particles set per run (DSMC keeps their number)
   std::vector<double> numax_dt;     // MCC nu_max * dt_phys * dt per run
   int sort_every = 4;
   int steps_since_sort = 0;
@@ -173,6 +174,7 @@ struct Ctx {
     return b;
   }
   FieldArgs field_args(int want_phi) const;
+  bool by_cell() const;
   template <typename R> PushArgs<R> push_args(int mode, int sort_mode = 0) const;
 
   // launches (no synchronisation)
