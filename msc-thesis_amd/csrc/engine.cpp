@@ -1078,6 +1078,11 @@ static int read_state(Ctx& x, int run, RunState* s) {
 // (state read, field, output), direct against records, FP32 (us): 59 / 65 at 10,000 particles,
 // 66 / 63 at 100,000, 104 / 76 at 1,000,001, 247 / 128 at 4,000,001, 1094 / 555 at 16,777,216.
 static const int OUT_DIRECT_MAX = 1 << 16;
+// Bytes up to which an output to the host is one copy.  Whole calls, the four arrays in one copy and
+// each by itself (us): FP32 65 / 100 at 1000 particles, 99 / 107 at 32,768; FP64 65 / 95 at 1000, 102 /
+// 108 at 20,000, 173 / 132 at 32,768.  (As records, converted by fours: FP32 2500 against 1830 at
+// 1,000,001, FP64 24,500 against 7450 at 4,000,001.)
+static const size_t OUT_ONCE_BYTES = 512 << 10;
 
 // Records of an output live in the run's slice of the particle buffer that is not in use (the
 // next sort overwrites it).
@@ -1114,19 +1119,35 @@ static int get_particles_t(Ctx& x, int run, void* ox, void* oy, void* ovx, void*
       return fail(PIC_ERR_HIP, std::string("get_particles: ") + hipGetErrorString(e));
     return PIC_OK;
   }
-  launch_out_particles<R>(x.stream, x.d_runs, x.d_st, run, np, p, E, rec, nullptr, nullptr,
-                          nullptr, nullptr);
+  // Host arrays: bound by the copies.  All four in one up to OUT_ONCE_BYTES; above it each by
+  // itself, FP64 straight into the caller's, FP32 in pieces that stay in cache until they are
+  // converted.
+  void* outs[4] = {ox, oy, ovx, ovy};
+  R* src[4];
+  for (int k = 0; k < 4; ++k) src[k] = outs[k] ? rec + (size_t)k * np : nullptr;
+  launch_out_particles<R>(x.stream, x.d_runs, x.d_st, run, np, p, E, nullptr, src[0], src[1],
+                          src[2], src[3]);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(x.stream);
-  double* outs[4] = {(double*)ox, (double*)oy, (double*)ovx, (double*)ovy};
-  const int chunk = std::min(np, 1 << 20);
-  std::vector<R> h(4 * (size_t)chunk);
-  for (int b = 0; b < np && e == hipSuccess; b += chunk) {
-    const int m = std::min(chunk, np - b);
-    e = hipMemcpy(h.data(), rec + 4 * (size_t)b, 4 * sizeof(R) * m, hipMemcpyDeviceToHost);
-    for (int k = 0; k < 4; ++k)
-      if (outs[k])
-        for (int i = 0; i < m; ++i) outs[k][b + i] = (double)h[4 * (size_t)i + k];
+  const bool once = 4 * sizeof(R) * np <= OUT_ONCE_BYTES;
+  const int piece = std::min(np, 1 << 20);
+  std::vector<R> h(once ? 4 * (size_t)np : sizeof(R) == 4 ? (size_t)piece : 0);
+  if (once && e == hipSuccess)
+    e = hipMemcpy(h.data(), rec, 4 * sizeof(R) * np, hipMemcpyDeviceToHost);
+  for (int k = 0; k < 4 && e == hipSuccess; ++k) {
+    double* o = (double*)outs[k];
+    if (!o) continue;
+    if (once) {
+      for (int i = 0; i < np; ++i) o[i] = (double)h[(size_t)k * np + i];
+    } else if (sizeof(R) == 8) {
+      e = hipMemcpy(o, src[k], sizeof(R) * np, hipMemcpyDeviceToHost);
+    } else {
+      for (int b = 0; b < np && e == hipSuccess; b += piece) {
+        const int m = std::min(piece, np - b);
+        e = hipMemcpy(h.data(), src[k] + b, sizeof(R) * m, hipMemcpyDeviceToHost);
+        for (int i = 0; i < m; ++i) o[b + i] = (double)h[i];
+      }
+    }
   }
   if (e != hipSuccess) return fail(PIC_ERR_HIP, std::string("get_particles: ") + hipGetErrorString(e));
   return PIC_OK;
