@@ -448,14 +448,57 @@ __global__ __launch_bounds__(PIC_WG) void k_op_cell_keys(const R* __restrict__ x
 //   GP_LDS     the padded pairs of a small grid, in every workgroup's LDS
 // Random positions are bound by the vector L1: 64 lanes of a load meet up to 64 lines, so the
 // number of load instructions sets the time (launch_op_gather_push has the measurements).
-enum { GP_NODES, GP_PACKED, GP_ROWS, GP_LDS };
+//   GP_AUTO    nodes, packed or rows by the word that k_op_pack_E leaves
+enum { GP_NODES, GP_PACKED, GP_ROWS, GP_LDS, GP_AUTO };
 
-// rows: the interleaved form, nx rows of 2 * (ny + 1) entries
+// Form for the order that the positions are in, judged by 64 pairs of neighbours spread over the
+// arrays: `ordered` when half of the pairs lie within a row (FP64: four) and 8 columns of each
+// other (a wave's gathers meet a few lines), `local` when within a sixteenth of the grid either
+// way, else `other`.
+// For one whole wave; every workgroup finds the same, as it reads the same particles.
+template <typename R>
+__device__ __forceinline__ int gp_form(const R* __restrict__ x, const R* __restrict__ y, int64_t n,
+                                       const Geo<R>& g, int ordered, int local, int other) {
+  const int64_t p = (n - 2) * (threadIdx.x & 63) / 63;
+  int cx, cy, dx, dy;
+  R f;
+  locate_w(x[p], g.idx, g.nx, cx, f);
+  locate_w(y[p], g.idy, g.ny, cy, f);
+  locate_w(x[p + 1], g.idx, g.nx, dx, f);
+  locate_w(y[p + 1], g.idy, g.ny, dy, f);
+  auto half_within = [&](int rows, int cols) {
+    return __popcll(__ballot(pwrap(dx - cx + rows, g.nx) <= 2 * rows &&
+                             pwrap(dy - cy + cols, g.ny) <= 2 * cols)) >= 32;
+  };
+  return half_within(sizeof(R) == 8 ? 4 : 1, 8) ? ordered : half_within(g.nx >> 4, g.ny >> 4) ? local : other;
+}
+
+// form: GP_PACKED or GP_ROWS (the interleaved form, nx rows of 2 * (ny + 1) entries).  choice (or
+// NULL): the form is gp_form's, with `form` as its other, and is written there; GP_NODES packs
+// nothing.
 template <typename R>
 __global__ __launch_bounds__(PIC_WG) void k_op_pack_E(const double* __restrict__ ex,
-                                                      const double* __restrict__ ey, int nx,
-                                                      int ny, int rows,
+                                                      const double* __restrict__ ey,
+                                                      const R* __restrict__ x,
+                                                      const R* __restrict__ y, int64_t n,
+                                                      int ordered, int local, int form,
+                                                      int* choice, int nx, int ny, double lx,
+                                                      double ly,
                                                       typename EWin<R>::R2* __restrict__ E) {
+  if (choice) {
+    __shared__ int chosen;
+    if (threadIdx.x < 64) {
+      const int c = gp_form<R>(x, y, n, make_geo<R>(nx, ny, lx, ly), ordered, local, form);
+      if (threadIdx.x == 0) {
+        chosen = c;
+        if (blockIdx.x == 0) *choice = c;
+      }
+    }
+    __syncthreads();
+    form = chosen;
+    if (form == GP_NODES) return;
+  }
+  const bool rows = form == GP_ROWS;
   const int lny = __builtin_ctz((unsigned)ny);
   const int G = nx * ny;
   for (int q = blockIdx.x * PIC_WG + threadIdx.x; q < G; q += gridDim.x * PIC_WG) {
@@ -482,37 +525,17 @@ __global__ __launch_bounds__(PIC_WG) void k_op_pack_E(const double* __restrict__
   }
 }
 
-template <typename R, int SRC>
-__global__ __launch_bounds__(SRC == GP_LDS ? GP_LDS_NT : PIC_WG) void k_op_gather_push(
-    R* x, R* y, R* vx, R* vy, int64_t n, const double* __restrict__ ex,
-    const double* __restrict__ ey, const typename EWin<R>::R2* __restrict__ E, int nx, int ny,
-    double lx, double ly, double dt, double qm, double c, double* partials) {
+// The pushes of a workgroup of NT threads, U particles per thread at a time; returns the thread's
+// share of sum |v_n|^2.  el: the padded field in LDS (GP_LDS).
+template <typename R, int SRC, int NT, int U>
+__device__ __forceinline__ double gp_span(R* x, R* y, R* vx, R* vy, int64_t n,
+                                          const double* __restrict__ ex,
+                                          const double* __restrict__ ey,
+                                          const typename EWin<R>::R2* __restrict__ E,
+                                          const typename EWin<R>::R2* el, const Geo<R>& g, R hk,
+                                          R dtr, double skc) {
   typedef typename EWin<R>::R2 R2;
-  constexpr int NT = SRC == GP_LDS ? GP_LDS_NT : PIC_WG, U = SRC == GP_NODES ? 1 : 4;
-  extern __shared__ double2 gp_lds[];
-  __shared__ double red[NT / 64];
-  const Geo<R> g = make_geo<R>(nx, ny, lx, ly);
-  const R hk = (R)(c * dt * qm), dtr = (R)dt;
-  const double skc = (c - 0.5) * dt * qm;
-  const int ny1 = ny + 1;
-  R2* el = reinterpret_cast<R2*>(gp_lds);
-  if (SRC == GP_LDS) {
-    const int lny = __builtin_ctz((unsigned)ny);
-#pragma unroll 4
-    for (int q = threadIdx.x; q < nx * ny; q += NT) {
-      const int i = q >> lny, j = q & (ny - 1);
-      R2 v;
-      v.x = (R)ex[q];
-      v.y = (R)ey[q];
-      el[i * ny1 + j] = v;
-      if (j == 0) el[i * ny1 + ny] = v;
-      if (i == 0) {
-        el[nx * ny1 + j] = v;
-        if (j == 0) el[nx * ny1 + ny] = v;
-      }
-    }
-    __syncthreads();
-  }
+  const int nx = g.nx, ny = g.ny, ny1 = ny + 1;
   double ke = 0;
   const int64_t stride = (int64_t)gridDim.x * NT;
   for (int64_t p0 = blockIdx.x * (int64_t)NT + threadIdx.x; p0 < n; p0 += U * stride) {
@@ -588,6 +611,55 @@ __global__ __launch_bounds__(SRC == GP_LDS ? GP_LDS_NT : PIC_WG) void k_op_gathe
       }
     }
   }
+  return ke;
+}
+
+template <typename R, int SRC>
+__global__ __launch_bounds__(SRC == GP_LDS ? GP_LDS_NT : PIC_WG) void k_op_gather_push(
+    R* x, R* y, R* vx, R* vy, int64_t n, const double* __restrict__ ex,
+    const double* __restrict__ ey, const typename EWin<R>::R2* __restrict__ E,
+    const int* __restrict__ choice, int nx, int ny, double lx, double ly, double dt, double qm,
+    double c, double* partials) {
+  typedef typename EWin<R>::R2 R2;
+  constexpr int NT = SRC == GP_LDS ? GP_LDS_NT : PIC_WG;
+  extern __shared__ double2 gp_lds[];
+  __shared__ double red[NT / 64];
+  const Geo<R> g = make_geo<R>(nx, ny, lx, ly);
+  const R hk = (R)(c * dt * qm), dtr = (R)dt;
+  const double skc = (c - 0.5) * dt * qm;
+  R2* el = reinterpret_cast<R2*>(gp_lds);
+  if (SRC == GP_LDS) {
+    const int lny = __builtin_ctz((unsigned)ny), ny1 = ny + 1;
+#pragma unroll 4
+    for (int q = threadIdx.x; q < nx * ny; q += NT) {
+      const int i = q >> lny, j = q & (ny - 1);
+      R2 v;
+      v.x = (R)ex[q];
+      v.y = (R)ey[q];
+      el[i * ny1 + j] = v;
+      if (j == 0) el[i * ny1 + ny] = v;
+      if (i == 0) {
+        el[nx * ny1 + j] = v;
+        if (j == 0) el[nx * ny1 + ny] = v;
+      }
+    }
+    __syncthreads();
+  }
+  const int form = SRC == GP_AUTO ? *choice : SRC;  // uniform
+  auto span = [&](auto src, auto u) {
+    return gp_span<R, decltype(src)::value, NT, decltype(u)::value>(x, y, vx, vy, n, ex, ey, E, el,
+                                                                   g, hk, dtr, skc);
+  };
+  using std::integral_constant;
+  // the node arrays beside the pairs: as many at a time as the pairs' registers hold
+  double ke;
+  if (SRC == GP_AUTO && form == GP_NODES)
+    ke = span(integral_constant<int, GP_NODES>(), integral_constant<int, sizeof(R) == 4 ? 2 : 4>());
+  else if (SRC == GP_AUTO && form == GP_PACKED)
+    ke = span(integral_constant<int, GP_PACKED>(), integral_constant<int, 4>());
+  else
+    ke = span(integral_constant<int, SRC == GP_AUTO ? GP_ROWS : SRC>(),
+              integral_constant<int, SRC == GP_NODES ? 1 : 4>());
   if (!partials) return;  // uniform
   ke = wave_sum(ke);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ke;
@@ -784,7 +856,8 @@ void launch_op_cell_keys(hipStream_t s, const R* x, const R* y, int64_t n, int n
 //   (32^2: 20 / 22 -> 20 / 21 at 262,144)
 //   packed, 512^2: 8,000,009 particles 281 / 319 -> 112 / 217 (with random velocities 316 ->
 //   148; the kernel 269 -> 97 + 5 to pack, FP32), 1,048,576: 56 / 60 -> 35 / 48, 524,288:
-//   36 / 38 -> 30 / 36, 262,144: 26 -> 27; 1024^2 at 524,288: 51 / 53 -> 40 / 47
+//   36 / 38 -> 30 / 36, 262,144: 26 -> 27; 1024^2 at 524,288: 51 / 53 -> 40 / 47, 2048^2 at
+//   1,048,577 100 / 106 -> 75 / 91, at 524,289 58 / 63 -> 54 / 65 (66 / 81 from HBM)
 // Interleaved rows instead of packed: where they take little of an XCD's 4 MiB L2, where the
 // packed pairs do not fit it either, or where the state is a large part of the last-level
 // cache, whose lines then come from HBM anyway; enough particles to pay for packing twice the
@@ -798,12 +871,24 @@ void launch_op_cell_keys(hipStream_t s, const R* x, const R* y, int64_t n, int n
 //         256^2: 8,000,009 146 / 241 -> 163 / 215, but 4,194,304 88 / 133 -> 100 / 132
 //         1024^2: 8,000,009 353 / 353 -> 275 / 284, 1,048,576 68 / 73 -> 67 / 77
 //         2048^2: 4,194,304 243 / 260 -> 198 / 230, but 1,048,576 88 / 106 -> 84 / 119
+// In a step of the operators (deposit, Poisson, E, push: the deposit follows the rows' stores past
+// the caches) the large state's line costs 1.6 % at 8,000,009 FP32 on 512^2 (235 -> 239 us packed ->
+// rows), gives 11 % at 20,000,003 (567 -> 510), 4 % at 8,000,009 FP64 on 256^2 (379 -> 362).
+// Grids whose pairs outgrow the L2, up to 8 particles per node: random positions want the pairs,
+// but those that lie in cell order meet few lines of the node arrays and pay for packing, and nearby
+// ones meet few lines of the packed form.  The caller's order is not known here, so the packing
+// looks (gp_form: 2 to 4 us).  Sorted / within 10 cells of it / random (us):
+//   FP64 2048^2, 4,194,307: node arrays 70 / 112 / 353, packed 96 / 121 / 241, rows 134 / 165 / 201,
+//   chosen 77 / 125 / 209; 1024^2, 1,048,579: 35 / 46 / 88, 40 / 50 / 69, 51 / 61 / 69, 39 / 53 / 71
+//   FP32 2048^2, 4,194,307: 52 / 106 / 336, 64 / 81 / 198, 72 / 93 / 144, 59 / 82 / 147; 1024^2,
+//   4,194,307: 47 / 88 / 272, 50 / 64 / 135, 55 / 70 / 118, 53 / 72 / 117
+// On smaller grids looking costs what it gives (FP64 512^2, 4,194,307, sorted 80 either way).
 GatherPushPlan gather_push_plan(int64_t n, int nx, int ny, int fp64) {
   GatherPushPlan p;
   const long long G = (long long)nx * ny, pad = (long long)(nx + 1) * (ny + 1);
   const long long bytes = pad * (fp64 ? 16 : 8);
   p.pairs = 0;
-  p.rows = 0;
+  p.rows = p.choose = p.ordered = p.local = 0;
   p.lds = 0;
   if (bytes <= 72 * 1024 && n >= std::max(262144ll, 256 * G)) {
     p.lds = (int)bytes;
@@ -813,11 +898,14 @@ GatherPushPlan gather_push_plan(int64_t n, int nx, int ny, int fp64) {
     p.blocks = (int)(b > 512 ? 512 : b);
     return p;
   }
-  if (n >= 524288 && n >= G / 8) {
+  if (n >= 524288 && n >= G / 4) {
     const long long state = n * (fp64 ? 32 : 16);
     p.rows = n >= std::max(1048576ll, G) &&
              (2 * bytes <= (4 << 20) / 3 || bytes > (6 << 20) || state >= (96ll << 20));
     p.pairs = p.rows ? 2ll * nx * (ny + 1) : pad;
+    p.choose = bytes > (6 << 20) && n <= 8 * G;
+    p.ordered = fp64 || n <= 2 * G ? GP_NODES : GP_PACKED;
+    p.local = fp64 && n < G ? GP_NODES : n <= 4 * G || !p.rows ? GP_PACKED : GP_ROWS;
   }
   const long long per = p.pairs ? 4 * PIC_WG : PIC_WG;
   const long long b = (n + per - 1) / per;
@@ -829,24 +917,27 @@ template <typename R>
 void launch_op_gather_push(hipStream_t s, const GatherPushPlan& p, R* x, R* y, R* vx, R* vy,
                            int64_t n, const double* ex, const double* ey, int nx, int ny,
                            double lx, double ly, double dt, double qm, double c,
-                           double* ke_partials, void* pairs) {
+                           double* ke_partials, void* pairs, int* choice) {
   typedef typename EWin<R>::R2 R2;
   R2* E = (R2*)pairs;
   if (p.lds) {
     k_op_gather_push<R, GP_LDS><<<p.blocks, GP_LDS_NT, p.lds, s>>>(
-        x, y, vx, vy, n, ex, ey, nullptr, nx, ny, lx, ly, dt, qm, c, ke_partials);
-  } else if (E) {
-    k_op_pack_E<R><<<grid_for((long long)nx * ny), PIC_WG, 0, s>>>(ex, ey, nx, ny, p.rows, E);
-    if (p.rows)
-      k_op_gather_push<R, GP_ROWS><<<p.blocks, PIC_WG, 0, s>>>(
-          x, y, vx, vy, n, nullptr, nullptr, E, nx, ny, lx, ly, dt, qm, c, ke_partials);
-    else
-      k_op_gather_push<R, GP_PACKED><<<p.blocks, PIC_WG, 0, s>>>(
-          x, y, vx, vy, n, nullptr, nullptr, E, nx, ny, lx, ly, dt, qm, c, ke_partials);
-  } else {
-    k_op_gather_push<R, GP_NODES><<<p.blocks, PIC_WG, 0, s>>>(
-        x, y, vx, vy, n, ex, ey, nullptr, nx, ny, lx, ly, dt, qm, c, ke_partials);
+        x, y, vx, vy, n, ex, ey, nullptr, nullptr, nx, ny, lx, ly, dt, qm, c, ke_partials);
+    return;
   }
+  auto push = [&](auto kernel) {
+    kernel<<<p.blocks, PIC_WG, 0, s>>>(x, y, vx, vy, n, ex, ey, E, choice, nx, ny, lx, ly, dt, qm,
+                                       c, ke_partials);
+  };
+  if (!E) return push(k_op_gather_push<R, GP_NODES>);
+  const int other = p.rows ? GP_ROWS : GP_PACKED;
+  // workgroups that look at the positions first: no more than fill the chip
+  const int blocks = std::min(grid_for((long long)nx * ny), choice ? 2048 : 8192);
+  k_op_pack_E<R><<<blocks, PIC_WG, 0, s>>>(ex, ey, x, y, n, p.ordered, p.local, other, choice, nx,
+                                           ny, lx, ly, E);
+  if (choice) push(k_op_gather_push<R, GP_AUTO>);
+  else if (p.rows) push(k_op_gather_push<R, GP_ROWS>);
+  else push(k_op_gather_push<R, GP_PACKED>);
 }
 
 #define PIC_INST(R)                                                                          \
@@ -864,6 +955,6 @@ void launch_op_gather_push(hipStream_t s, const GatherPushPlan& p, R* x, R* y, R
   template void launch_op_gather_push<R>(hipStream_t, const GatherPushPlan&, R*, R*, R*, R*, \
                                          int64_t, const double*, const double*, int, int,   \
                                          double, double, double, double, double, double*,   \
-                                         void*);
+                                         void*, int*);
 PIC_INST(float)
 PIC_INST(double)

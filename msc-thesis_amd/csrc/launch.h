@@ -162,14 +162,17 @@ struct GatherPushPlan {
   int lds;              // bytes of the padded field in LDS, 0: not there
   long long pairs;      // (Ex, Ey) pairs of the packed field, 0: not used
   int rows;             // packed with the two node rows of a cell interleaved
+  int choose;           // 1: the form goes by the order of the positions (gp_form)
+  int ordered, local;   // then those for ordered and for local positions
 };
 GatherPushPlan gather_push_plan(int64_t n, int nx, int ny, int fp64);
-// pairs: memory for the plan's packed field, or NULL (then the node arrays are read)
+// pairs: memory for the plan's packed field, or NULL (then the node arrays are read); choice: a word
+// for a plan that chooses, else NULL
 template <typename R>
 void launch_op_gather_push(hipStream_t s, const GatherPushPlan& p, R* x, R* y, R* vx, R* vy,
                            int64_t n, const double* ex, const double* ey, int nx, int ny,
                            double lx, double ly, double dt, double qm, double c,
-                           double* ke_partials, void* pairs);
+                           double* ke_partials, void* pairs, int* choice);
 void launch_op_fixed_to_double(hipStream_t s, const unsigned long long* hi,
                                const unsigned long long* lo, long long G, int fp64,
                                double scale, double* out);

@@ -308,12 +308,14 @@ int pic_op_gather_push(void* x, void* y, void* vx, void* vy, int64_t n, int prec
     (void)hipGetLastError();  // no memory for the packed field: the node arrays are read
     pairs = nullptr;
   }
+  int* choice = nullptr;
+  if (pairs && p.choose) PIC_HIP(m.get(&choice, 1));
   if (fp64)
     launch_op_gather_push<double>(s, p, (double*)x, (double*)y, (double*)vx, (double*)vy, n, ex,
-                                  ey, g->nx, g->ny, g->lx, g->ly, dt, qm, c, parts, pairs);
+                                  ey, g->nx, g->ny, g->lx, g->ly, dt, qm, c, parts, pairs, choice);
   else
     launch_op_gather_push<float>(s, p, (float*)x, (float*)y, (float*)vx, (float*)vy, n, ex, ey,
-                                 g->nx, g->ny, g->lx, g->ly, dt, qm, c, parts, pairs);
+                                 g->nx, g->ny, g->lx, g->ly, dt, qm, c, parts, pairs, choice);
   if (ke) launch_reduce_sum(s, parts, p.blocks, ke);
   PIC_HIP(hipGetLastError());
   PIC_HIP(hipStreamSynchronize(s));
