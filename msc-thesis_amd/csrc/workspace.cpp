@@ -6,8 +6,8 @@
 //   - A block belongs to one call at a time: it is taken from the free list and goes back only
 //     when the call has waited for its stream (Workspace::done), so no other stream or thread
 //     can meet work that still uses it.  A call that ends early frees its blocks instead.
-//   - Per device at most KEEP_BYTES in KEEP_BLOCKS are kept, the oldest freed first; all of
-//     them are freed when a context is destroyed, when a context needs the memory, and when an
+//   - Per device at most KEEP_BYTES in KEEP_BLOCKS are kept, the oldest freed first (a block above
+//     KEEP_BYTES is freed and evicts none); all of them are freed when a context is destroyed, when a context needs the memory, and when an
 //     allocation here fails (which is then tried once more).
 //   - The list itself is never destroyed: the runtime may be gone when the process ends.
 #include <algorithm>
@@ -106,11 +106,21 @@ Workspace::~Workspace() {
     give_back(blocks);  // frees wait for the device
     return;
   }
+  // blocks that evict each other go back the largest first, so that the small ones stay
+  size_t total = 0;
+  for (const Block& b : blocks) total += b.bytes;
+  if (total > KEEP_BYTES)
+    std::sort(blocks.begin(), blocks.end(),
+              [](const Block& a, const Block& b) { return a.bytes > b.bytes; });
   std::vector<Block> out;
   {
     Pool& q = pool();
     std::lock_guard<std::mutex> lk(q.mu);
     for (const Block& b : blocks) {
+      if (b.bytes > KEEP_BYTES) {  // would evict all the others and not fit itself
+        out.push_back(b);
+        continue;
+      }
       size_t held = b.bytes, count = 1;
       for (const Block& k : q.kept)
         if (k.device == b.device) {
@@ -127,8 +137,7 @@ Workspace::~Workspace() {
         out.push_back(q.kept[i]);
         q.kept.erase(q.kept.begin() + (long)i);
       }
-      if (held > KEEP_BYTES) out.push_back(b);
-      else q.kept.push_back(b);
+      q.kept.push_back(b);
     }
   }
   give_back(out);
