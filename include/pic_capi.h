@@ -80,11 +80,15 @@ typedef struct pic_config {
   int64_t capacity;          /* particle capacity per run (>= n); 0 => n at set time */
   int32_t precision;         /* PIC_FP32 | PIC_FP64 */
   int32_t device;            /* HIP device ordinal */
-  int32_t sort_every;        /* steps between cell sorts; 0 => autotuner default */
-  int32_t tile;              /* deposit tile side in cells (power of two); 0 => default */
-  int32_t halo;              /* deposit LDS window halo in cells; 0 => default */
-  int32_t splits;            /* workgroups per tile; 0 => default (sized by the particles
-                                per tile; in DSMC runs per tile, from each tile's count) */
+  int32_t sort_every;        /* steps between cell sorts; 0 => default (8; 4 in
+                                fast runs, by the speeds the runs hold) */
+  int32_t tile;              /* deposit tile side in cells (power of two); 0 =>
+                                default (by grid and particle count) */
+  int32_t halo;              /* deposit LDS window halo in cells; 0 => default (8; 16
+                                in fast runs) */
+  int32_t splits;            /* workgroups per tile; 0 => default (by the grid and the
+                                particle count; in DSMC runs shared out on the device or
+                                sized per tile, by the particles held) */
   int32_t collide;           /* PIC_COLLIDE_* */
   int32_t reserved0;
   uint64_t seed;             /* Philox4x32-10 key for every random stream */
@@ -153,7 +157,8 @@ int pic_stream(pic_ctx* ctx, void** stream);  /* hipStream_t of the context */
 /* Use (1) or bypass (0) captured hipGraphs for the step loop (default 1). */
 int pic_use_graphs(pic_ctx* ctx, int enable);
 /* Tiling / sort cadence in use (after defaults or autotuning); splits reads 0 when the
- * splits are sized per tile (DSMC runs asked for the default). */
+ * default splits of a DSMC run are in use.  The default halo and sort cadence follow the
+ * speeds of the particles set. */
 int pic_get_tuning(pic_ctx* ctx, int* tile, int* halo, int* splits, int* sort_every);
 int pic_set_tuning(pic_ctx* ctx, int tile, int halo, int splits, int sort_every);
 /* 1 when the tile sort runs inside the push launches (the step before a sort step counts

@@ -82,9 +82,9 @@ static double unit_drift(const pic_config& c) {
 }
 
 // Cells a thermal particle crosses per step, from the speeds a run holds: m8 are the means of
-// vx^8 and vy^8, whose eighth root is 105^(1/8) = 1.79 thermal speeds of a Maxwellian and the speed
-// itself of cold beams (which have no tail, so need that much less halo).  At least that of beams
-// of unit speed, the engine's units: cold particles do not stay cold.
+// vx^8 and vy^8, whose eighth root is 105^(1/8) = 1.79 thermal speeds of a Maxwellian and the
+// speed itself of cold beams (which have no tail, so need that much less halo).  At least that
+// of beams of unit speed, the engine's units: cold particles do not stay cold.
 static double held_drift(const pic_config& c, const double m8[2]) {
   const double q = std::pow(105.0, -0.125);
   const double d = q * c.dt * std::max(std::pow(m8[0], 0.125) / (c.lx / c.nx),
@@ -99,10 +99,11 @@ static double key_reach(const pic_config& c, int cadence) {
 }
 
 // Sort cadence when none is asked for: every 8 steps while the thermal drift from the keys is 13
-// cells or less (2.6 per step, with MCC 1.4), else every 4.  Steps sorted every 8 / 4 (us), 512^2
-// FP32 with 16 particles per cell: thermal speeds of 2 cells per step 60 / 64, 4 84 / 66, 6 137 / 73,
-// beams of 4 60 / 63, 6 85 / 64, 10 184 / 81; 256^2 FP64: thermal 2 42 / 44, 3 50 / 45, beams of 3
-// 40 / 43, 5 51 / 44, 10 142 / 65; 256^2 with MCC, thermal 1 68 / 70, 1.5 97 / 71, 2.5 194 / 101.
+// cells or less (2.6 per step, with MCC 1.4), else every 4.  Steps sorted every 8 / 4 (us):
+//   512^2 FP32, 16 particles per cell: thermal speeds of 2 cells per step 60 / 64, 4 84 / 66,
+//   6 137 / 73; beams of 4 60 / 63, 6 85 / 64, 10 184 / 81
+//   256^2 FP64: thermal 2 42 / 44, 3 50 / 45; beams of 3 40 / 43, 5 51 / 44, 10 142 / 65
+//   256^2 with MCC: thermal 1 68 / 70, 1.5 97 / 71, 2.5 194 / 101
 int Ctx::default_cadence() const {
   for (int r = 0; r < nruns; ++r)
     if (!(drift[r] * key_reach(cfg[r], 8) <= 13.0)) return 4;
@@ -120,12 +121,12 @@ static const int PUSH_LDS_MAX = 160 * 1024 - 256;
 
 // Tiling of a run whose share of the launch is `items` workgroups; nonzero values are kept.
 //   tile    the largest up to 32 that leaves half as many tiles as items (at most 128), 8 at
-//           least: a push workgroup pays for its windows, but a 64^2 grid in 16 tiles of 16^2 leaves most
-//           CUs idle (two-stream, 64^2, 409,600 FP64 particles: 46 us per step in 16 x 4
-//           workgroups, 26 in 64 x 4).  64 on FP32 grids that 32 leaves in more than 512 tiles
-//           (1024^2, 16 M particles: 375 us per step with 16, 259 with 32, 217 with 64)
-//           A halo the caller gives may not fit such tiles (1024^2 FP32, halo 24: 204 KB with 64,
-//           68 KB with 16): they are halved to 16 cells until the window fits
+//           least: a push workgroup pays for its windows, but a 64^2 grid in 16 tiles of 16^2
+//           leaves most CUs idle (two-stream, 64^2, 409,600 FP64 particles: 46 us per step in
+//           16 x 4 workgroups, 26 in 64 x 4).  64 on FP32 grids that 32 leaves in more than 512
+//           tiles (1024^2, 16 M particles: 375 us per step with 16, 259 with 32, 217 with 64).
+//           A halo the caller gives may not fit such tiles (1024^2 FP32, halo 24: 204 KB with
+//           64, 68 KB with 16): they are halved to 16 cells until the window fits
 //   halo    16 where the drift of 2.5 thermal speeds from the sort's keys passes 8 cells, else 8
 //   splits  as many as make up the items, of 256 particles at least and 65,536 at most
 static Tuning default_tuning(const pic_config& c, int tile, int halo, int splits, int cadence,
@@ -370,7 +371,6 @@ int Ctx::build_items() {
     maxb = std::max(maxb, d.nbuckets);
     d.tbase = tsum; tsum += (long long)d.nbuckets * d.nchunks;
     d.toffbase = toffsum; toffsum += d.nbuckets + 1;
-    d.key_tile_major = 1;
     d.tscan_item_begin = (int)tscan_items.size();
     for (long long s = 0; s < (long long)d.nbuckets * d.nchunks; s += PIC_CELL_CHUNK)
       tscan_items.push_back(make_int2(r, (int)s));
@@ -492,9 +492,8 @@ int Ctx::alloc() {
     any_mcc |= c.collide == PIC_COLLIDE_MCC;
     any_dsmc |= c.collide == PIC_COLLIDE_DSMC;
   }
-  // device memory the buffers below take (particle double buffers, sort keys / ranks /
-  // permutation / segment scratch, MCC birth buffers, grids): refuse before allocating
-  // anything when the device cannot hold it
+  // device memory the buffers below take (particle double buffers, sort keys and ranks, MCC
+  // birth buffers, grids): refuse before allocating anything when the device cannot hold it
   {
     long long maxcap = 0;
     for (auto& c : cfg) maxcap = std::max<long long>(maxcap, c.capacity);
@@ -1078,14 +1077,14 @@ static int read_state(Ctx& x, int run, RunState* s) {
 // (state read, field, output), direct against records, FP32 (us): 59 / 65 at 10,000 particles,
 // 66 / 63 at 100,000, 104 / 76 at 1,000,001, 247 / 128 at 4,000,001, 1094 / 555 at 16,777,216.
 static const int OUT_DIRECT_MAX = 1 << 16;
-// Bytes up to which an output to the host is one copy.  Whole calls, the four arrays in one copy and
-// each by itself (us): FP32 65 / 100 at 1000 particles, 99 / 107 at 32,768; FP64 65 / 95 at 1000, 102 /
-// 108 at 20,000, 173 / 132 at 32,768.  (As records, converted by fours: FP32 2500 against 1830 at
-// 1,000,001, FP64 24,500 against 7450 at 4,000,001.)
+// Bytes up to which an output to the host is one copy.  Whole calls, the four arrays in one
+// copy and each by itself (us): FP32 65 / 100 at 1000 particles, 99 / 107 at 32,768; FP64
+// 65 / 95 at 1000, 102 / 108 at 20,000, 173 / 132 at 32,768.  (As records, converted by fours:
+// FP32 2500 against 1830 at 1,000,001, FP64 24,500 against 7450 at 4,000,001.)
 static const size_t OUT_ONCE_BYTES = 512 << 10;
 
-// Records of an output live in the run's slice of the particle buffer that is not in use (the
-// next sort overwrites it).
+// An output is built in the run's slice of the particle buffer that is not in use (the next
+// sort overwrites it): records for device arrays, the arrays themselves for host ones.
 template <typename R>
 static int get_particles_t(Ctx& x, int run, void* ox, void* oy, void* ovx, void* ovy, int64_t n,
                            int sync, bool device_dst) {

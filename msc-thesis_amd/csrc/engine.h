@@ -106,7 +106,7 @@ struct Ctx {
   RunDesc* d_runs = nullptr;
   RunState* d_st = nullptr;
   // x, y, vx, vy of a buffer are one allocation (at px), one after the other, so that the
-  // buffer not in use (a sort's target) can hold the 4-value records of an output
+  // buffer not in use (a sort's target) can hold an output: 4-value records, or its arrays
   void* px[2] = {nullptr, nullptr};
   void* py[2] = {nullptr, nullptr};
   void* pvx[2] = {nullptr, nullptr};

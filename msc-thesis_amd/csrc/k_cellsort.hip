@@ -151,9 +151,10 @@ __global__ __launch_bounds__(PIC_WG) void k_scan_local(const RunDesc* __restrict
 // The chunk's base added to its offsets: the base is the sum of the run's chunk totals
 // before it (integer adds, so any order gives the same base), added up by the workgroup
 // itself, which saves a launch that scanned the chunk totals.  Also the tile offsets toff[t] =
-// offsets[t T^2] (the cell numbering is tile-major: tile t owns cells [t T^2, (t + 1) T^2)).  The run's last chunk writes the total: offsets[G], nsorted and the
-// closing tile offset; the first workgroup clears the count of cells too large for the
-// within-cell sort's small kernel (which appends to it next).
+// offsets[t T^2] (the cell numbering is tile-major: tile t owns cells [t T^2, (t + 1) T^2)).
+// The run's last chunk writes the total: offsets[G], nsorted and the closing tile offset; the
+// first workgroup clears the count of cells too large for the within-cell sort's small kernel
+// (which appends to it next).
 __global__ __launch_bounds__(PIC_WG) void k_scan_add(const RunDesc* __restrict__ runs,
                                                      RunState* __restrict__ st,
                                                      int* __restrict__ offsets,

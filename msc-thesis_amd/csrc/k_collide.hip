@@ -319,8 +319,8 @@ __device__ __forceinline__ int dsmc_cell_rm(int c, const DsmcArgs& a) {
 }
 
 // One candidate: the particles pi, pj at slots (pi(2m), pi(2m+1)) of the cell's round
-// permutation, accepted when u gm < g with gm = max(gmax at the round's start, g); an accepted pair keeps
-// its centre-of-mass velocity and turns its relative velocity to a uniform direction.
+// permutation, accepted when u gm < g with gm = max(gmax at the round's start, g); an accepted
+// pair keeps its centre-of-mass velocity and turns its relative velocity to a uniform direction.
 // Returns g (for the round's new gmax); counts acceptances in acc.
 __device__ __forceinline__ double dsmc_candidate(const DsmcArgs& a, long long pi, long long pj,
                                                  int cr, uint32_t s32, long long k, double gm,

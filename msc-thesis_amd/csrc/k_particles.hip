@@ -470,7 +470,8 @@ __device__ __forceinline__ int gp_form(const R* __restrict__ x, const R* __restr
     return __popcll(__ballot(pwrap(dx - cx + rows, g.nx) <= 2 * rows &&
                              pwrap(dy - cy + cols, g.ny) <= 2 * cols)) >= 32;
   };
-  return half_within(sizeof(R) == 8 ? 4 : 1, 8) ? ordered : half_within(g.nx >> 4, g.ny >> 4) ? local : other;
+  if (half_within(sizeof(R) == 8 ? 4 : 1, 8)) return ordered;
+  return half_within(g.nx >> 4, g.ny >> 4) ? local : other;
 }
 
 // form: GP_PACKED or GP_ROWS (the interleaved form, nx rows of 2 * (ny + 1) entries).  choice (or
@@ -871,17 +872,19 @@ void launch_op_cell_keys(hipStream_t s, const R* x, const R* y, int64_t n, int n
 //         256^2: 8,000,009 146 / 241 -> 163 / 215, but 4,194,304 88 / 133 -> 100 / 132
 //         1024^2: 8,000,009 353 / 353 -> 275 / 284, 1,048,576 68 / 73 -> 67 / 77
 //         2048^2: 4,194,304 243 / 260 -> 198 / 230, but 1,048,576 88 / 106 -> 84 / 119
-// In a step of the operators (deposit, Poisson, E, push: the deposit follows the rows' stores past
-// the caches) the large state's line costs 1.6 % at 8,000,009 FP32 on 512^2 (235 -> 239 us packed ->
-// rows), gives 11 % at 20,000,003 (567 -> 510), 4 % at 8,000,009 FP64 on 256^2 (379 -> 362).
+// In a step of the operators (deposit, Poisson, E, push: the deposit follows the rows' stores
+// past the caches) the large state's line costs 1.6 % at 8,000,009 FP32 on 512^2 (235 -> 239 us
+// packed -> rows), gives 11 % at 20,000,003 (567 -> 510), 4 % at 8,000,009 FP64 on 256^2
+// (379 -> 362).
 // Grids whose pairs outgrow the L2, up to 8 particles per node: random positions want the pairs,
-// but those that lie in cell order meet few lines of the node arrays and pay for packing, and nearby
-// ones meet few lines of the packed form.  The caller's order is not known here, so the packing
-// looks (gp_form: 2 to 4 us).  Sorted / within 10 cells of it / random (us):
-//   FP64 2048^2, 4,194,307: node arrays 70 / 112 / 353, packed 96 / 121 / 241, rows 134 / 165 / 201,
-//   chosen 77 / 125 / 209; 1024^2, 1,048,579: 35 / 46 / 88, 40 / 50 / 69, 51 / 61 / 69, 39 / 53 / 71
-//   FP32 2048^2, 4,194,307: 52 / 106 / 336, 64 / 81 / 198, 72 / 93 / 144, 59 / 82 / 147; 1024^2,
-//   4,194,307: 47 / 88 / 272, 50 / 64 / 135, 55 / 70 / 118, 53 / 72 / 117
+// but those that lie in cell order meet few lines of the node arrays and pay for packing, and
+// nearby ones meet few lines of the packed form.  The caller's order is not known here, so the
+// packing looks (gp_form: 2 to 4 us).  Sorted / within 10 cells of it / random (us), by node
+// arrays; packed; rows; as chosen:
+//   FP64 2048^2, 4,194,307: 70 / 112 / 353; 96 / 121 / 241; 134 / 165 / 201; 77 / 125 / 209
+//        1024^2, 1,048,579: 35 / 46 / 88; 40 / 50 / 69; 51 / 61 / 69; 39 / 53 / 71
+//   FP32 2048^2, 4,194,307: 52 / 106 / 336; 64 / 81 / 198; 72 / 93 / 144; 59 / 82 / 147
+//        1024^2, 4,194,307: 47 / 88 / 272; 50 / 64 / 135; 55 / 70 / 118; 53 / 72 / 117
 // On smaller grids looking costs what it gives (FP64 512^2, 4,194,307, sorted 80 either way).
 GatherPushPlan gather_push_plan(int64_t n, int nx, int ny, int fp64) {
   GatherPushPlan p;

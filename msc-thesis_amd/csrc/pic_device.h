@@ -13,7 +13,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#define PIC_WG 256                   // threads per workgroup of every kernel
+#define PIC_WG 256                   // threads per workgroup, where a kernel names no other
 #define PIC_FFT_MAX 2048             // largest grid side
 #define PIC_FFT_LOG 11               // log2(PIC_FFT_MAX)
 #define PIC_TW_LOG 11                // twiddle table: exp(-2 pi i k / 2048), k < 1024
@@ -32,7 +32,6 @@ struct RunDesc {
   int pcap, fft_pp;                  // fft_pp: row pairs per workgroup of the forward rows
   int nbuckets, nchunks;             // tiles (sort buckets) and PIC_CHUNK particle chunks
   int tscan_item_begin, tscan_item_end;
-  int key_tile_major;                // 1: cell keys ordered tile-major (engine sorts)
   int fft_rf;                        // rows per workgroup of the inverse (field) rows
   long long tbase;                   // bucket x chunk count table base (nbuckets*nchunks)
   long long toffbase;                // tile offsets base (nbuckets + 1)
@@ -266,15 +265,4 @@ __device__ __forceinline__ double block_sum(double v, double* scratch4) {
   double r = 0.0;
   if (threadIdx.x == 0) r = ((scratch4[0] + scratch4[1]) + scratch4[2]) + scratch4[3];
   return r;
-}
-
-__device__ __forceinline__ int wave_min_i(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
-  return v;
-}
-__device__ __forceinline__ int wave_max_i(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-  return v;
 }

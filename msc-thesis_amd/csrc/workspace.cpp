@@ -6,9 +6,10 @@
 //   - A block belongs to one call at a time: it is taken from the free list and goes back only
 //     when the call has waited for its stream (Workspace::done), so no other stream or thread
 //     can meet work that still uses it.  A call that ends early frees its blocks instead.
-//   - Per device at most KEEP_BYTES in KEEP_BLOCKS are kept, the oldest freed first (a block above
-//     KEEP_BYTES is freed and evicts none); all of them are freed when a context is destroyed, when a context needs the memory, and when an
-//     allocation here fails (which is then tried once more).
+//   - Per device at most KEEP_BYTES in KEEP_BLOCKS are kept, the oldest freed first (a block
+//     above KEEP_BYTES is freed and evicts none); all of them are freed when a context is
+//     destroyed, when a context needs the memory, and when an allocation here fails (which is
+//     then tried once more).
 //   - The list itself is never destroyed: the runtime may be gone when the process ends.
 #include <algorithm>
 #include <mutex>
