@@ -143,7 +143,6 @@ struct Ctx {
   unsigned long long* dsmc_slots = nullptr;
   int* birth_parent = nullptr;
   float* birth_buf = nullptr;
-  double* speed_part = nullptr;        // [2 * SPEED_BLOCKS]
   float* gmax = nullptr;               // per cell (ctotal)
   // output scratch
   int* flag = nullptr;
@@ -157,7 +156,8 @@ struct Ctx {
   int alloc();
   int default_cadence() const;
   void tune_runs();
-  int retune_for_speeds(int run, int64_t n);
+  bool tuned_by_speeds(int run) const;
+  int retune_for_speeds(int run, int64_t n, const double* sums);
   int check_tunings() const;
   int build_items();
   std::vector<int> push_order() const;

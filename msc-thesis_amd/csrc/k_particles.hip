@@ -694,6 +694,9 @@ __global__ void k_reduce_sum(const double* parts, int n, double* out) {
   if (threadIdx.x == 0) *out = v;
 }
 
+// Eighth moments of the velocities.  Bound by the read of the velocities; 1024 workgroups, as 256
+// leave too few loads in flight: the call that sets 16,777,216 FP32 particles takes 1016 us
+// without this kernel, 1108 with 256 workgroups, 1044 with 1024; 10,000 particles 112, 115, 118.
 template <typename R>
 __global__ __launch_bounds__(PIC_WG) void k_speed8(const R* __restrict__ vx,
                                                    const R* __restrict__ vy, int64_t n,

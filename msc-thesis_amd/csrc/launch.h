@@ -145,7 +145,8 @@ void launch_out_particles(hipStream_t s, const RunDesc* runs, RunState* st, int 
 template <typename R>
 void launch_out_split(hipStream_t s, const void* rec, int n, R* ox, R* oy, R* ovx, R* ovy);
 // sums of vx^8 and vy^8 over n particles from slot base on: part[SPEED_BLOCKS][2]
-#define SPEED_BLOCKS 256
+// (device or pinned memory)
+#define SPEED_BLOCKS 1024
 template <typename R>
 void launch_speed8(hipStream_t s, PartBufs<R> p, long long base, int64_t n, double* part);
 template <typename R>
