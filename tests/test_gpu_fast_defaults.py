@@ -81,6 +81,33 @@ def test_a_fast_run_of_a_batch():
         assert all(np.array_equal(a, r) for a, r in zip(g, ref))
 
 
+@pytest.mark.parametrize("order", [(0, 1, 2), (2, 0, 1)])
+def test_a_batch_is_laid_out_when_its_last_run_is_set(order):
+    """Whichever run comes last, also one whose own values are given; and again when a run of a
+    full batch gets other particles."""
+    runs = []
+    for k, v in enumerate((0.2, 7.0, 0.2)):
+        cfg, p = case(128, 128, 20_000, _lib.PIC_FP32, 0.01, 24 + k)
+        runs.append((cfg, with_speeds(cfg, p, v, v)))
+    runs[2][0].halo = 8
+    slow = with_speeds(runs[1][0], case(128, 128, 20_000, _lib.PIC_FP32, 0.01, 25)[1], 0.2, 0.2)
+    with Batch([c for c, _ in runs]) as b:
+        for k in order:
+            b.set_particles(*runs[k][1], run=k)
+        assert b.tuning()["sort_every"] == 4
+        b.step(10)
+        got = [b.particles(run=k, sync=False) for k in range(3)]
+        b.set_particles(*slow, run=1)
+        assert b.tuning()["sort_every"] == 8
+        b.step(10)
+        again = b.particles(run=1, sync=False)
+    for (cfg, p), g in zip(runs, got):
+        _, ref = run(cfg, p, None)
+        assert all(np.array_equal(a, r) for a, r in zip(g, ref))
+    _, ref = run(runs[1][0], slow, None)
+    assert all(np.array_equal(a, r) for a, r in zip(again, ref))
+
+
 def test_mcc_reach():
     """With MCC the keys are not led: the line is 1.44 cells per step, the halo's 0.36."""
     for v, every, halo in ((0.2, 8, 8), (0.5, 8, 16), (1.2, 8, 16), (1.7, 4, 16)):
